@@ -1,4 +1,4 @@
-// myea_gemm.hip — FP32 MFMA dense contraction for gfx950 (CDNA4), LDS-staged.
+// myea_gemm.hip — dense FP32 contraction for gfx950 (CDNA4) on the BF16 matrix cores, LDS-staged.
 //
 // One kernel template covers the three contractions of the fully-connected and LSTM path:
 //   forward  Y  = X W^T          (A k-contiguous, B k-contiguous)   Forward_Pass__FC,
@@ -7,23 +7,34 @@
 //   weights  dW += delta^T X     (A m-contiguous, B n-contiguous)   Update_Derivative_Weight__FC,
 //            Neural_Network__Update_Derivative_Weight__OpenMP.cpp:178-216
 //
-// Tiling: a workgroup of 256 lanes (4 wavefronts, 2 x 2) owns a BM x BN tile of C; each wavefront owns
-// (BM/2) x (BN/2) as TM x TN accumulators of v_mfma_f32_32x32x2_f32 (16 VGPRs each).  The K loop moves
-// BK = 32 columns per step through LDS stages with one barrier per step; the fragments of the next 8 k's are read from
-// LDS while the MFMAs of the current 8 issue.  General path (any alignment): global -> registers (guarded scalar loads,
-// issued before the MFMA block of the current step) -> LDS, two stages.  Operands keep their global orientation in LDS,
-// so no transposes are needed:
-//   k-contiguous operand : LDS [rows][BK + 4]   fragment = one ds_read_b128 per 4 MFMA k-steps
-//   mn-contiguous operand: LDS [BK][rows + 8]   fragment = conflict-free ds_read_b32 per k
-// When the operands are 16-byte aligned the tiles do not pass through registers at all: global_load_lds_dwordx4 writes
-// 1 KiB per wavefront instruction straight into LDS (lane l lands at base + 16 l), which rules out per-row padding, so
-//   k-contiguous operand : LDS [rows][BK], the 16-byte chunk c of row r stored at chunk c ^ ((r >> 1) & 7)
-//   mn-contiguous operand: LDS [BK][rows] in 1 KiB pieces, each padded so that k and k + 4 sit 32 banks apart
-// both again conflict-free for the fragment reads.
-// Inside a group of 8 k's, MFMA step j of lane-half h consumes k = 4h + j for BOTH operands, which is
-// what makes the two layouts interchangeable.
+// Arithmetic.  gfx950 multiplies FP32 at 157 TFLOP/s and BF16 at 2.5 PFLOP/s.  An FP32 number IS the sum of three BF16 numbers:
+// hi = x rounded to BF16, mid = (x - hi) rounded to BF16, lo = what is left (8 + 8 + 8 significant bits, signs included, cover
+// the 24 of x; both differences are exact in FP32).  Of the nine products of two such sums the six with a weight above 2^-24 are
+// formed - hi hi, hi mid, mid hi, mid mid, hi lo, lo hi - each exact in the matrix unit, all accumulated in FP32.  What is left
+// out is below 2^-25 of a product.  The five smaller products have an accumulator of their own, added at the end: an accumulator
+// as large as the result is rounded once per 16 k's, where v_mfma_f32_32x32x2_f32 rounds it at every second k, and the measured
+// error against 64-bit sums is smaller than that instruction's (normal operands, 2-norm: 4e-7 against 1.15e-6 at k = 4096,
+// 1.3e-7 against 4.1e-7 at k = 512; positive ones: 6.0e-7 against 1.7e-6 at k = 16384).  Six BF16 instructions for 16 k's
+// take 6 x 32 cycles of a SIMD's matrix unit where the FP32 ones take 8 x 64: the ceiling moves from 157 to 419 TFLOP/s, and to
+// 190 at the 1.14 PFLOP/s that a large BF16 product was measured to sustain on this card.  Measured, FP32 instruction -> this:
+// 1024 x 4096 x 4096 forward 314 -> 221 us, its weight gradient 304 -> 197 us (174 TFLOP/s), 16384 x 2048 x 512 269 -> 193 us
+// (178 TFLOP/s); 333 x 1201 x 1201, whose rows are no 16-byte multiples, 50 -> 25 us.
+// Infinities and NaN do not survive the split (inf - inf), nor do finite values that round to a BF16 infinity: such a product
+// always leaves a non-finite accumulator, and a wavefront that finds one computes its accumulators again with the FP32
+// instruction (redo_in_f32), so the results are those of FP32 arithmetic there too.
 //
-// Accumulator layout of v_mfma_f32_32x32x2_f32: register r of lane l holds
+// Tiling: a workgroup of 256 lanes (4 wavefronts, 2 x 2) owns a BM x BN tile of C; each wavefront owns (BM/2) x (BN/2) as
+// TM x TN accumulators of v_mfma_f32_32x32x16_bf16 (16 VGPRs each).  A K step moves BK columns: global -> registers (asked for
+// two steps ahead or four), split there once, three BF16 planes -> LDS (two stages, one barrier per step).  What bounds a step is
+// issue: per 16 k's of a 128 x 128 tile a wavefront has 24 matrix instructions (768 cycles) and about 100 vector ones (400), so
+// the splitting of the next step is spread between the matrix instructions of this one (2048 x 2048 x 2048: 114 us with the
+// compiler's order, 98 us so).  An operand's place in LDS
+// does not depend on its orientation in memory:
+//   [plane][k / 8][row][8 k's]     a fragment (row l % 32, k's 8 (l / 32) .. + 7 of lane l) is one conflict-free ds_read_b128
+// A k-contiguous operand is read as two 16-byte loads per lane, the other kind as eight 4-byte loads that are coalesced over
+// the rows; neither needs more than 4-byte alignment, so odd widths and leading dimensions take the same path.
+//
+// Accumulator layout of v_mfma_f32_32x32x16_bf16, as of v_mfma_f32_32x32x2_f32: register r of lane l holds
 //   C[(r / 4) * 8 + (l / 32) * 4 + (r % 4)][l % 32].
 #include <cstdlib>
 #include <mutex>
@@ -39,213 +50,104 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kBK = 32;
-constexpr int kPadK = 4;   // k-contiguous LDS rows: BK + 4 floats (144 B, keeps 16 B alignment)
-constexpr int kPadMN = 8;  // mn-contiguous LDS rows: rows + 8 floats
+constexpr int kBK = 32;   // slabs and halves of a k range are multiples of this
 
-template <int ROWS, bool KC>
-struct TileShape {
-    static constexpr int kLd = KC ? (kBK + kPadK) : (ROWS + kPadMN);
-    static constexpr int kFloats = KC ? ROWS * kLd : kBK * kLd;
-    static constexpr int kVec = ROWS * kBK / 4;            // float4 per tile
-    static constexpr int kPasses = kVec / kThreads;        // float4 per thread
-    static_assert(kVec % kThreads == 0, "tile must be a multiple of the workgroup");
-};
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));   // a 16-byte load from any element's address
 
-// Global -> register -> LDS mover for one operand tile (ROWS x BK): guarded scalar loads, any alignment (the general,
-// slower path; aligned operands take the direct path below).
-template <int ROWS, bool KC>
-struct TileMover {
-    using S = TileShape<ROWS, KC>;
-    f32x4 reg[S::kPasses];
-    const float *base; long ld; int row0, extent;
+// K columns per step: two stages of the 128 x 128 tile at 16 leave room for two workgroups a CU, the smaller tiles take a whole
+// 128-byte line of a k-contiguous row at a time
+constexpr int step_of(int bm, int bn) { return bm * bn >= 128 * 128 ? 16 : 32; }
 
-    // base: operand origin; ld: leading dimension; row0: first row (m or n) of the tile; extent: M or N
-    __device__ __forceinline__ void init(const float *__restrict__ base_, long ld_, int row0_, int extent_, int)
-    {
-        base = base_; ld = ld_; row0 = row0_; extent = extent_;
-    }
-
-    // k0: first k of the step; K: end of the k range
-    __device__ __forceinline__ void load(int k0, int K)
-    {
-        const int t = threadIdx.x;
-#pragma unroll
-        for (int p = 0; p < S::kPasses; ++p) {
-            int row, k;
-            if (KC) {
-                constexpr int vec_per_row = kBK / 4;
-                constexpr int rows_per_pass = kThreads / vec_per_row;
-                row = t / vec_per_row + p * rows_per_pass;
-                k = (t % vec_per_row) * 4;
-            } else {
-                constexpr int vec_per_k = ROWS / 4;
-                constexpr int k_per_pass = kThreads / vec_per_k;
-                k = t / vec_per_k + p * k_per_pass;
-                row = (t % vec_per_k) * 4;
-            }
-            const int gr = row0 + row, gk = k0 + k;
-            f32x4 v = {0.f, 0.f, 0.f, 0.f};
-            if (KC) {
-                const float *src = base + (long)gr * ld + gk;
-                if (gr < extent) {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (gk + e < K) v[e] = src[e];
-                }
-            } else {
-                const float *src = base + (long)gk * ld + gr;
-                if (gk < K) {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (gr + e < extent) v[e] = src[e];
-                }
-            }
-            reg[p] = v;
-        }
-    }
-
-    __device__ __forceinline__ void fill(float *, int k0, int K) { load(k0, K); }
-    __device__ __forceinline__ void commit(float *tile) const { store(tile); }
-    template <int N>
-    static __device__ __forceinline__ void wait() {}
-
-    __device__ __forceinline__ void store(float *lds) const
-    {
-        const int t = threadIdx.x;
-#pragma unroll
-        for (int p = 0; p < S::kPasses; ++p) {
-            int idx;
-            if (KC) {
-                constexpr int vec_per_row = kBK / 4;
-                constexpr int rows_per_pass = kThreads / vec_per_row;
-                idx = (t / vec_per_row + p * rows_per_pass) * S::kLd + (t % vec_per_row) * 4;
-            } else {
-                constexpr int vec_per_k = ROWS / 4;
-                constexpr int k_per_pass = kThreads / vec_per_k;
-                idx = (t / vec_per_k + p * k_per_pass) * S::kLd + (t % vec_per_k) * 4;
-            }
-            *reinterpret_cast<f32x4 *>(lds + idx) = reg[p];
-        }
-    }
-};
-
-// Fragment of one 32-row MFMA operand tile for a group of 8 k's: frag[j] feeds MFMA step j.
-template <int ROWS, bool KC>
-__device__ __forceinline__ f32x4 read_fragment(const float *lds, int tile_row, int kgroup, int lane32, int half)
+// two FP32 numbers -> the two BF16 numbers of each plane, packed
+__device__ __forceinline__ void split_pair(float x0, float x1, unsigned &hi, unsigned &mid, unsigned &lo)
 {
-    using S = TileShape<ROWS, KC>;
-    if (KC) {
-        return *reinterpret_cast<const f32x4 *>(lds + (tile_row + lane32) * S::kLd + kgroup * 8 + half * 4);
-    } else {
-        f32x4 v;
-        const float *src = lds + (kgroup * 8 + half * 4) * S::kLd + tile_row + lane32;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = src[j * S::kLd];
-        return v;
-    }
+    hi = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2){x0, x1}, bf16x2));
+    const float r0 = x0 - __uint_as_float(hi << 16), r1 = x1 - __uint_as_float(hi & 0xffff0000u);
+    mid = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2){r0, r1}, bf16x2));
+    const float q0 = r0 - __uint_as_float(mid << 16), q1 = r1 - __uint_as_float(mid & 0xffff0000u);
+    lo = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2){q0, q1}, bf16x2));
 }
 
-// ---- direct global -> LDS path (16-byte aligned operands) --------------------------------------------------------
-template <int ROWS, bool KC>
-struct DirectShape {
-    static constexpr int kPieces = ROWS * kBK * 4 / 1024;          // wavefront-wide 1 KiB pieces per tile
-    static constexpr int kPerWave = kPieces / 4;
-    static constexpr int kRowsPerPiece = KC ? 8 : 256 / ROWS;      // tile rows (KC) or k rows (MN) per piece
-    static constexpr int kPiecePad = KC ? 0 : (ROWS == 128 ? 16 : 32);
-    static constexpr int kPieceFloats = 256 + kPiecePad;
-    static constexpr int kFloats = kPieces * kPieceFloats;
-    static_assert(ROWS == 64 || ROWS == 128, "tile rows");
+// Where one operand tile (ROWS x BK, three planes) lies in an LDS stage: 16-byte chunks of 8 k's.
+template <int ROWS, int BK>
+struct PlaneShape {
+    static constexpr int kChunkRow = ROWS * 16 + 64;            // bytes of one [k / 8] slice; the pad keeps the slices' equal rows on different banks
+    static constexpr int kPlane = (BK / 8) * kChunkRow;
+    static constexpr int kBytes = 3 * kPlane;
+    static constexpr int kChunks = ROWS * BK / 8;
+    static constexpr int kPerThread = kChunks / kThreads;
+    static_assert(kChunks % kThreads == 0, "a tile's chunks go round the workgroup evenly");
+    static __device__ __forceinline__ int at(int plane, int k8, int row) { return plane * kPlane + k8 * kChunkRow + row * 16; }
 };
 
-template <int ROWS, bool KC>
-struct DirectMover {
-    using S = DirectShape<ROWS, KC>;
-    const float *ptr[S::kPerWave];
-    int kofs[S::kPerWave];      // k of the lane's 16 bytes inside the K step (for the predicated last step)
-    long step;
+// Global -> registers -> three planes in LDS for one operand tile; `AHEAD` steps wait in registers.
+template <int ROWS, int BK, bool KC, int AHEAD>
+struct SplitMover {
+    using S = PlaneShape<ROWS, BK>;
+    float reg[AHEAD][S::kPerThread][8];
+    const float *ptr[S::kPerThread];   // the chunk's first element in the step that is loaded next
+    long ld, step;
 
-    __device__ __forceinline__ void init(const float *__restrict__ base, long ld, int row0, int extent, int k0)
+    static __device__ __forceinline__ int row_of(int p) { const int q = threadIdx.x + p * kThreads; return KC ? q / (BK / 8) : q % ROWS; }
+    static __device__ __forceinline__ int k8_of(int p) { const int q = threadIdx.x + p * kThreads; return KC ? q % (BK / 8) : q / ROWS; }
+
+    // base: operand origin; row0: first row (m or n) of the tile; rows beyond the extent repeat the last one (never stored)
+    __device__ __forceinline__ void init(const float *base, long ld_, int row0, int extent, int k0)
     {
-        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+        ld = ld_; step = KC ? (long)BK : (long)BK * ld;
 #pragma unroll
-        for (int q = 0; q < S::kPerWave; ++q) {
-            const int piece = wave * S::kPerWave + q;
+        for (int p = 0; p < S::kPerThread; ++p) {
+            const long row = min(row0 + row_of(p), extent - 1), k = k0 + k8_of(p) * 8;
+            ptr[p] = base + (KC ? row * ld + k : k * ld + row);
+        }
+    }
+
+    // asks for a whole step, and moves on to the next one if there is another whole one (`more`)
+    __device__ __forceinline__ void load(int slot, bool more)
+    {
+        const long onward = more ? step : 0;
+#pragma unroll
+        for (int p = 0; p < S::kPerThread; ++p) {
             if (KC) {
-                const int row = piece * 8 + (lane >> 3);
-                const int c = (lane & 7) ^ ((row >> 1) & 7);
-                ptr[q] = base + (long)min(row0 + row, extent - 1) * ld + k0 + c * 4;
-                kofs[q] = c * 4;
+                *reinterpret_cast<f32x4 *>(reg[slot][p]) = *reinterpret_cast<const f32x4_any *>(ptr[p]);
+                *reinterpret_cast<f32x4 *>(reg[slot][p] + 4) = *reinterpret_cast<const f32x4_any *>(ptr[p] + 4);
             } else {
-                const int k = piece * S::kRowsPerPiece + (lane * 4) / ROWS, col = (lane * 4) % ROWS;
-                ptr[q] = base + (long)(k0 + k) * ld + min(row0 + col, extent - 4);
-                kofs[q] = k;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) reg[slot][p][e] = ptr[p][e * ld];
             }
+            ptr[p] += onward;
         }
-        step = KC ? (long)kBK : (long)kBK * ld;
     }
 
-    // Starts filling `tile` (LDS) with the K step that begins at k0; K is the end of the k range.
-    __device__ __forceinline__ void fill(float *tile, int k0, int K)
+    // the last, partial step: `left` k's, zeros behind them (in both operands)
+    __device__ __forceinline__ void load_tail(int left)
     {
-        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-        if (k0 + kBK <= K) {
 #pragma unroll
-            for (int q = 0; q < S::kPerWave; ++q) {
-                float *dst = tile + (wave * S::kPerWave + q) * S::kPieceFloats;   // wave-uniform
-                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)ptr[q],
-                                                 (__attribute__((address_space(3))) void *)dst, 16, 0, 0);
-                ptr[q] += step;
-            }
-        } else {   // last, partial step: through registers, zero filled along k
+        for (int p = 0; p < S::kPerThread; ++p)
 #pragma unroll
-            for (int q = 0; q < S::kPerWave; ++q) {
-                f32x4 v = {0.f, 0.f, 0.f, 0.f};
-                if (k0 + kofs[q] < K) v = *reinterpret_cast<const f32x4 *>(ptr[q]);
-                *reinterpret_cast<f32x4 *>(tile + (wave * S::kPerWave + q) * S::kPieceFloats + lane * 4) = v;
+            for (int e = 0; e < 8; ++e) {
+                reg[0][p][e] = 0.f;
+                if (k8_of(p) * 8 + e < left) reg[0][p][e] = ptr[p][KC ? (long)e : e * ld];
             }
+    }
+
+    __device__ __forceinline__ void store(int slot, char *tile) const
+    {
+#pragma unroll
+        for (int p = 0; p < S::kPerThread; ++p) {
+            unsigned hi[4], mid[4], lo[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) split_pair(reg[slot][p][2 * e], reg[slot][p][2 * e + 1], hi[e], mid[e], lo[e]);
+            const int row = row_of(p), k8 = k8_of(p);
+            *reinterpret_cast<u32x4 *>(tile + S::at(0, k8, row)) = (u32x4){hi[0], hi[1], hi[2], hi[3]};
+            *reinterpret_cast<u32x4 *>(tile + S::at(1, k8, row)) = (u32x4){mid[0], mid[1], mid[2], mid[3]};
+            *reinterpret_cast<u32x4 *>(tile + S::at(2, k8, row)) = (u32x4){lo[0], lo[1], lo[2], lo[3]};
         }
     }
-    __device__ __forceinline__ void commit(float *) const {}
-    // the direct loads count on vmcnt; they must have landed before the barrier that publishes the stage
-    // n = number of younger loads that may stay in flight (those of the step after next)
-    template <int N>
-    static __device__ __forceinline__ void wait() { __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14)); }   // vmcnt(N)
-};
-
-template <int ROWS, bool KC>
-__device__ __forceinline__ f32x4 read_fragment_direct(const float *lds, int tile_row, int kgroup, int lane32, int half)
-{
-    using S = DirectShape<ROWS, KC>;
-    if (KC) {
-        const int row = tile_row + lane32;
-        const int slot = (kgroup * 2 + half) ^ ((row >> 1) & 7);
-        return *reinterpret_cast<const f32x4 *>(lds + row * kBK + slot * 4);
-    } else {
-        f32x4 v;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int k = kgroup * 8 + half * 4 + j;
-            v[j] = lds[(k / S::kRowsPerPiece) * S::kPieceFloats + (k % S::kRowsPerPiece) * ROWS + tile_row + lane32];
-        }
-        return v;
-    }
-}
-
-// data path of one operand: how a tile gets into LDS and how fragments come out of it
-template <int ROWS, bool KC, bool VEC>
-struct OperandPath {
-    using Mover = TileMover<ROWS, KC>;
-    static constexpr int kFloats = TileShape<ROWS, KC>::kFloats;
-    static constexpr int kLoads = 0;
-    static __device__ __forceinline__ f32x4 frag(const float *lds, int tile_row, int g, int lane32, int half) { return read_fragment<ROWS, KC>(lds, tile_row, g, lane32, half); }
-};
-template <int ROWS, bool KC>
-struct OperandPath<ROWS, KC, true> {
-    using Mover = DirectMover<ROWS, KC>;
-    static constexpr int kFloats = DirectShape<ROWS, KC>::kFloats;
-    static constexpr int kLoads = DirectShape<ROWS, KC>::kPerWave;   // vmcnt events per wavefront per K step
-    static __device__ __forceinline__ f32x4 frag(const float *lds, int tile_row, int g, int lane32, int half) { return read_fragment_direct<ROWS, KC>(lds, tile_row, g, lane32, half); }
 };
 
 struct GemmDev {
@@ -313,7 +215,8 @@ __device__ __forceinline__ void store_tile_as(const GemmDev &p, const f32x16 (&a
         }
 #pragma unroll
         for (int i = 0; i < TM; ++i) {
-            const int row0 = at.m0 + at.wave_m + i * 32 + at.half * 4;
+            int row0 = at.m0 + at.wave_m + i * 32 + at.half * 4;
+            asm volatile("" : "+v"(row0));   // the addresses of this accumulator's rows are formed here: hoisted, those of all accumulators together spill
             float column_sum = 0.f, column_sum2 = 0.f;   // per kind: see col_partials
             // What an accumulator's elements read from other tensors - the addend, the pre-activation or the activation, x-hat -
             // is asked for four elements at a time, ahead of their arithmetic: read where it is used, every load would sit behind
@@ -416,14 +319,52 @@ __device__ __forceinline__ void store_tile_kind(const GemmDev &p, const f32x16 (
     }
 }
 
+// The accumulators of one wavefront again, with the FP32 matrix instruction and operands straight from memory: for products in
+// which infinities, NaN or overflows took part.  Rows and columns beyond the matrix repeat the last one.
+template <bool A_KC, bool B_KC, int TM, int TN>
+__device__ __forceinline__ void redo_in_f32(const GemmDev &p, f32x16 (&acc)[TM][TN], int row, int col, int half, int k_begin, int k_end)
+{
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+    for (int k0 = k_begin; k0 < k_end; k0 += 2) {
+        const int k = k0 + half;
+        float a[TM], b[TN];
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+            const long m = min(row + i * 32, p.M - 1);
+            a[i] = k < k_end ? p.A[A_KC ? m * p.lda + k : k * p.lda + m] : 0.f;
+        }
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            const long n = min(col + j * 32, p.N - 1);
+            b[j] = k < k_end ? p.B[B_KC ? n * p.ldb + k : k * p.ldb + n] : 0.f;
+        }
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[j], acc[i][j], 0, 0, 0);
+    }
+}
+
+template <int BM, int BN>
+constexpr int stage_bytes() { return PlaneShape<BM, step_of(BM, BN)>::kBytes + PlaneShape<BN, step_of(BM, BN)>::kBytes; }
+
 // One workgroup's share of a contraction: tile number `block` of problem `p`, staged through `smem`.
-template <int BM, int BN, bool A_KC, bool B_KC, bool VEC>
-__device__ __forceinline__ void gemm_tile(const GemmDev &p, const int block, float *smem)
+template <int BM, int BN, bool A_KC, bool B_KC>
+__device__ __forceinline__ void gemm_tile(const GemmDev &p, const int block, char *smem)
 {
     constexpr int TM = BM / 64, TN = BN / 64;  // 32x32 accumulators per wavefront along m / n
-    using PA = OperandPath<BM, A_KC, VEC>;
-    using PB = OperandPath<BN, B_KC, VEC>;
-    constexpr int kStage = PA::kFloats + PB::kFloats;  // one LDS stage = A tile then B tile
+    constexpr int BK = step_of(BM, BN);
+    using SA = PlaneShape<BM, BK>;
+    using SB = PlaneShape<BN, BK>;
+    constexpr int kAhead = BM * BN > 64 * 64 ? 2 : 4;   // steps that wait in registers (even: a step's stage is known at compile time)
+    using MA = SplitMover<BM, BK, A_KC, kAhead>;
+    using MB = SplitMover<BN, BK, B_KC, kAhead>;
+    constexpr int kStage = SA::kBytes + SB::kBytes;  // one LDS stage = A planes then B planes
 
     // Workgroup -> tile.  Consecutive workgroup ids land on different XCDs (8 of them, each with its own
     // L2), so give every XCD a contiguous run of tile ids, and walk tiles in bands of 8 m-tiles so that a
@@ -445,94 +386,109 @@ __device__ __forceinline__ void gemm_tile(const GemmDev &p, const int block, flo
     const int lane32 = lane & 31, half = lane >> 5;
     const int wave_m = (wave >> 1) * (BM / 2), wave_n = (wave & 1) * (BN / 2);
 
-    f32x16 acc[TM][TN];
+    f32x16 acc[TM][TN], small[TM][TN];   // the hi hi products; the others
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = small[i][j][r] = 0.f;
 
-    typename PA::Mover moveA;
-    typename PB::Mover moveB;
-    const int nk = (k_end - k_begin + kBK - 1) / kBK;
-    // LDS stages.  Register path: 2 (the next step's tile waits in registers).  Direct path: 3 - the loads of step
-    // kt + 2 are issued while step kt computes, so a load has two steps of compute to hide behind and only the loads of
-    // step kt + 1 must have landed (vmcnt(loads of one step)) at the barrier.
-    constexpr int NS = (VEC && BM * BN < 128 * 128) ? 3 : 2;   // 128 x 128 keeps two stages so that two workgroups fit a CU
-    constexpr int kInFlight = PA::kLoads + PB::kLoads;
-
-    moveA.init(p.A, p.lda, m0, p.M, k_begin);
-    moveB.init(p.B, p.ldb, n0, p.N, k_begin);
-    moveA.fill(smem, k_begin, k_end);
-    moveB.fill(smem + PA::kFloats, k_begin, k_end);
-    moveA.commit(smem);
-    moveB.commit(smem + PA::kFloats);
-    if (NS == 3 && nk > 1) {
-        moveA.fill(smem + kStage, k_begin + kBK, k_end);
-        moveB.fill(smem + kStage + PA::kFloats, k_begin + kBK, k_end);
-        PA::Mover::template wait<kInFlight>();
-    } else {
-        PA::Mover::template wait<0>();
-    }
-    __syncthreads();
-
-    int cur = 0;   // stage holding step kt
-    // Fragments are double buffered in registers: the LDS reads of group g + 1 are in flight while the MFMAs of group g
-    // issue.  The barrier that publishes the next stage sits in front of the LAST group of a step - its fragments are
-    // already in registers by then - so the first fragments of the next step are read behind that group's MFMAs
-    // instead of in front of an idle matrix pipe.
-    f32x4 fa[2][TM], fb[2][TN];
+    bf16x8 fa[BK / 16][3][TM], fb[BK / 16][3][TN];
+    auto read = [&](const char *la) {
+        const char *lb = la + SA::kBytes;
 #pragma unroll
-    for (int i = 0; i < TM; ++i) fa[0][i] = PA::frag(smem, wave_m + i * 32, 0, lane32, half);
+        for (int ks = 0; ks < BK / 16; ++ks)
 #pragma unroll
-    for (int j = 0; j < TN; ++j) fb[0][j] = PB::frag(smem + PA::kFloats, wave_n + j * 32, 0, lane32, half);
-    for (int kt = 0; kt < nk; ++kt) {
-        const int ahead = NS - 1;                       // how many steps ahead the fill runs
-        const bool more = kt + ahead < nk;
-        int nxt = cur + ahead; if (nxt >= NS) nxt -= NS;
-        float *next = smem + nxt * kStage;
-        if (more) {   // that stage was last read before the previous barrier
-            moveA.fill(next, k_begin + (kt + ahead) * kBK, k_end);
-            moveB.fill(next + PA::kFloats, k_begin + (kt + ahead) * kBK, k_end);
-        }
-        const float *la = smem + cur * kStage, *lb = la + PA::kFloats;
-        const int following = cur + 1 == NS ? 0 : cur + 1;   // stage of step kt + 1
+            for (int pl = 2; pl >= 0; --pl) {
 #pragma unroll
-        for (int g = 0; g < kBK / 8; ++g) {
-            const int cb = g & 1, nb = cb ^ 1;
-            if (g + 1 < kBK / 8) {
+                for (int i = 0; i < TM; ++i) fa[ks][pl][i] = *reinterpret_cast<const bf16x8 *>(la + SA::at(pl, ks * 2 + half, wave_m + i * 32 + lane32));
 #pragma unroll
-                for (int i = 0; i < TM; ++i) fa[nb][i] = PA::frag(la, wave_m + i * 32, g + 1, lane32, half);
-#pragma unroll
-                for (int j = 0; j < TN; ++j) fb[nb][j] = PB::frag(lb, wave_n + j * 32, g + 1, lane32, half);
-            } else {
-                if (more) {
-                    moveA.commit(next);
-                    moveB.commit(next + PA::kFloats);
-                }
-                // step kt + 1 must have landed; with three stages the fill of step kt + 2 may stay in flight
-                if (NS == 3 && more) PA::Mover::template wait<kInFlight>();
-                else PA::Mover::template wait<0>();
-                __syncthreads();
-                if (kt + 1 < nk) {
-                    const float *na = smem + following * kStage, *nbp = na + PA::kFloats;
-#pragma unroll
-                    for (int i = 0; i < TM; ++i) fa[nb][i] = PA::frag(na, wave_m + i * 32, 0, lane32, half);
-#pragma unroll
-                    for (int j = 0; j < TN; ++j) fb[nb][j] = PB::frag(nbp, wave_n + j * 32, 0, lane32, half);
-                }
+                for (int j = 0; j < TN; ++j) fb[ks][pl][j] = *reinterpret_cast<const bf16x8 *>(lb + SB::at(pl, ks * 2 + half, wave_n + j * 32 + lane32));
             }
-            __builtin_amdgcn_sched_barrier(0);  // keep the prefetch ahead of this group's MFMAs (the scheduler sinks it otherwise)
+    };
+    auto multiply = [&]() {
+        constexpr int pa[6] = {0, 2, 1, 0, 1, 0}, pb[6] = {2, 0, 1, 1, 0, 0};   // hi hi last
 #pragma unroll
-            for (int s = 0; s < 4; ++s)
+        for (int ks = 0; ks < BK / 16; ++ks)
+#pragma unroll
+            for (int q = 0; q < 6; ++q)
 #pragma unroll
                 for (int i = 0; i < TM; ++i)
 #pragma unroll
                     for (int j = 0; j < TN; ++j)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[cb][i][s], fb[cb][j][s], acc[i][j], 0, 0, 0);
+                        (q < 5 ? small[i][j] : acc[i][j]) = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[ks][pa[q]][i], fb[ks][pb[q]][j], q < 5 ? small[i][j] : acc[i][j], 0, 0, 0);
+    };
+    // The order of a step's instructions: the fragments first, then a few of the splitting's between every two matrix instructions,
+    // which leave the wavefront idle otherwise (left alone the compiler splits everything before the first of them).
+    constexpr int kMatrix = 6 * TM * TN * (BK / 16), kWrites = 3 * (MA::S::kPerThread + MB::S::kPerThread), kSplit = 11 * 4 * (MA::S::kPerThread + MB::S::kPerThread);
+    auto interleave = [&]() {
+        __builtin_amdgcn_sched_group_barrier(0x100, 3 * (TM + TN) * (BK / 16), 0);   // LDS reads
+#pragma unroll
+        for (int q = 0; q < kMatrix; ++q) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);           // a matrix instruction
+            __builtin_amdgcn_sched_group_barrier(0x002, (kSplit + kMatrix - 1) / kMatrix + 1, 0);   // vector arithmetic
+            if (q % (kMatrix / kWrites) == kMatrix / kWrites - 1) __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);   // an LDS write
         }
-        cur = following;
+    };
+    // The whole steps.  While step kt multiplies from its stage, step kt + 1 is split out of the registers into the other stage,
+    // those registers ask for step kt + 1 + kAhead, and one barrier ends the step.  Loads and stores behind the last whole step
+    // repeat it: no branch in the loop, so every wait counts exactly the loads it needs.
+    MA moveA;
+    MB moveB;
+    moveA.init(p.A, p.lda, m0, p.M, k_begin);
+    moveB.init(p.B, p.ldb, n0, p.N, k_begin);
+    const int whole = (k_end - k_begin) / BK, left = (k_end - k_begin) - whole * BK;
+    if (whole > 0) {
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+            moveA.load(u, u + 1 < whole);
+            moveB.load(u, u + 1 < whole);
+        }
+        moveA.store(0, smem);
+        moveB.store(0, smem + SA::kBytes);
+        moveA.load(0, kAhead + 1 < whole);
+        moveB.load(0, kAhead + 1 < whole);
+        __syncthreads();
+        for (int kt = 0; kt < whole; kt += kAhead) {
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u) {
+                if (u > 0 && kt + u >= whole) break;
+                char *next = smem + ((u + 1) & 1) * kStage;
+                read(smem + (u & 1) * kStage);   // in front of the stores: the compiler cannot tell the stages apart
+                moveA.store((u + 1) % kAhead, next);
+                moveB.store((u + 1) % kAhead, next + SA::kBytes);
+                moveA.load((u + 1) % kAhead, kt + u + 2 + kAhead < whole);
+                moveB.load((u + 1) % kAhead, kt + u + 2 + kAhead < whole);
+                multiply();
+                interleave();
+                __syncthreads();
+            }
+        }
+    }
+    if (left > 0) {
+        moveA.init(p.A, p.lda, m0, p.M, k_end - left);
+        moveB.init(p.B, p.ldb, n0, p.N, k_end - left);
+        moveA.load_tail(left);
+        moveB.load_tail(left);
+        moveA.store(0, smem);
+        moveB.store(0, smem + SA::kBytes);
+        __syncthreads();
+        read(smem);
+        multiply();
+    }
+    {   // an infinity, a NaN or a value that is a BF16 infinity took part (or the result itself is one): FP32 says what it is
+        float finite = 0.f;
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    acc[i][j][r] += small[i][j][r];
+                    finite = fmaf(acc[i][j][r], 0.f, finite);
+                }
+        if (__any(finite != 0.f)) redo_in_f32<A_KC, B_KC, TM, TN>(p, acc, m0 + wave_m + lane32, n0 + wave_n + lane32, half, k_begin, k_end);
     }
 
     if (BM == BN && p.pair_partials) {   // only launches of square tiles are split this way
@@ -618,11 +574,11 @@ __device__ __forceinline__ void gemm_tile(const GemmDev &p, const int block, flo
     else store_tile_kind<false, TM, TN>(p, acc, at);
 }
 
-template <int BM, int BN, bool A_KC, bool B_KC, bool VEC>
-__global__ __launch_bounds__(kThreads, 2) void gemm_f32_mfma_kernel(GemmDev p)
+template <int BM, int BN, bool A_KC, bool B_KC>
+__global__ __launch_bounds__(kThreads, 2) void gemm_f32_kernel(GemmDev p)
 {
-    extern __shared__ __attribute__((aligned(16))) float smem[];
-    gemm_tile<BM, BN, A_KC, B_KC, VEC>(p, (int)blockIdx.x, smem);
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    gemm_tile<BM, BN, A_KC, B_KC>(p, (int)blockIdx.x, smem);
 }
 
 // Two independent contractions in one launch, 128 x 128 tiles each: workgroups [0, first_blocks) work on `a` (A k-contiguous,
@@ -636,20 +592,20 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_mfma_kernel(GemmDev p)
 template <int BMA, int BNA>
 __global__ __launch_bounds__(kThreads, 2) void gemm_pair_kernel(GemmDev a, GemmDev b, int first_blocks)
 {
-    extern __shared__ __attribute__((aligned(16))) float smem[];
-    if ((int)blockIdx.x < first_blocks) gemm_tile<BMA, BNA, true, false, true>(a, (int)blockIdx.x, smem);
-    else gemm_tile<128, 128, false, false, true>(b, (int)blockIdx.x - first_blocks, smem);
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    if ((int)blockIdx.x < first_blocks) gemm_tile<BMA, BNA, true, false>(a, (int)blockIdx.x, smem);
+    else gemm_tile<128, 128, false, false>(b, (int)blockIdx.x - first_blocks, smem);
 }
 
-template <int BM, int BN, bool A_KC, bool B_KC, bool VEC>
+template <int BM, int BN, bool A_KC, bool B_KC>
 int launch_one(hipStream_t stream, GemmDev d)
 {
-    constexpr size_t lds_bytes = ((VEC && BM * BN < 128 * 128) ? 3 : 2) * (OperandPath<BM, A_KC, VEC>::kFloats + OperandPath<BN, B_KC, VEC>::kFloats) * sizeof(float);
-    auto kern = gemm_f32_mfma_kernel<BM, BN, A_KC, B_KC, VEC>;
+    constexpr size_t lds_bytes = 2 * stage_bytes<BM, BN>();
+    auto kern = gemm_f32_kernel<BM, BN, A_KC, B_KC>;
     static std::once_flag attr_once;  // per instantiation; launches may come from several host threads
     static hipError_t attr_status = hipSuccess;
     std::call_once(attr_once, [&] { attr_status = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes); });
-    if (attr_status != hipSuccess) return hip_fail(attr_status, "hipFuncSetAttribute(gemm_f32_mfma_kernel)");
+    if (attr_status != hipSuccess) return hip_fail(attr_status, "hipFuncSetAttribute(gemm_f32_kernel)");
     d.nbm = (d.M + BM - 1) / BM;
     d.nbn = (d.N + BN - 1) / BN;
     const long nblocks = (long)d.nbm * d.nbn * d.ksplit;
@@ -660,30 +616,13 @@ int launch_one(hipStream_t stream, GemmDev d)
 }
 
 template <int BM, int BN>
-int launch_layout_vec(hipStream_t stream, const GemmDev &d, bool a_kc, bool b_kc)
+int launch_layout(hipStream_t stream, const GemmDev &d, bool a_kc, bool b_kc)
 {
-    if (a_kc && b_kc) return launch_one<BM, BN, true, true, true>(stream, d);
-    if (a_kc && !b_kc) return launch_one<BM, BN, true, false, true>(stream, d);
-    return launch_one<BM, BN, false, false, true>(stream, d);
+    if (a_kc && b_kc) return launch_one<BM, BN, true, true>(stream, d);
+    if (a_kc && !b_kc) return launch_one<BM, BN, true, false>(stream, d);
+    if (!a_kc && !b_kc) return launch_one<BM, BN, false, false>(stream, d);
+    return launch_one<BM, BN, false, true>(stream, d);
 }
-
-// short-M, short-N problems (the per-time-step recurrent contractions): 64 x 64 tiles
-int launch_layout_vec_small(hipStream_t stream, const GemmDev &d, bool a_kc, bool b_kc)
-{
-    if (a_kc && b_kc) return launch_one<64, 64, true, true, true>(stream, d);
-    if (a_kc && !b_kc) return launch_one<64, 64, true, false, true>(stream, d);
-    return launch_one<64, 64, false, false, true>(stream, d);
-}
-
-// guarded scalar loads, any alignment, any layout: the general (slow) path
-int launch_layout_scalar(hipStream_t stream, const GemmDev &d, bool a_kc, bool b_kc)
-{
-    if (a_kc && b_kc) return launch_one<64, 64, true, true, false>(stream, d);
-    if (a_kc && !b_kc) return launch_one<64, 64, true, false, false>(stream, d);
-    if (!a_kc && !b_kc) return launch_one<64, 64, false, false, false>(stream, d);
-    return launch_one<64, 64, false, true, false>(stream, d);
-}
-
 
 // ---- a narrow product ---------------------------------------------------------------------------------------------------
 // C [M][N] = A B with N <= 32 and K <= 64 - a layer of an independently recurrent stack over T x batch rows, forward or backward.
@@ -820,8 +759,8 @@ bool gemm_can_fuse_activation(int act)
            act == MYEA_AF_TANH || act == MYEA_AF_SIGMOID;
 }
 
-// checks a problem and fills the kernel's argument block; *vec: operands take the direct (16-byte aligned) path
-static int prepare_gemm(const GemmParams &p, GemmDev &d, bool *vec)
+// checks a problem and fills the kernel's argument block
+static int prepare_gemm(const GemmParams &p, GemmDev &d)
 {
     if (p.M <= 0 || p.N <= 0 || p.K < 0) { set_last_error("gemm: bad shape M=%d N=%d K=%d", p.M, p.N, p.K); return MYEA_E_INVALID; }
     if (!p.A || !p.B || !p.C) { set_last_error("gemm: null operand"); return MYEA_E_INVALID; }
@@ -859,12 +798,6 @@ static int prepare_gemm(const GemmParams &p, GemmDev &d, bool *vec)
         d.slab = p.split_k_slab;
         if (d.ksplit != p.split_k) { set_last_error("gemm: split-K count %d does not divide K=%d into %d-wide chunks; use gemm_split_k()", p.split_k, p.K, chunk); return MYEA_E_INVALID; }
     }
-
-    // 128-bit global loads need 16-byte aligned rows; otherwise fall back to guarded scalar loads.
-    auto aligned = [](const float *ptr, long ld, long contiguous_extent) {
-        return (reinterpret_cast<uintptr_t>(ptr) & 15u) == 0 && (ld & 3) == 0 && (contiguous_extent & 3) == 0;
-    };
-    *vec = aligned(p.A, p.lda, p.a_k_contiguous ? p.K : p.M) && aligned(p.B, p.ldb, p.b_k_contiguous ? p.K : p.N);
     return MYEA_OK;
 }
 
@@ -894,9 +827,8 @@ int launch_narrow_dw(hipStream_t stream, const float *delta, const float *x, flo
 int launch_gemm(hipStream_t stream, const GemmParams &p)
 {
     GemmDev d;
-    bool vec = false;
     {
-        const int rc = prepare_gemm(p, d, &vec);
+        const int rc = prepare_gemm(p, d);
         if (rc != MYEA_OK) return rc;
     }
     const bool a_kc = p.a_k_contiguous != 0, b_kc = p.b_k_contiguous != 0;
@@ -912,11 +844,12 @@ int launch_gemm(hipStream_t stream, const GemmParams &p)
         MYEA_HIP_TRY(hipGetLastError());
         return MYEA_OK;
     }
-    if (!vec || (!a_kc && b_kc)) return launch_layout_scalar(stream, d, a_kc, b_kc);
-    // Tile choice: 128 x 128 when that still yields at least two workgroups per CU (256 CUs), else
-    // 64-row tiles to keep the chip filled for short-M / short-N problems.
+    // Tile choice: 128 x 128 from one workgroup per CU (256 CUs) on - its operand reuse is worth more than a second workgroup
+    // (2048 x 2048 x 2048, 256 such tiles: 98 us, 512 tiles of 64 x 128: 110 us) - else 64-row tiles to keep the chip filled for
+    // short-M / short-N problems.
     const long tiles_128 = (long)((p.M + 127) / 128) * ((p.N + 127) / 128);
-    if (tiles_128 * d.ksplit >= 512) return launch_layout_vec<128, 128>(stream, d, a_kc, b_kc);   // slabs of a split k count: they fill the chip like tiles do
+    const bool pair_128 = p.pair_partials && p.pair_tickets && d.ksplit == 1 && gemm_pair_k_128(p.M, p.N, p.K);   // see below
+    if (tiles_128 * d.ksplit >= 256 && !pair_128) return launch_layout<128, 128>(stream, d, a_kc, b_kc);   // slabs of a split k count: they fill the chip like tiles do
     // At most one 64 x 64 tile per compute unit and a k worth splitting: two workgroups per tile, half of k each, combined in
     // the launch - a second wavefront per SIMD to fill the first one's waits, which such a launch otherwise lacks.
     // MYEA_GEMM_PAIR_K=0 keeps one workgroup per tile.
@@ -925,22 +858,22 @@ int launch_gemm(hipStream_t stream, const GemmParams &p)
     // The same one size up: at most one 128 x 128 tile per compute unit (a batch of 1024 in front of 4096 units) would run as 64 x
     // 128 tiles to put two workgroups on every compute unit; two workgroups sharing a 128 x 128 tile's k do that with the larger
     // tile's operand reuse.
-    if ((pair_k & 2) && p.pair_partials && p.pair_tickets && d.ksplit == 1 && gemm_pair_k_128(p.M, p.N, p.K)) {
+    if ((pair_k & 2) && pair_128) {
         d.ksplit = 2;
         d.kchunk = ((p.K + 1) / 2 + kBK - 1) / kBK * kBK;
         d.pair_partials = p.pair_partials; d.pair_tickets = p.pair_tickets;
-        return launch_layout_vec<128, 128>(stream, d, a_kc, b_kc);
+        return launch_layout<128, 128>(stream, d, a_kc, b_kc);
     }
     const long tiles_64 = (long)((p.M + 63) / 64) * ((p.N + 63) / 64);
     if (p.pair_partials && p.pair_tickets && !pair_k_off && d.ksplit == 1 && tiles_64 <= kGemmPairTiles && tiles_64 % 8 == 0 && tiles_64 >= 128 && p.K >= 512) {
         d.ksplit = 2;
         d.kchunk = ((p.K + 1) / 2 + kBK - 1) / kBK * kBK;
         d.pair_partials = p.pair_partials; d.pair_tickets = p.pair_tickets;
-        return launch_layout_vec_small(stream, d, a_kc, b_kc);
+        return launch_layout<64, 64>(stream, d, a_kc, b_kc);
     }
-    if (tiles_128 * 2 * d.ksplit < 256) return launch_layout_vec_small(stream, d, a_kc, b_kc);
-    if (p.M <= p.N) return launch_layout_vec<64, 128>(stream, d, a_kc, b_kc);
-    return launch_layout_vec<128, 64>(stream, d, a_kc, b_kc);
+    if (tiles_128 * 2 * d.ksplit < 256) return launch_layout<64, 64>(stream, d, a_kc, b_kc);
+    if (p.M <= p.N) return launch_layout<64, 128>(stream, d, a_kc, b_kc);
+    return launch_layout<128, 64>(stream, d, a_kc, b_kc);
 }
 
 // `a` = (A k-contiguous, B n-contiguous), `b` = (both k-strided), neither split along k, 16-byte aligned operands, and `a`
@@ -950,12 +883,10 @@ int launch_gemm_pair(hipStream_t stream, const GemmParams &a, const GemmParams &
 {
     if (!a.a_k_contiguous || a.b_k_contiguous || b.a_k_contiguous || b.b_k_contiguous || a.split_k > 1 || b.split_k > 1) return 1;
     GemmDev da, db;
-    bool va = false, vb = false;
-    int rc = prepare_gemm(a, da, &va);
+    int rc = prepare_gemm(a, da);
     if (rc != MYEA_OK) return rc;
-    rc = prepare_gemm(b, db, &vb);
+    rc = prepare_gemm(b, db);
     if (rc != MYEA_OK) return rc;
-    if (!va || !vb) return 1;
     db.nbm = (b.M + 127) / 128; db.nbn = (b.N + 127) / 128;
     const long nb = (long)db.nbm * db.nbn;
     // Worth it when `a` alone would leave the CUs with one workgroup each and `b` brings about as much work in at least as
@@ -965,7 +896,7 @@ int launch_gemm_pair(hipStream_t stream, const GemmParams &a, const GemmParams &
         const double wa = (double)a.K * tile * tile * (double)na, wb = (double)b.K * 128.0 * 128.0 * (double)nb;
         return na >= 128 && na <= 256 && (na & 7) == 0 && nb >= na && wa <= 2.0 * wb && wb <= 2.0 * wa;
     };
-    constexpr size_t lds_b = 2 * (OperandPath<128, false, true>::kFloats + OperandPath<128, false, true>::kFloats) * sizeof(float);
+    constexpr size_t lds_b = 2 * stage_bytes<128, 128>();
     if (fits(128)) {
         // beside a long dX of 128 x 128 tiles the adds at the L2 were measured faster than stores (4096-wide layers at batch
         // 1024: 475 against 482 us); everywhere else a store onto known zeros wins
@@ -973,8 +904,7 @@ int launch_gemm_pair(hipStream_t stream, const GemmParams &a, const GemmParams &
         if (b.accumulate && !store128) db.accumulate = 1;
         da.nbm = (a.M + 127) / 128; da.nbn = (a.N + 127) / 128;
         const long na = (long)da.nbm * da.nbn;
-        constexpr size_t lds_a = 2 * (OperandPath<128, true, true>::kFloats + OperandPath<128, false, true>::kFloats) * sizeof(float);
-        constexpr size_t lds_bytes = lds_a > lds_b ? lds_a : lds_b;
+        constexpr size_t lds_bytes = lds_b;
         static std::once_flag attr_once;
         static hipError_t attr_status = hipSuccess;
         std::call_once(attr_once, [&] { attr_status = hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_pair_kernel<128, 128>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes); });
@@ -983,7 +913,7 @@ int launch_gemm_pair(hipStream_t stream, const GemmParams &a, const GemmParams &
     } else if (fits(64)) {
         da.nbm = (a.M + 63) / 64; da.nbn = (a.N + 63) / 64;
         const long na = (long)da.nbm * da.nbn;
-        constexpr size_t lds_a = 3 * (OperandPath<64, true, true>::kFloats + OperandPath<64, false, true>::kFloats) * sizeof(float);
+        constexpr size_t lds_a = 2 * stage_bytes<64, 64>();
         constexpr size_t lds_bytes = lds_a > lds_b ? lds_a : lds_b;
         static std::once_flag attr_once;
         static hipError_t attr_status = hipSuccess;

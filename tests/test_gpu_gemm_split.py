@@ -1,0 +1,52 @@
+"""The FP32 contraction on the BF16 matrix cores (three BF16 numbers an operand): every tile shape at its edges and remainders of
+a K step against float64, and operands that the split cannot carry (infinities, NaN, values that round to a BF16 infinity)
+against what FP32 arithmetic gives."""
+import numpy as np
+import pytest
+import torch
+
+from myea_amd import binding as mb
+from tests.test_gpu_kernels import _gemm
+
+pytestmark = pytest.mark.gpu
+
+LAYOUTS = [(1, 1), (1, 0), (0, 0), (0, 1)]
+# tiles of 64 x 64, 64 x 128, 128 x 64 and 128 x 128; k's below, at and beyond a step of 16 or 32
+SHAPES = [(190, 1100, 1), (65, 1300, 15), (600, 640, 33), (1500, 1501, 16), (1409, 1500, 65), (3001, 700, 31), (2049, 2050, 17), (2180, 1921, 48)]
+
+
+def _operands(a_kc, b_kc, M, N, K, seed):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    A, B = torch.randn((M, K), generator=g, device="cuda"), torch.randn((K, N), generator=g, device="cuda")
+    return A, B, (A if a_kc else A.t()).contiguous(), (B.t() if b_kc else B).contiguous()
+
+
+@pytest.mark.parametrize("a_kc,b_kc", LAYOUTS)
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_tiles_and_remainders_against_float64(a_kc, b_kc, M, N, K):
+    """An accumulator takes one rounding (2^-23 of what it holds, at most the sum of the magnitudes) per 16 k's, a few more join
+    the parts; the products left out are below 2^-24 of theirs."""
+    A, B, Ad, Bd = _operands(a_kc, b_kc, M, N, K, M + N + K)
+    C = torch.full((M, N), float("nan"), device="cuda")
+    _gemm(mb.load_library(), a_kc, b_kc, 0, M, N, K, Ad, Bd, C)
+    bound = 2.0 ** -23 * (-(-K // 16) + 8) * (A.double().abs() @ B.double().abs())
+    assert bool(((C.double() - A.double() @ B.double()).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("a_kc,b_kc", LAYOUTS)
+@pytest.mark.parametrize("M,N", [(100, 90), (1500, 1501), (2049, 2050)])
+def test_values_the_split_cannot_carry(a_kc, b_kc, M, N):
+    K = 40
+    A, B, _, _ = _operands(a_kc, b_kc, M, N, K, 3)
+    A[3, 5], A[10, 39], B[0, 20], A[50, 0], A[60] = float("inf"), float("nan"), -float("inf"), 3.4e38, 0.0
+    B[0, :20] = 0.25   # 3.4e38 rounds to a BF16 infinity; its products here are finite
+    Ad, Bd = (A if a_kc else A.t()).contiguous(), (B.t() if b_kc else B).contiguous()
+    C = torch.zeros((M, N), device="cuda")
+    _gemm(mb.load_library(), a_kc, b_kc, 0, M, N, K, Ad, Bd, C)
+    want, got = (A.cpu().double() @ B.cpu().double()).float().numpy(), C.cpu().numpy()
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    infinite = np.isinf(want)
+    assert np.array_equal(np.isinf(got), infinite) and np.array_equal(got[infinite], want[infinite])
+    finite = np.isfinite(want)
+    magnitudes = (np.nan_to_num(A.abs().cpu().double().numpy(), posinf=0.0)) @ (np.nan_to_num(B.abs().cpu().double().numpy(), posinf=0.0))
+    assert np.all(np.abs(got[finite].astype(np.float64) - want[finite]) <= 2.0 ** -23 * (K + 8) * magnitudes[finite])
