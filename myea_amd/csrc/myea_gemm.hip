@@ -624,6 +624,145 @@ int launch_layout(hipStream_t stream, const GemmDev &d, bool a_kc, bool b_kc)
     return launch_one<BM, BN, false, true>(stream, d);
 }
 
+// ---- a short product ----------------------------------------------------------------------------------------------------
+// A product with too few 64 x 64 tiles to occupy the chip - a batch of 128 in front of 256 units is 8 of them - spends the tiled
+// kernel's time in its K steps, one behind the other on a few compute units.  Here a workgroup owns 32 rows x 32 columns and its
+// kShortWaves wavefronts share k: each takes every kShortWaves-th run of 32 k's, asks for its operands straight from memory in
+// the lanes that multiply them (A: lane l takes row l % 32, k's 8 (l / 32) .. + 7 of a group of 16; B alike), a run ahead of the
+// one it splits and multiplies; no LDS and no barrier until the wavefronts' accumulators are added, in wavefront order, by the
+// first, which runs the tiled kernel's epilogue.  What bounds it is the latency of the first operands and the splitting, which
+// every workgroup of a row or column of tiles repeats; a layer of 256 units over a batch of 128 (k = 784) went from 19 to 8 us.
+constexpr int kShortWaves = 8;
+constexpr int kShortRun = 32;   // k's: one 128-byte line of a k-contiguous row
+
+template <bool KC>
+struct ShortOperand {
+    float reg[2][2][8];   // [slot][group of 16 k's][k]
+    const float *at;      // of the run that is loaded next
+    long ld, step;
+    int k, K;             // first k of this lane in that run
+
+    __device__ __forceinline__ void init(const float *base, long ld_, int row, int extent, int k0, int K_)
+    {
+        const long r = min(row, extent - 1);
+        ld = ld_; k = k0; K = K_;
+        at = base + (KC ? r * ld + k : k * ld + r);
+        step = KC ? (long)kShortRun * kShortWaves : (long)kShortRun * kShortWaves * ld;
+    }
+    __device__ __forceinline__ void load(int slot)
+    {
+        if (k + 24 <= K) {   // this lane's last k of the run is k + 23
+#pragma unroll
+            for (int g = 0; g < 2; ++g) {
+                if (KC) {
+                    *reinterpret_cast<f32x4 *>(reg[slot][g]) = *reinterpret_cast<const f32x4_any *>(at + g * 16);
+                    *reinterpret_cast<f32x4 *>(reg[slot][g] + 4) = *reinterpret_cast<const f32x4_any *>(at + g * 16 + 4);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) reg[slot][g][e] = at[(g * 16 + e) * ld];
+                }
+            }
+        } else {
+#pragma unroll
+            for (int g = 0; g < 2; ++g)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    reg[slot][g][e] = 0.f;
+                    if (k + g * 16 + e < K) reg[slot][g][e] = at[KC ? (long)(g * 16 + e) : (g * 16 + e) * ld];
+                }
+        }
+        at += step; k += kShortRun * kShortWaves;
+    }
+    __device__ __forceinline__ void split(int slot, int g, bf16x8 (&planes)[3]) const
+    {
+        u32x4 hi, mid, lo;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            unsigned h, m, l;
+            split_pair(reg[slot][g][2 * e], reg[slot][g][2 * e + 1], h, m, l);
+            hi[e] = h; mid[e] = m; lo[e] = l;
+        }
+        planes[0] = __builtin_bit_cast(bf16x8, hi); planes[1] = __builtin_bit_cast(bf16x8, mid); planes[2] = __builtin_bit_cast(bf16x8, lo);
+    }
+};
+
+template <bool A_KC, bool B_KC>
+__global__ __launch_bounds__(64 * kShortWaves) void short_gemm_kernel(GemmDev p)
+{
+    __shared__ f32x4 handed[kShortWaves - 1][4][64];   // the accumulators of the wavefronts behind the first
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lane32 = lane & 31, half = lane >> 5;
+    const int nblocks = p.nbm * p.nbn, split = (int)blockIdx.x / nblocks, pid = (int)blockIdx.x - split * nblocks;
+    const int m0 = pid % p.nbm * 32, n0 = pid / p.nbm * 32;
+    const int k_begin = split * p.kchunk, k_end = min(p.K, k_begin + p.kchunk);
+    f32x16 acc[1][1], small;   // the hi hi products; the others
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[0][0][r] = small[r] = 0.f;
+    ShortOperand<A_KC> a;
+    ShortOperand<B_KC> b;
+    const int first = k_begin + wave * kShortRun;
+    a.init(p.A, p.lda, m0 + lane32, p.M, first + half * 8, k_end);
+    b.init(p.B, p.ldb, n0 + lane32, p.N, first + half * 8, k_end);
+    const int runs = first < k_end ? (k_end - first + kShortRun * kShortWaves - 1) / (kShortRun * kShortWaves) : 0;
+    auto multiply = [&](int slot) {
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+            bf16x8 pa[3], pb[3];
+            a.split(slot, g, pa);
+            b.split(slot, g, pb);
+            constexpr int qa[5] = {0, 2, 1, 0, 1}, qb[5] = {2, 0, 1, 1, 0};
+#pragma unroll
+            for (int q = 0; q < 5; ++q) small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pa[qa[q]], pb[qb[q]], small, 0, 0, 0);
+            acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pa[0], pb[0], acc[0][0], 0, 0, 0);
+        }
+    };
+    if (runs > 0) { a.load(0); b.load(0); }
+    for (int r = 0; r < runs; r += 2) {
+        if (r + 1 < runs) { a.load(1); b.load(1); }
+        multiply(0);
+        if (r + 1 >= runs) break;
+        if (r + 2 < runs) { a.load(0); b.load(0); }
+        multiply(1);
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[0][0][r] += small[r];
+    if (wave) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) handed[wave - 1][r][lane] = (f32x4){acc[0][0][r * 4], acc[0][0][r * 4 + 1], acc[0][0][r * 4 + 2], acc[0][0][r * 4 + 3]};
+    }
+    __syncthreads();
+    if (wave) return;
+    float finite = 0.f;
+#pragma unroll
+    for (int w = 0; w < kShortWaves - 1; ++w)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const f32x4 v = handed[w][r][lane];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[0][0][r * 4 + e] += v[e];
+        }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) finite = fmaf(acc[0][0][r], 0.f, finite);
+    if (__any(finite != 0.f)) redo_in_f32<A_KC, B_KC, 1, 1>(p, acc, m0 + lane32, n0 + lane32, half, k_begin, k_end);
+    const TilePlace at{m0, n0, 0, 0, lane32, half, (long)split * p.slab};
+    if (m0 + 32 <= p.M && n0 + 32 <= p.N) store_tile_kind<true, 1, 1>(p, acc, at);
+    else store_tile_kind<false, 1, 1>(p, acc, at);
+}
+
+int launch_short(hipStream_t stream, GemmDev d, bool a_kc, bool b_kc)
+{
+    d.nbm = (d.M + 31) / 32;
+    d.nbn = (d.N + 31) / 32;
+    const long nblocks = (long)d.nbm * d.nbn * d.ksplit;
+    if (nblocks <= 0 || nblocks > 0x7fffffffL) { set_last_error("gemm: grid of %ld workgroups out of range", nblocks); return MYEA_E_INVALID; }
+    const dim3 grid((unsigned)nblocks), group(64 * kShortWaves);
+    if (a_kc && b_kc) hipLaunchKernelGGL((short_gemm_kernel<true, true>), grid, group, 0, stream, d);
+    else if (a_kc) hipLaunchKernelGGL((short_gemm_kernel<true, false>), grid, group, 0, stream, d);
+    else if (b_kc) hipLaunchKernelGGL((short_gemm_kernel<false, true>), grid, group, 0, stream, d);
+    else hipLaunchKernelGGL((short_gemm_kernel<false, false>), grid, group, 0, stream, d);
+    MYEA_HIP_TRY(hipGetLastError());
+    return MYEA_OK;
+}
+
 // ---- a narrow product ---------------------------------------------------------------------------------------------------
 // C [M][N] = A B with N <= 32 and K <= 64 - a layer of an independently recurrent stack over T x batch rows, forward or backward.
 // The tiled kernel spends such a launch on its set-up, its predicated scalar loads and its stages (rows of 31 floats are no
@@ -864,7 +1003,11 @@ int launch_gemm(hipStream_t stream, const GemmParams &p)
         d.pair_partials = p.pair_partials; d.pair_tickets = p.pair_tickets;
         return launch_layout<128, 128>(stream, d, a_kc, b_kc);
     }
+    // Fewer than 128 tiles of 64 x 64, slabs counted (half the compute units): the short product, whose workgroups are four times as
+    // many and keep eight wavefronts busy each.  us, tiled -> short: 128 x 256 x 784 16.0 -> 8.0, 512 x 100 x 2048 34 -> 18, 256 x
+    // 1024 x 1024 19.0 -> 12.0, 333 x 1201 x 1201 (114 tiles) 25.3 -> 22.8; at 128 tiles (512 x 1024 x 1024) 19.1 -> 21.4.
     const long tiles_64 = (long)((p.M + 63) / 64) * ((p.N + 63) / 64);
+    if (tiles_64 * d.ksplit < 128) return launch_short(stream, d, a_kc, b_kc);
     if (p.pair_partials && p.pair_tickets && !pair_k_off && d.ksplit == 1 && tiles_64 <= kGemmPairTiles && tiles_64 % 8 == 0 && tiles_64 >= 128 && p.K >= 512) {
         d.ksplit = 2;
         d.kchunk = ((p.K + 1) / 2 + kBK - 1) / kBK * kBK;

@@ -1436,6 +1436,9 @@ static int fc_dw_slabs(size_t H, size_t In, size_t rows, size_t first_connection
     if (rows > 0x7fffffffu) return 1;
     const int narrow = narrow_dw_slabs(H, In, rows);   // a narrow layer's kernel of its own: always through slabs
     if (narrow > 0) return narrow > 1 ? narrow : 2;    // (room for two, so that "more than one slab" still says "through slabs")
+    // Short of 1024 rows one launch is as good as slabs without the pass that adds them: each of the short product's eight wavefronts
+    // has four runs of 32 rows at most (37 x 1201 over 333 rows: 11 + 4 us through two slabs, 7 us so).
+    if (rows < 1024) return 1;
     return gemm_split_k((int)H, (int)In, (int)rows);
 }
 

@@ -50,3 +50,14 @@ def test_values_the_split_cannot_carry(a_kc, b_kc, M, N):
     finite = np.isfinite(want)
     magnitudes = (np.nan_to_num(A.abs().cpu().double().numpy(), posinf=0.0)) @ (np.nan_to_num(B.abs().cpu().double().numpy(), posinf=0.0))
     assert np.all(np.abs(got[finite].astype(np.float64) - want[finite]) <= 2.0 ** -23 * (K + 8) * magnitudes[finite])
+
+
+@pytest.mark.parametrize("a_kc,b_kc", LAYOUTS)
+@pytest.mark.parametrize("M,N,K", [(1, 33, 1), (31, 1, 23), (33, 32, 24), (32, 65, 31), (64, 64, 33), (95, 100, 255), (100, 31, 257), (700, 600, 545)])
+def test_short_products_against_float64(a_kc, b_kc, M, N, K):
+    """Fewer than 128 tiles of 64 x 64: eight wavefronts share k in runs of 32, of which the last ones may have none or a part."""
+    A, B, Ad, Bd = _operands(a_kc, b_kc, M, N, K, M + N + K)
+    C = torch.full((M, N), float("nan"), device="cuda")
+    _gemm(mb.load_library(), a_kc, b_kc, 0, M, N, K, Ad, Bd, C)
+    bound = 2.0 ** -23 * (-(-K // 16) + 8) * (A.double().abs() @ B.double().abs())
+    assert bool(((C.double() - A.double() @ B.double()).abs() <= bound).all())
