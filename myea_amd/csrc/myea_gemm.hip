@@ -41,36 +41,18 @@
 
 #include "myea_device_af.h"
 #include "myea_kernels.h"
+#include "myea_split.h"
 
 namespace myea {
-
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 namespace {
 
 constexpr int kThreads = 256;
 constexpr int kBK = 32;   // slabs and halves of a k range are multiples of this
 
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));   // a 16-byte load from any element's address
-
 // K columns per step: two stages of the 128 x 128 tile at 16 leave room for two workgroups a CU, the smaller tiles take a whole
 // 128-byte line of a k-contiguous row at a time
 constexpr int step_of(int bm, int bn) { return bm * bn >= 128 * 128 ? 16 : 32; }
-
-// two FP32 numbers -> the two BF16 numbers of each plane, packed
-__device__ __forceinline__ void split_pair(float x0, float x1, unsigned &hi, unsigned &mid, unsigned &lo)
-{
-    hi = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2){x0, x1}, bf16x2));
-    const float r0 = x0 - __uint_as_float(hi << 16), r1 = x1 - __uint_as_float(hi & 0xffff0000u);
-    mid = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2){r0, r1}, bf16x2));
-    const float q0 = r0 - __uint_as_float(mid << 16), q1 = r1 - __uint_as_float(mid & 0xffff0000u);
-    lo = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2){q0, q1}, bf16x2));
-}
 
 // Where one operand tile (ROWS x BK, three planes) lies in an LDS stage: 16-byte chunks of 8 k's.
 template <int ROWS, int BK>
@@ -673,17 +655,6 @@ struct ShortOperand {
         }
         at += step; k += kShortRun * kShortWaves;
     }
-    __device__ __forceinline__ void split(int slot, int g, bf16x8 (&planes)[3]) const
-    {
-        u32x4 hi, mid, lo;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            unsigned h, m, l;
-            split_pair(reg[slot][g][2 * e], reg[slot][g][2 * e + 1], h, m, l);
-            hi[e] = h; mid[e] = m; lo[e] = l;
-        }
-        planes[0] = __builtin_bit_cast(bf16x8, hi); planes[1] = __builtin_bit_cast(bf16x8, mid); planes[2] = __builtin_bit_cast(bf16x8, lo);
-    }
 };
 
 template <bool A_KC, bool B_KC>
@@ -707,11 +678,10 @@ __global__ __launch_bounds__(64 * kShortWaves) void short_gemm_kernel(GemmDev p)
 #pragma unroll
         for (int g = 0; g < 2; ++g) {
             bf16x8 pa[3], pb[3];
-            a.split(slot, g, pa);
-            b.split(slot, g, pb);
-            constexpr int qa[5] = {0, 2, 1, 0, 1}, qb[5] = {2, 0, 1, 1, 0};
+            split_eight(a.reg[slot][g], pa);
+            split_eight(b.reg[slot][g], pb);
 #pragma unroll
-            for (int q = 0; q < 5; ++q) small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pa[qa[q]], pb[qb[q]], small, 0, 0, 0);
+            for (int q = 0; q < 5; ++q) small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pa[kSmallA[q]], pb[kSmallB[q]], small, 0, 0, 0);
             acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pa[0], pb[0], acc[0][0], 0, 0, 0);
         }
     };

@@ -278,7 +278,8 @@ struct LstmFusedBackward {
     size_t B, C;
     int first_step;           // the sequence's first step: no forget-gate delta
     const float *dG_next;     // [B][4C] gate deltas of the step processed after this one
-    const float *WrecT;       // [C][4C] transposed packed recurrent weights
+    const float *WrecT;       // [C][4C] transposed packed recurrent weights (launch_lstm_fused_backward)
+    const float *Wrec;        // [4C][C] the packed recurrent weights (launch_lstm_step_backward)
     const float *peep;        // [3][C]
     const float *acts, *acts_next;   // [B][4C]
     const float *c_prev;      // [B][C], unused on the first step
@@ -291,6 +292,10 @@ struct LstmFusedBackward {
 bool lstm_fused_supported(size_t C, size_t cells_per_block);
 int launch_lstm_fused_forward(hipStream_t s, const LstmFusedForward &p);
 int launch_lstm_fused_backward(hipStream_t s, const LstmFusedBackward &p);
+// the same step for any width, one cell per block, while it is small enough (lstm_step_fits)
+bool lstm_step_fits(size_t C, size_t cells_per_block, size_t B);
+int launch_lstm_step_forward(hipStream_t s, const LstmFusedForward &p);
+int launch_lstm_step_backward(hipStream_t s, const LstmFusedBackward &p);
 int launch_transpose(hipStream_t s, size_t rows, size_t cols, const float *src, float *dst);
 
 // ---- LSTM time loop as one resident launch (one cell per block, C in {128, 256, 512, 1024}) --------------------------

@@ -1338,14 +1338,15 @@ int Net::lstm_forward_step(LstmLayer &q, size_t B, size_t s)
     const bool zone = q.zone_state != nullptr && state == MYEA_STATE_TRAINING;
     const uint8_t *zs = zone ? q.zone_state + t * q.zone_stride : nullptr, *zo = zone ? q.zone_output + t * q.zone_stride : nullptr;
     int nparts = 0;
-    if (s > 0 && q.fused) {   // recurrent contraction and gate math of the step in one launch
+    const bool step = !q.fused && !fused_lstm_disabled() && lstm_step_fits(q.C, q.cpb, B);
+    if (s > 0 && (q.fused || step)) {   // recurrent contraction and gate math of the step in one launch
         LstmFusedForward f{};
         f.B = B; f.C = q.C;
         f.h_prev = q.h + tp * Bmax * q.C; f.Wrec = q.Wrec; f.bias = bias; f.peep = q.peep;
         f.acts = acts_t; f.c_prev = q.c + tp * Bmax * q.C;
         f.c = q.c + t * Bmax * q.C; f.ca = q.ca + t * Bmax * q.C; f.h = q.h + t * Bmax * q.C;
         f.zone_state = zs; f.zone_output = zo;
-        return launch_lstm_fused_forward(stream, f);
+        return step ? launch_lstm_step_forward(stream, f) : launch_lstm_fused_forward(stream, f);
     }
     if (s > 0) {
         GemmParams g{};
@@ -1662,14 +1663,15 @@ int Net::lstm_backward_step(LstmLayer &q, size_t B, size_t s)
     float *dh_t = q.dh + t * Bmax * q.C;
     const bool last = s == T - 1, first = s == 0;
     int nparts = 0;
-    if (!last && q.fused) {   // dh[t] += dG[tn] Wrec and the gate deltas of step t in one launch
+    const bool step = !q.fused && !fused_lstm_disabled() && lstm_step_fits(q.C, q.cpb, B);
+    if (!last && (q.fused || step)) {   // dh[t] += dG[tn] Wrec and the gate deltas of step t in one launch
         LstmFusedBackward f{};
         f.B = B; f.C = q.C; f.first_step = first;
-        f.dG_next = q.dG + tn * Bmax * q.G; f.WrecT = q.WrecT; f.peep = q.peep;
+        f.dG_next = q.dG + tn * Bmax * q.G; f.WrecT = q.WrecT; f.Wrec = q.Wrec; f.peep = q.peep;
         f.acts = q.acts + t * Bmax * q.G; f.acts_next = q.acts + tn * Bmax * q.G;
         f.c_prev = first ? nullptr : q.c + tp * Bmax * q.C; f.ca = q.ca + t * Bmax * q.C;
         f.dh = dh_t; f.dG = q.dG + t * Bmax * q.G; f.dc = q.dc + t * Bmax * q.C; f.dc_next = q.dc + tn * Bmax * q.C;
-        return launch_lstm_fused_backward(stream, f);
+        return step ? launch_lstm_step_backward(stream, f) : launch_lstm_fused_backward(stream, f);
     }
     if (!last) {  // Backward_Pass__LSTM_Derivative__Output, recurrent part (:1174-1226)
         GemmParams g{};

@@ -13,7 +13,8 @@
 // barrier, only vmcnt.
 //
 // Layout requirements (checked on the host): one cell per block (K == C, G == 4C) and C a multiple of 32.
-// Everything else runs on the generic path (contraction + lstm_*_step_kernel).
+// Layers of one cell per block and another width take the second pair of kernels below while a step is small (lstm_step_fits);
+// everything else runs on the generic path (contraction + lstm_*_step_kernel).
 //
 // MFMA operand layouts used below (k may be permuted freely as long as A and B agree):
 //   v_mfma_f32_32x32x2_f32: lane l supplies A[row l%32][k l/32] and B[k l/32][col l%32]; accumulator register r of
@@ -28,12 +29,10 @@
 //
 // NN/ = Neural_Network_Library_Windows/Source_Files/Neural_Network/.
 #include "myea_kernels.h"
+#include "myea_split.h"
 
 namespace myea {
 namespace {
-
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kThreads = 256;
 constexpr int kFwdStages = 2, kBwdStages = 4;   // LDS stages (of 32 k) per wavefront
@@ -349,6 +348,145 @@ __global__ __launch_bounds__(kThreads) void transpose_kernel(size_t rows, size_t
 
 bool aligned16(const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15u) == 0; }
 
+// ---- any width ---------------------------------------------------------------------------------------------------
+// The step of a layer whose width is no multiple of 32, as long as it is small: one launch instead of a contraction (its slabs)
+// and a gate kernel.  Nothing but the launches and the latency of the first loads bounds such a step (200 cells, 60 examples:
+// 5.9 + 5.3 us forward, 5.5 + 5.2 us backward as two launches), so the wavefronts of a workgroup share k in runs of 32, every
+// lane takes the operands it multiplies straight from memory (any alignment) and splits them for the BF16 matrix cores, the
+// partial tiles meet in LDS once, and 256 lanes finish a pair (example, cell) each, having asked for what the gate math reads
+// before the first run.  A pair whose sum is not finite computes it again in FP32.
+constexpr int kStepForwardWaves = 8, kStepBackwardWaves = 16;
+
+// Tile: 32 examples x 8 cells; column j of the tile is gate j / 8 of cell j % 8.
+__global__ __launch_bounds__(64 * kStepForwardWaves) void lstm_step_forward_kernel(LstmFusedForward p)
+{
+    __shared__ f32x4 parts[kStepForwardWaves][4][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lane32 = lane & 31, half = lane >> 5;
+    const int C = (int)p.C, B = (int)p.B, ntc = (C + 7) / 8;
+    const int c0 = (int)blockIdx.x % ntc * 8, r0 = (int)blockIdx.x / ntc * 32;
+    const int row = (threadIdx.x >> 3) & 31, cell = threadIdx.x & 7, b = min(r0 + row, B - 1), c = min(c0 + cell, C - 1);
+    const bool mine = threadIdx.x < 256 && r0 + row < B && c0 + cell < C;
+    float e_in[4] = {0.f, 0.f, 0.f, 0.f}, e_peep[3] = {0.f, 0.f, 0.f}, e_cp = 0.f;
+    if (mine) {
+#pragma unroll
+        for (int gate = 0; gate < 4; ++gate) e_in[gate] = p.acts[(size_t)b * 4 * C + gate * C + c];
+#pragma unroll
+        for (int gate = 0; gate < 3; ++gate) e_peep[gate] = p.peep[gate * C + c];
+        e_cp = p.c_prev[(size_t)b * C + c];
+    }
+    const float *a_row = p.h_prev + (size_t)min(r0 + lane32, B - 1) * C;
+    const float *b_row = p.Wrec + ((size_t)(lane32 >> 3) * C + min(c0 + (lane32 & 7), C - 1)) * C;
+    f32x16 acc, small;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = small[r] = 0.f;
+    for (int k0 = wave * 32; k0 < C; k0 += 32 * kStepForwardWaves) {
+        float a[2][8], w[2][8];
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+            const int k = k0 + g * 16 + half * 8;
+            load_eight<true>(a[g], a_row + k, 0, k, C);
+            load_eight<true>(w[g], b_row + k, 0, k, C);
+        }
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+            bf16x8 pa[3], pb[3];
+            split_eight(a[g], pa);
+            split_eight(w[g], pb);
+#pragma unroll
+            for (int q = 0; q < 5; ++q) small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pa[kSmallA[q]], pb[kSmallB[q]], small, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pa[0], pb[0], acc, 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+        parts[wave][r][lane] = (f32x4){acc[r * 4] + small[r * 4], acc[r * 4 + 1] + small[r * 4 + 1], acc[r * 4 + 2] + small[r * 4 + 2], acc[r * 4 + 3] + small[r * 4 + 3]};
+    __syncthreads();
+    if (!mine) return;
+    float s[4];
+#pragma unroll
+    for (int gate = 0; gate < 4; ++gate) {
+        s[gate] = 0.f;
+#pragma unroll
+        for (int w = 0; w < kStepForwardWaves; ++w) s[gate] += parts[w][row >> 3][((row >> 2) & 1) * 32 + gate * 8 + cell][row & 3];
+        if (!(fabsf(s[gate]) < INFINITY)) {
+            s[gate] = 0.f;
+            for (int k = 0; k < C; ++k) s[gate] = fmaf(p.h_prev[(size_t)b * C + k], p.Wrec[((size_t)gate * C + c) * C + k], s[gate]);
+        }
+        s[gate] += e_in[gate];
+        s[gate] += p.bias[gate * C + c];
+    }
+    const float z = tanh_f(s[0]), gi = sigmoid_f(s[1] + e_cp * e_peep[0]), gf = sigmoid_f(s[2] + e_cp * e_peep[1]);
+    float cs = z * gi + gf * e_cp;
+    if (p.zone_state && !p.zone_state[c]) cs = e_cp;
+    const float ca = tanh_f(cs), go = sigmoid_f(s[3] + cs * e_peep[2]);
+    float hv = ca * go;
+    if (p.zone_output && !p.zone_output[c]) hv = p.h_prev[(size_t)b * C + c];
+    float *acts = p.acts + (size_t)b * 4 * C + c;
+    acts[0] = z; acts[C] = gi; acts[2 * C] = gf; acts[3 * C] = go;
+    p.c[(size_t)b * C + c] = cs; p.ca[(size_t)b * C + c] = ca; p.h[(size_t)b * C + c] = hv;
+}
+
+// Tile: 16 examples x 16 cells of dh, k = 4 C.
+__global__ __launch_bounds__(64 * kStepBackwardWaves) void lstm_step_backward_kernel(LstmFusedBackward p)
+{
+    __shared__ f32x4 parts[kStepBackwardWaves][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lane16 = lane & 15, quad = lane >> 4;
+    const int C = (int)p.C, B = (int)p.B, G = 4 * C, ntc = (C + 15) / 16;
+    const int c0 = (int)blockIdx.x % ntc * 16, r0 = (int)blockIdx.x / ntc * 16;
+    const int row = (threadIdx.x >> 4) & 15, cell = threadIdx.x & 15, b = min(r0 + row, B - 1), c = min(c0 + cell, C - 1);
+    const bool mine = threadIdx.x < 256 && r0 + row < B && c0 + cell < C;
+    const size_t at_c = (size_t)b * C + c, at_g = (size_t)b * G + c;
+    float gate[4] = {0.f, 0.f, 0.f, 0.f}, peep[3] = {0.f, 0.f, 0.f}, ca = 0.f, dh = 0.f, di_n = 0.f, df_n = 0.f, f_n = 0.f, dc_n = 0.f, cp = 0.f;
+    if (mine) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g) gate[g] = p.acts[at_g + g * C];
+#pragma unroll
+        for (int g = 0; g < 3; ++g) peep[g] = p.peep[g * C + c];
+        ca = p.ca[at_c]; dh = p.dh[at_c];
+        di_n = p.dG_next[at_g + C]; df_n = p.dG_next[at_g + 2 * C]; f_n = p.acts_next[at_g + 2 * C]; dc_n = p.dc_next[at_c];
+        if (!p.first_step) cp = p.c_prev[at_c];
+    }
+    const float *a_row = p.dG_next + (size_t)min(r0 + lane16, B - 1) * G;
+    const float *b_col = p.Wrec + min(c0 + lane16, C - 1);
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f}, small = {0.f, 0.f, 0.f, 0.f};
+    for (int k0 = wave * 32; k0 < G; k0 += 32 * kStepBackwardWaves) {
+        const int k = k0 + quad * 8;
+        float a[8], w[8];
+        load_eight<true>(a, a_row + k, 0, k, G);
+        load_eight<false>(w, b_col + (size_t)k * C, C, k, G);
+        bf16x8 pa[3], pb[3];
+        split_eight(a, pa);
+        split_eight(w, pb);
+#pragma unroll
+        for (int q = 0; q < 5; ++q) small = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pa[kSmallA[q]], pb[kSmallB[q]], small, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pa[0], pb[0], acc, 0, 0, 0);
+    }
+    parts[wave][lane] = acc + small;   // register r of lane l: row (l / 16) * 4 + r, column l % 16
+    __syncthreads();
+    if (!mine) return;
+    float s = 0.f;
+#pragma unroll
+    for (int w = 0; w < kStepBackwardWaves; ++w) s += parts[w][(row >> 2) * 16 + cell][row & 3];
+    if (!(fabsf(s) < INFINITY)) {
+        s = 0.f;
+        for (int k = 0; k < G; ++k) s = fmaf(p.dG_next[(size_t)b * G + k], p.Wrec[(size_t)k * C + c], s);
+    }
+    const float v = dh + s, z = gate[0], gi = gate[1], gf = gate[2], go = gate[3];
+    p.dh[at_c] = v;
+    const float ddo = go * (1.f - go) * (v * ca);
+    float e = v * go * (1.f - ca * ca);
+    e += peep[2] * ddo;
+    e += peep[0] * di_n;
+    e += peep[1] * df_n;
+    e += dc_n * f_n;
+    p.dc[at_c] = e;
+    float *dG = p.dG + at_g;
+    dG[0] = e * gi * (1.f - z * z);
+    dG[C] = e * z * (gi * (1.f - gi));
+    dG[2 * C] = p.first_step ? 0.f : e * cp * (gf * (1.f - gf));
+    dG[3 * C] = ddo;
+}
+
 }  // namespace
 
 bool lstm_fused_supported(size_t C, size_t cells_per_block) { return cells_per_block == 1 && C >= 32 && C % 32 == 0 && C <= (1u << 20); }
@@ -417,6 +555,29 @@ int launch_transpose(hipStream_t s, size_t rows, size_t cols, const float *src, 
 {
     if (rows == 0 || cols == 0) return MYEA_OK;
     hipLaunchKernelGGL(transpose_kernel, dim3((unsigned)((cols + 31) / 32), (unsigned)((rows + 31) / 32)), dim3(kThreads), 0, s, rows, cols, src, dst);
+    MYEA_HIP_TRY(hipGetLastError());
+    return MYEA_OK;
+}
+
+// One workgroup per compute unit at most in either direction: beyond that the operands that every tile reads for itself cost more
+// than the launch that is saved (512 examples of 1000 cells would read 1 GB a step).
+bool lstm_step_fits(size_t C, size_t cells_per_block, size_t B)
+{
+    return cells_per_block == 1 && C > 0 && B > 0 && (B + 31) / 32 * ((C + 7) / 8) <= 256 && (B + 15) / 16 * ((C + 15) / 16) <= 256;
+}
+
+int launch_lstm_step_forward(hipStream_t s, const LstmFusedForward &p)
+{
+    if (!lstm_step_fits(p.C, 1, p.B)) { set_last_error("LSTM step: %zu x %zu is not its shape", p.B, p.C); return MYEA_E_INVALID; }
+    hipLaunchKernelGGL(lstm_step_forward_kernel, dim3((unsigned)((p.B + 31) / 32 * ((p.C + 7) / 8))), dim3(64 * kStepForwardWaves), 0, s, p);
+    MYEA_HIP_TRY(hipGetLastError());
+    return MYEA_OK;
+}
+
+int launch_lstm_step_backward(hipStream_t s, const LstmFusedBackward &p)
+{
+    if (!lstm_step_fits(p.C, 1, p.B)) { set_last_error("LSTM step: %zu x %zu is not its shape", p.B, p.C); return MYEA_E_INVALID; }
+    hipLaunchKernelGGL(lstm_step_backward_kernel, dim3((unsigned)((p.B + 15) / 16 * ((p.C + 15) / 16))), dim3(64 * kStepBackwardWaves), 0, s, p);
     MYEA_HIP_TRY(hipGetLastError());
     return MYEA_OK;
 }
