@@ -735,8 +735,7 @@ int launch_short(hipStream_t stream, GemmDev d, bool a_kc, bool b_kc)
 
 // ---- a narrow product ---------------------------------------------------------------------------------------------------
 // C [M][N] = A B with N <= 32 and K <= 64 - a layer of an independently recurrent stack over T x batch rows, forward or backward.
-// The tiled kernel spends such a launch on its set-up, its predicated scalar loads and its stages (rows of 31 floats are no
-// 16-byte multiples): a few microseconds of instructions fetched to be run once.  Here a wavefront owns 32 rows of C: the
+// The tiled kernel spends such a launch on its set-up and its stages: a few microseconds of instructions fetched to be run once.  Here a wavefront owns 32 rows of C: the
 // lane's operands of v_mfma_f32_32x32x2f32 are asked for straight from memory, all of a round of 32 k's together (A: lane l
 // takes row l % 32 at k + l / 32; B: column l % 32), then the round's 16 matrix instructions; no LDS, one round or two.  The
 // accumulator has the layout of the tiled kernel's, so its epilogue (store_tile_kind) finishes the tile: every kind of
@@ -777,7 +776,7 @@ __global__ __launch_bounds__(kThreads) void narrow_gemm_kernel(GemmDev p)
 // loads and one matrix instruction per pair of rows, no LDS, no tile edges to test; a loop of a few dozen instructions.
 // The wavefronts of a workgroup add their 32 x 32 accumulators in wavefront order and store one slab [H][In]; the slabs
 // are added by launch_slab_sum_add, as the slabs of a split-K launch are.  (The tiled kernel spends its time on such a
-// shape in its set-up, its predicated scalar loads of operands whose rows are not 16-byte multiples, and its epilogue.)
+// shape in its set-up and its epilogue.)
 constexpr int kNarrowAhead = 16;   // pairs of rows a wavefront asks for at once: its whole share when the launch is not capped
 constexpr int kNarrowWaves = 8;    // wavefronts a workgroup: fewer slabs to add afterwards
 __global__ __launch_bounds__(64 * kNarrowWaves) void narrow_dw_kernel(const float *__restrict__ delta, const float *__restrict__ x, float *__restrict__ slabs,
@@ -989,9 +988,8 @@ int launch_gemm(hipStream_t stream, const GemmParams &p)
     return launch_layout<128, 64>(stream, d, a_kc, b_kc);
 }
 
-// `a` = (A k-contiguous, B n-contiguous), `b` = (both k-strided), neither split along k, 16-byte aligned operands, and `a`
-// no more than about one 128 x 128 tile per CU: both in ONE launch (gemm_pair_kernel).  Returns MYEA_OK when launched,
-// 1 when the pair form does not apply (the caller launches the two one after the other), a negative code on an error.
+// `a` = (A k-contiguous, B n-contiguous), `b` = (both k-strided), neither split along k, any alignment, and `a` no
+// more than about one 128 x 128 tile per CU: both in ONE launch (gemm_pair_kernel).  Returns MYEA_OK when launched, 1 when the pair form does not apply (the caller launches the two one after the other), a negative code on an error.
 int launch_gemm_pair(hipStream_t stream, const GemmParams &a, const GemmParams &b)
 {
     if (!a.a_k_contiguous || a.b_k_contiguous || b.a_k_contiguous || b.b_k_contiguous || a.split_k > 1 || b.split_k > 1) return 1;
@@ -1011,8 +1009,8 @@ int launch_gemm_pair(hipStream_t stream, const GemmParams &a, const GemmParams &
     };
     constexpr size_t lds_b = 2 * stage_bytes<128, 128>();
     if (fits(128)) {
-        // beside a long dX of 128 x 128 tiles the adds at the L2 were measured faster than stores (4096-wide layers at batch
-        // 1024: 475 against 482 us); everywhere else a store onto known zeros wins
+        // beside a long dX of 128 x 128 tiles adds at the L2 and stores take the same time (4096-wide layers at a batch of 1024:
+        // 27.45 and 27.35 ms for eight steps); everywhere else a store onto known zeros wins
         static const int store128 = [] { const char *e = std::getenv("MYEA_DW_STORE_PAIR128"); return e ? std::atoi(e) : 0; }();
         if (b.accumulate && !store128) db.accumulate = 1;
         da.nbm = (a.M + 127) / 128; da.nbn = (a.N + 127) / 128;

@@ -61,3 +61,21 @@ def test_short_products_against_float64(a_kc, b_kc, M, N, K):
     _gemm(mb.load_library(), a_kc, b_kc, 0, M, N, K, Ad, Bd, C)
     bound = 2.0 ** -23 * (-(-K // 16) + 8) * (A.double().abs() @ B.double().abs())
     assert bool(((C.double() - A.double() @ B.double()).abs() <= bound).all())
+
+
+def test_pair_of_odd_widths_matches_the_separate_launches():
+    """Rows that are no 16-byte multiples ride in the paired launch too: 128 tiles of dX beside 256 of dW, bit for bit."""
+    from tests.test_gpu_paired_backward import _pair, _step
+    B = 1021
+    specs = [dict(units=2045), dict(units=2047, activation="RELU"), dict(units=2047, activation="TANH"), dict(units=5, activation="LINEAR")]
+    desc, (a, b), X, Y, _ = _pair(specs, B)
+    b.profile_enable(True)
+    for _ in range(2):
+        _step(a, B, X, Y, fused=False)
+        _step(b, B, X, Y, fused=True)
+    pairs = b.profile_read(4)
+    b.profile_enable(False)
+    assert pairs[0] >= 2, pairs
+    assert np.array_equal(a.download_gradient(), b.download_gradient())
+    for li in range(1, desc.n_layers):
+        assert np.array_equal(a.download_tensor(li, mb.TENSOR["ERRORS"]), b.download_tensor(li, mb.TENSOR["ERRORS"]))
