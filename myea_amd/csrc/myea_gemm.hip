@@ -822,30 +822,45 @@ __global__ __launch_bounds__(64 * kNarrowWaves) void narrow_dw_kernel(const floa
 
 // Number of K slabs for a contraction whose M x N alone does not fill the chip; 1 when the plain launch already does.
 // Short k: about one workgroup per CU with 64 x 64 tiles, each slab at least 128 k's deep.
-int gemm_split_k(int M, int N, int K)
+static long split_k_wanted(int M, int N, int K)
 {
     const long tiles_128 = (long)((M + 127) / 128) * ((N + 127) / 128);
     if (tiles_128 * 2 >= 256) return 1;
-    long want;
+    long want, most = 16;
     if (K >= 4096) {
         // long k (weight gradients over T x batch rows): enough slabs for ~1000 workgroups of 128 x 64, each slab at least
         // 1024 k's deep - the larger tile's operand reuse is worth more than the pass over the slabs that sums them
-        want = (512 + tiles_128 - 1) / tiles_128;
         // (a product no larger than one 64 x 64 tile has no operand reuse to protect: slabs 256 k's deep, up to 32 of them)
-        const long depth = (M <= 64 && N <= 64) ? 256 : 1024;
-        if (want > K / depth) want = K / depth;
-        if (depth == 256) { if (want > 32) want = 32; if (want < 1) want = 1; const int c = (int)(((K + want - 1) / want + kBK - 1) / kBK * kBK); return (K + c - 1) / c; }
+        const bool one_tile = M <= 64 && N <= 64;
+        want = (512 + tiles_128 - 1) / tiles_128;
+        const long by_k = K / (one_tile ? 256 : 1024);
+        if (want > by_k) want = by_k;
+        if (one_tile) most = 32;
     } else {
         const long tiles_64 = (long)((M + 63) / 64) * ((N + 63) / 64);
         want = (256 + tiles_64 - 1) / tiles_64;
         const long max_by_k = K / 128 > 0 ? K / 128 : 1;
         if (want > max_by_k) want = max_by_k;
     }
-    if (want > 16) want = 16;
-    if (want < 1) want = 1;
+    if (want > most) want = most;
+    return want < 1 ? 1 : want;
+}
+
+int gemm_split_k(int M, int N, int K)
+{
+    const long want = split_k_wanted(M, N, K);
+    if (want == 1) return 1;
     // the launcher rounds the chunk up to a multiple of 32: return the slab count that rounding produces
     const int chunk = (int)(((K + want - 1) / want + kBK - 1) / kBK * kBK);
     return (K + chunk - 1) / chunk;
+}
+
+// No k up to K takes more slabs than this: what a workspace for them is sized by.  (Fewer k's may take more of them: 16 at 4095,
+// 4 at 4096.  On either side of that line the wanted number only grows with k, and the rounding of the chunk only lowers it.)
+int gemm_split_k_most(int M, int N, int K)
+{
+    const long shallow = split_k_wanted(M, N, K < 4095 ? K : 4095), deep = split_k_wanted(M, N, K);
+    return (int)(shallow > deep ? shallow : deep);
 }
 
 unsigned gemm_pair_polls()
@@ -911,14 +926,22 @@ static int prepare_gemm(const GemmParams &p, GemmDev &d)
 
 // Slabs the narrow weight-gradient kernel writes for these shapes: 0 when the shape is not its own (the tiled kernel takes it).
 // A wavefront gets at least 32 rows (one round of loads), a launch at most 128 workgroups.
+constexpr int kNarrowSlabs = 128;
 int narrow_dw_slabs(size_t H, size_t In, size_t rows)
 {
     if (H == 0 || In == 0 || H > 32 || In > 32 || rows < 512 || rows > 0x7fffffffu) return 0;
     static const bool off = [] { const char *e = std::getenv("MYEA_NARROW_DW"); return e && e[0] == '0'; }();
     if (off) return 0;
     size_t per_wave = 2 * kNarrowAhead;
-    while ((rows + kNarrowWaves * per_wave - 1) / (kNarrowWaves * per_wave) > 128) per_wave *= 2;
+    while ((rows + kNarrowWaves * per_wave - 1) / (kNarrowWaves * per_wave) > kNarrowSlabs) per_wave *= 2;
     return (int)((rows + kNarrowWaves * per_wave - 1) / (kNarrowWaves * per_wave));
+}
+
+// No number of rows up to `rows` takes more: 128 at 32768 rows, 65 at 32769.
+int narrow_dw_slabs_most(size_t H, size_t In, size_t rows)
+{
+    constexpr size_t full = (size_t)kNarrowSlabs * kNarrowWaves * 2 * kNarrowAhead;   // the most rows that every wavefront takes in one round
+    return narrow_dw_slabs(H, In, rows < full ? rows : full);
 }
 
 // delta [rows][H], x [rows][In], both dense; slabs: narrow_dw_slabs(H, In, rows) x [H][In]

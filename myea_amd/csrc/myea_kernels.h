@@ -74,6 +74,7 @@ struct GemmParams {
 constexpr int kGemmPairTiles = 256;   // tiles the two buffers above serve
 
 int gemm_split_k(int M, int N, int K);
+int gemm_split_k_most(int M, int N, int K);   // the largest of any k up to K: what a workspace is sized by
 // polls a tile's second workgroup waits for the first: 2^24 (seconds), or MYEA_GEMM_PAIR_SPIN_POLLS (0: give up at once, for tests
 // of that path; read at every call)
 unsigned gemm_pair_polls();
@@ -86,6 +87,7 @@ int launch_gemm(hipStream_t stream, const GemmParams &p);
 // The weight gradient delta^T X of a layer with at most 32 outputs and 32 inputs over many rows, as slabs [H][In] to be added:
 // narrow_dw_slabs gives their number (0: not this kernel's shape), launch_narrow_dw writes them.
 int narrow_dw_slabs(size_t H, size_t In, size_t rows);
+int narrow_dw_slabs_most(size_t H, size_t In, size_t rows);   // the largest of any number of rows up to this one
 int launch_narrow_dw(hipStream_t stream, const float *delta, const float *x, float *slabs, size_t H, size_t In, size_t rows);
 // dX = delta W (`a`) and dW += delta^T X (`b`) in one launch when their shapes suit it; MYEA_OK = launched, 1 = does not
 // apply (launch them one after the other), negative = error

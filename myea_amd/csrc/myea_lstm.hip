@@ -76,7 +76,13 @@ namespace {
         if (rc__ != MYEA_OK) return rc__; \
     } while (0)
 
-constexpr size_t kMaxSlabs = 16;
+// Slabs that the weight gradient of one LSTM operand (G x width, k over up to `rows` rows) may take: room for 16, and for the 32 of a
+// product no larger than one 64 x 64 tile where the rows are long enough for more than 16.
+size_t gradient_slabs(size_t G, size_t width, size_t rows)
+{
+    const int most = gemm_split_k_most((int)G, (int)width, rows < 0x7fffffffu ? (int)rows : 0x7fffffff);
+    return most > 16 ? (size_t)most : 16;
+}
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 struct LstmGeom {
@@ -1203,8 +1209,8 @@ int Net::lstm_create_layer(size_t li)
         q->fused = !q->norm && lstm_fused_supported(q->C, q->cpb) && !fused_lstm_disabled();
         if (q->fused) MYEA_TRY(dev_alloc_zero(&q->WrecT, q->C * q->G));
         if (q->fused) MYEA_TRY(dev_alloc_zero(&q->sums, (B + 31) / 32 * 7 * q->C));
-        MYEA_TRY(dev_alloc_zero(&q->gWin, kMaxSlabs * q->G * q->In));   // split-K slabs of the weight-gradient contractions
-        MYEA_TRY(dev_alloc_zero(&q->gWrec, kMaxSlabs * q->G * q->C));
+        MYEA_TRY(dev_alloc_zero(&q->gWin, gradient_slabs(q->G, q->In, T * B) * q->G * q->In));   // split-K slabs of the weight-gradient contractions
+        MYEA_TRY(dev_alloc_zero(&q->gWrec, gradient_slabs(q->G, q->C, T * B) * q->G * q->C));
         q->gWin_own = q->gWin; q->gWrec_own = q->gWrec;
         if (T > 1 && gemm_pair_k_128((int)q->G, (int)q->C, (int)((T - 1) * B))) {
             MYEA_TRY(dev_alloc_zero(&q->pair_partials, (size_t)kGemmPairTiles * 128 * 128));
@@ -1263,23 +1269,27 @@ size_t Net::lstm_scratch_floats() const
 
 static size_t round_up_64(size_t n) { return (n + 63) / 64 * 64; }
 
-size_t Net::lstm_gradient_slab_floats() const
+// rows of one weight-gradient contraction of an LSTM layer: a partial batch over several time steps takes one per time step, unsplit
+size_t Net::lstm_gradient_rows(size_t B) const { return d.number_recurrent_depth > 1 && B != d.batch_size ? 1 : d.number_recurrent_depth * B; }
+
+size_t Net::lstm_gradient_slab_floats(size_t B) const
 {
+    const size_t rows = lstm_gradient_rows(B);
     size_t need = 0;
     for (const DevLayer &o : L)
         for (const LstmLayer *q : {o.lstm, o.lstm2})
-            if (q) need += round_up_64(kMaxSlabs * q->G * q->In) + round_up_64(kMaxSlabs * q->G * q->C);
+            if (q) need += round_up_64(gradient_slabs(q->G, q->In, rows) * q->G * q->In) + round_up_64(gradient_slabs(q->G, q->C, rows) * q->G * q->C);
     return need;
 }
 
-void Net::lstm_bind_gradient_slabs(float *base)
+void Net::lstm_bind_gradient_slabs(float *base, size_t B)
 {
     for (DevLayer &o : L)
         for (LstmLayer *q : {o.lstm, o.lstm2}) {
             if (!q) continue;
             if (!base) { q->gWin = q->gWin_own; q->gWrec = q->gWrec_own; continue; }
-            q->gWin = base; base += round_up_64(kMaxSlabs * q->G * q->In);
-            q->gWrec = base; base += round_up_64(kMaxSlabs * q->G * q->C);
+            q->gWin = base; base += round_up_64(gradient_slabs(q->G, q->In, lstm_gradient_rows(B)) * q->G * q->In);
+            q->gWrec = base; base += round_up_64(gradient_slabs(q->G, q->C, lstm_gradient_rows(B)) * q->G * q->C);
         }
 }
 

@@ -249,8 +249,10 @@ struct Net {
     size_t lstm_scratch_floats() const;
     // packed weight-gradient slabs of all LSTM directions: their total size (each rounded up to 64 floats), and
     // re-pointing them into `base` (null: back to the layers' own buffers)
-    size_t lstm_gradient_slab_floats() const;
-    void lstm_bind_gradient_slabs(float *base);
+    size_t lstm_gradient_rows(size_t B) const;
+    size_t lstm_gradient_slab_floats(size_t B) const;
+    void lstm_bind_gradient_slabs(float *base, size_t B);
+    size_t fc_dw_slab_floats(size_t B) const;
     int lstm_update_derivative_weight(size_t li, size_t B, bool reductions);
     int lstm_update_derivative_weight_reductions(LstmLayer &q, size_t B);
     const float *lstm_tensor(size_t li, int kind, size_t *count);

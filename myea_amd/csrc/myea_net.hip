@@ -238,7 +238,8 @@ static int check_desc(const myea_net_desc &d)
     return MYEA_OK;
 }
 
-static int fc_dw_slabs(size_t H, size_t In, size_t rows, size_t first_connection_index);
+static int fc_dw_slabs(size_t H, size_t In, size_t rows);
+static int fc_dw_slabs_most(size_t H, size_t In, size_t rows);
 
 int Net::create(const myea_net_desc &desc)
 {
@@ -402,11 +403,12 @@ int Net::create(const myea_net_desc &desc)
         MYEA_TRY(dev_alloc(&scratch, need));
         scratch_floats = need;
     }
-    {   // weight gradients of narrow layers over long T x batch row ranges run as split-K contractions into slabs
+    {   // weight gradients of narrow layers over long T x batch row ranges run as split-K contractions into slabs; a smaller batch
+        // may take more of them than the largest
         size_t need = 0;
         for (size_t li = 1; li < d.n_layers; ++li) {
             if (!layer_is_dense(d.layers[li])) continue;
-            const int slabs = fc_dw_slabs(L[li].H, L[li].In, T * B, d.layers[li].first_connection_index);
+            const int slabs = fc_dw_slabs_most(L[li].H, L[li].In, T * B);
             if (slabs > 1) need = std::max(need, (size_t)slabs * L[li].H * L[li].In);
         }
         if (need) MYEA_TRY(dev_alloc(&dw_slabs, need));
@@ -416,7 +418,7 @@ int Net::create(const myea_net_desc &desc)
         size_t pool = 0, count = 0;
         for (size_t li = 1; li < d.n_layers; ++li) {
             if (!layer_is_dense(d.layers[li])) continue;
-            const int slabs = narrow_dw_slabs(L[li].H, L[li].In, T * B);
+            const int slabs = narrow_dw_slabs_most(L[li].H, L[li].In, T * B);
             if (slabs > 0) { narrow_slab_at[li] = pool; pool += ((size_t)slabs * L[li].H * L[li].In + 63) / 64 * 64; ++count; }
             if (L[li].du_rows) ++count;   // the shares of an independently recurrent layer's self weights go through the same table
         }
@@ -1430,9 +1432,8 @@ int Net::backward_pass(size_t B)
 // FF__Update_Derivative_Weight_Batch (NN/Neural_Network__Update_Derivative_Weight__OpenMP.cpp:24-59):
 // dW += delta^T X (:178-216) with X = the previous layer's post-dropout outputs, db += column sums (:218-242).
 // slabs of the split-K form of a fully-connected layer's weight gradient; 1 = the plain accumulating contraction
-static int fc_dw_slabs(size_t H, size_t In, size_t rows, size_t first_connection_index)
+static int fc_dw_slabs(size_t H, size_t In, size_t rows)
 {
-    (void)first_connection_index;
     if (rows > 0x7fffffffu) return 1;
     const int narrow = narrow_dw_slabs(H, In, rows);   // a narrow layer's kernel of its own: always through slabs
     if (narrow > 0) return narrow > 1 ? narrow : 2;    // (room for two, so that "more than one slab" still says "through slabs")
@@ -1440,6 +1441,26 @@ static int fc_dw_slabs(size_t H, size_t In, size_t rows, size_t first_connection
     // has four runs of 32 rows at most (37 x 1201 over 333 rows: 11 + 4 us through two slabs, 7 us so).
     if (rows < 1024) return 1;
     return gemm_split_k((int)H, (int)In, (int)rows);
+}
+
+// no number of rows up to `rows` takes more slabs
+static int fc_dw_slabs_most(size_t H, size_t In, size_t rows)
+{
+    const int narrow = narrow_dw_slabs_most(H, In, rows), split = rows < 1024 ? 1 : gemm_split_k_most((int)H, (int)In, (int)std::min<size_t>(rows, 0x7fffffffu));
+    return std::max(narrow > 1 ? narrow : 2 * narrow, split);
+}
+
+// what the dense layers' weight gradients write into dw_slabs for a batch of B
+size_t Net::fc_dw_slab_floats(size_t B) const
+{
+    const size_t T = d.number_recurrent_depth, rows = T > 1 && B != d.batch_size ? B : T * B;
+    size_t need = 0;
+    for (size_t li = 1; li < d.n_layers; ++li) {
+        if (!layer_is_dense(d.layers[li])) continue;
+        const int slabs = fc_dw_slabs(L[li].H, L[li].In, rows);
+        if (slabs > 1) need = std::max(need, (size_t)slabs * L[li].H * L[li].In);
+    }
+    return need;
 }
 
 // the weight gradient of fully-connected layer li as one accumulating contraction dW += delta^T X (false when it takes the
@@ -1451,7 +1472,7 @@ bool Net::fc_dw_params(size_t li, size_t B, GemmParams *out)
     const size_t T = d.number_recurrent_depth, Bmax = d.batch_size, In = o.In, H = o.H;
     if (T > 1 && B != Bmax) return false;
     const size_t rows = T > 1 ? T * B : B;
-    if (dw_slabs && fc_dw_slabs(H, In, rows, l.first_connection_index) > 1) return false;
+    if (dw_slabs && fc_dw_slabs(H, In, rows) > 1) return false;
     const float *x = layer_outputs(o.prev);
     if (o.group == 2) x = o.values;
     else if (o.group == 1 && layer_uses_norm(l)) x = o.normalizes;
@@ -1495,9 +1516,13 @@ int Net::update_derivative_weight_contraction(size_t li, size_t B)
         g.C = gradient + l.first_connection_index; g.ldc = (long)In;
         g.M = (int)H; g.N = (int)In; g.K = (int)rows;
         g.accumulate = 1; g.c_is_zero = dw_may_store(li) ? 1 : 0; g.epilogue = EPI_NONE;
-        int slabs = dw_slabs ? fc_dw_slabs(H, In, rows, l.first_connection_index) : 1;
+        int slabs = dw_slabs ? fc_dw_slabs(H, In, rows) : 1;
         const int narrow = dw_slabs ? narrow_dw_slabs(H, In, rows) : 0;
         if (slabs > 1) { g.C = dw_slabs; g.accumulate = 0; g.c_is_zero = 0; g.split_k = slabs; g.split_k_slab = (long)(H * In); }
+        if ((size_t)std::max(slabs, narrow) * H * In > dw_slab_floats && (slabs > 1 || narrow > 0)) {
+            set_last_error("layer %zu: %d slabs of a weight gradient over %zu rows do not fit their workspace", li, std::max(slabs, narrow), rows);
+            return MYEA_E_INVALID;
+        }
         if (li < dw_zero.size()) dw_zero[li] = 0;   // from here on the slice holds this product, stored or added from the slabs
         prof_begin(2);
         // a narrow layer over all of its rows: the slabs wait in the layer's slice for the one launch that adds every layer's
@@ -1625,7 +1650,9 @@ int Net::update_derivative_weight(size_t B, size_t first, size_t end)
 int Net::update_derivative_weight_no_alloc(size_t B, size_t first, size_t end)
 {
     auto round_up = [](size_t n) { return (n + 63) / 64 * 64; };
-    const size_t need = round_up(scratch_floats) + round_up(dw_slab_floats) + lstm_gradient_slab_floats();
+    // (a network whose full batch does not fit is refused at every batch)
+    const size_t slab_floats = std::max(fc_dw_slab_floats(B), fc_dw_slab_floats(d.batch_size));
+    const size_t need = round_up(scratch_floats) + round_up(slab_floats) + std::max(lstm_gradient_slab_floats(B), lstm_gradient_slab_floats(d.batch_size));
     if (need > kStaticScratchFloats) {
         set_last_error("Update_Derivative_Weight (no allocation): this network's kernels need %zu bytes of scratch memory, the static buffer holds %zu",
                        need * sizeof(float), kStaticScratchFloats * sizeof(float));
@@ -1636,15 +1663,15 @@ int Net::update_derivative_weight_no_alloc(size_t B, size_t first, size_t end)
     float *at = static_scratch;
     scratch = at; at += round_up(scratch_floats);
     if (own_slabs) dw_slabs = at;
-    at += round_up(dw_slab_floats);
+    at += round_up(slab_floats);
     defer_folds = false;   // a narrow layer's slabs are added right behind its contraction: no table to upload, no wait for the stream
-    lstm_bind_gradient_slabs(at);
+    lstm_bind_gradient_slabs(at, B);
     const bool was_profiling = profiling;
     profiling = false;   // the profiling taps create events on demand
     const int rc = update_derivative_weight(B, first, end);
     profiling = was_profiling;
     scratch = own_scratch; dw_slabs = own_slabs; defer_folds = true;
-    lstm_bind_gradient_slabs(nullptr);
+    lstm_bind_gradient_slabs(nullptr, B);
     return rc;
 }
 
