@@ -7,9 +7,9 @@
 //   weights  dW += delta^T X     (A m-contiguous, B n-contiguous)   Update_Derivative_Weight__FC,
 //            Neural_Network__Update_Derivative_Weight__OpenMP.cpp:178-216
 //
-// Arithmetic.  gfx950 multiplies FP32 at 157 TFLOP/s and BF16 at 2.5 PFLOP/s.  An FP32 number IS the sum of three BF16 numbers:
-// hi = x rounded to BF16, mid = (x - hi) rounded to BF16, lo = what is left (8 + 8 + 8 significant bits, signs included, cover
-// the 24 of x; both differences are exact in FP32).  Of the nine products of two such sums the six with a weight above 2^-24 are
+// Arithmetic.  gfx950 multiplies FP32 at 157 TFLOP/s and BF16 at 2.5 PFLOP/s.  An FP32 number below 2^103 is the sum of three BF16
+// numbers, but for a power of two that keeps the smallest of them normal (myea_split.h): hi = x rounded to BF16, mid = (x - hi)
+// rounded to BF16, lo = what is left (8 + 8 + 8 significant bits, signs included, cover the 24 of x; both differences are exact in FP32).  Of the nine products of two such sums the six with a weight above 2^-24 are
 // formed - hi hi, hi mid, mid hi, mid mid, hi lo, lo hi - each exact in the matrix unit, all accumulated in FP32.  What is left
 // out is below 2^-25 of a product.  The five smaller products have an accumulator of their own, added at the end: an accumulator
 // as large as the result is rounded once per 16 k's, where v_mfma_f32_32x32x2_f32 rounds it at every second k, and the measured
@@ -19,14 +19,14 @@
 // 190 at the 1.14 PFLOP/s that a large BF16 product was measured to sustain on this card.  Measured, FP32 instruction -> this:
 // 1024 x 4096 x 4096 forward 314 -> 221 us, its weight gradient 304 -> 197 us (174 TFLOP/s), 16384 x 2048 x 512 269 -> 193 us
 // (178 TFLOP/s); 333 x 1201 x 1201, whose rows are no 16-byte multiples, 50 -> 25 us.
-// Infinities and NaN do not survive the split (inf - inf), nor do finite values that round to a BF16 infinity: such a product
+// Infinities and NaN do not survive the split (inf - inf), nor do finite values whose scaled hi is a BF16 infinity: such a product
 // always leaves a non-finite accumulator, and a wavefront that finds one computes its accumulators again with the FP32
 // instruction (redo_in_f32), so the results are those of FP32 arithmetic there too.
 //
 // Tiling: a workgroup of 256 lanes (4 wavefronts, 2 x 2) owns a BM x BN tile of C; each wavefront owns (BM/2) x (BN/2) as
 // TM x TN accumulators of v_mfma_f32_32x32x16_bf16 (16 VGPRs each).  A K step moves BK columns: global -> registers (asked for
 // two steps ahead or four), split there once, three BF16 planes -> LDS (two stages, one barrier per step).  What bounds a step is
-// issue: per 16 k's of a 128 x 128 tile a wavefront has 24 matrix instructions (768 cycles) and about 100 vector ones (400), so
+// issue: per 16 k's of a 128 x 128 tile a wavefront has 24 matrix instructions (768 cycles) and about 120 vector ones (480), so
 // the splitting of the next step is spread between the matrix instructions of this one (2048 x 2048 x 2048: 114 us with the
 // compiler's order, 98 us so).  An operand's place in LDS
 // does not depend on its orientation in memory:
@@ -401,15 +401,18 @@ __device__ __forceinline__ void gemm_tile(const GemmDev &p, const int block, cha
                     for (int j = 0; j < TN; ++j)
                         (q < 5 ? small[i][j] : acc[i][j]) = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[ks][pa[q]][i], fb[ks][pb[q]][j], q < 5 ? small[i][j] : acc[i][j], 0, 0, 0);
     };
-    // The order of a step's instructions: the fragments first, then a few of the splitting's between every two matrix instructions,
-    // which leave the wavefront idle otherwise (left alone the compiler splits everything before the first of them).
-    constexpr int kMatrix = 6 * TM * TN * (BK / 16), kWrites = 3 * (MA::S::kPerThread + MB::S::kPerThread), kSplit = 11 * 4 * (MA::S::kPerThread + MB::S::kPerThread);
+    // The order of a step's instructions: the fragments first, then some of the splitting's between every two matrix instructions,
+    // which leave the wavefront idle otherwise (left alone the compiler splits everything before the first of them).  A pair of
+    // elements takes 13 vector instructions; room for 32 is left, so that the splitting is done behind two fifths of the matrix
+    // instructions and its stores have the others to land behind (us at room for 13 -> 32: 512 x 2048 x 2048 40.6 -> 36.6,
+    // 1024 x 1000 x 4096 76 -> 68.7, 1024 x 4096 x 4096 194 -> 185).
+    constexpr int kMatrix = 6 * TM * TN * (BK / 16), kWrites = 3 * (MA::S::kPerThread + MB::S::kPerThread), kRoom = 32 * 4 * (MA::S::kPerThread + MB::S::kPerThread);
     auto interleave = [&]() {
         __builtin_amdgcn_sched_group_barrier(0x100, 3 * (TM + TN) * (BK / 16), 0);   // LDS reads
 #pragma unroll
         for (int q = 0; q < kMatrix; ++q) {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);           // a matrix instruction
-            __builtin_amdgcn_sched_group_barrier(0x002, (kSplit + kMatrix - 1) / kMatrix + 1, 0);   // vector arithmetic
+            __builtin_amdgcn_sched_group_barrier(0x002, (kRoom + kMatrix - 1) / kMatrix + 1, 0);   // vector arithmetic
             if (q % (kMatrix / kWrites) == kMatrix / kWrites - 1) __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);   // an LDS write
         }
     };
@@ -467,7 +470,7 @@ __device__ __forceinline__ void gemm_tile(const GemmDev &p, const int block, cha
             for (int j = 0; j < TN; ++j)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
-                    acc[i][j][r] += small[i][j][r];
+                    acc[i][j][r] = unscaled(acc[i][j][r] + small[i][j][r]);
                     finite = fmaf(acc[i][j][r], 0.f, finite);
                 }
         if (__any(finite != 0.f)) redo_in_f32<A_KC, B_KC, TM, TN>(p, acc, m0 + wave_m + lane32, n0 + wave_n + lane32, half, k_begin, k_end);
@@ -711,7 +714,10 @@ __global__ __launch_bounds__(64 * kShortWaves) void short_gemm_kernel(GemmDev p)
             for (int e = 0; e < 4; ++e) acc[0][0][r * 4 + e] += v[e];
         }
 #pragma unroll
-    for (int r = 0; r < 16; ++r) finite = fmaf(acc[0][0][r], 0.f, finite);
+    for (int r = 0; r < 16; ++r) {
+        acc[0][0][r] = unscaled(acc[0][0][r]);
+        finite = fmaf(acc[0][0][r], 0.f, finite);
+    }
     if (__any(finite != 0.f)) redo_in_f32<A_KC, B_KC, 1, 1>(p, acc, m0 + lane32, n0 + lane32, half, k_begin, k_end);
     const TilePlace at{m0, n0, 0, 0, lane32, half, (long)split * p.slab};
     if (m0 + 32 <= p.M && n0 + 32 <= p.N) store_tile_kind<true, 1, 1>(p, acc, at);

@@ -408,6 +408,7 @@ __global__ __launch_bounds__(64 * kStepForwardWaves) void lstm_step_forward_kern
         s[gate] = 0.f;
 #pragma unroll
         for (int w = 0; w < kStepForwardWaves; ++w) s[gate] += parts[w][row >> 3][((row >> 2) & 1) * 32 + gate * 8 + cell][row & 3];
+        s[gate] = unscaled(s[gate]);
         if (!(fabsf(s[gate]) < INFINITY)) {
             s[gate] = 0.f;
             for (int k = 0; k < C; ++k) s[gate] = fmaf(p.h_prev[(size_t)b * C + k], p.Wrec[((size_t)gate * C + c) * C + k], s[gate]);
@@ -467,6 +468,7 @@ __global__ __launch_bounds__(64 * kStepBackwardWaves) void lstm_step_backward_ke
     float s = 0.f;
 #pragma unroll
     for (int w = 0; w < kStepBackwardWaves; ++w) s += parts[w][(row >> 2) * 16 + cell][row & 3];
+    s = unscaled(s);
     if (!(fabsf(s) < INFINITY)) {
         s = 0.f;
         for (int k = 0; k < G; ++k) s = fmaf(p.dG_next[(size_t)b * G + k], p.Wrec[(size_t)k * C + c], s);

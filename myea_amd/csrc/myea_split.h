@@ -1,5 +1,12 @@
 // myea_split.h — an FP32 number as the sum of three BF16 numbers: what the kernels that multiply on the BF16 matrix cores share.
 // myea_gemm.hip says which products are formed and what that leaves of the error.
+//
+// Range.  BF16 has FP32's exponents but 8 bits: the third number of an operand below 2^-110 would fall among the subnormals and lose
+// bits (3.5e-5 of an operand of 2^-120, all of one below 2^-134).  So an operand is split as x * 2^24: the last bit of the smallest
+// FP32 subnormal becomes 2^-125, a normal number, and the sum is exact for every x below 2^103.  The sums of products come out times
+// 2^48 and go through unscaled() before anything else is done with them.  Larger operands and sums beyond 2^79 leave an infinity
+// or a NaN, and whoever finds one computes the sum again in FP32.  The two multiplications are 2 of the 13 vector instructions a pair
+// takes.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -17,9 +24,15 @@ typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));   // a 
 // the smaller five of the six products a_x b_y, in this order; hi hi has an accumulator of its own
 constexpr int kSmallA[5] = {0, 2, 1, 0, 1}, kSmallB[5] = {2, 0, 1, 1, 0};
 
+constexpr float kSplitScale = 0x1p24f, kSplitUnscale = 0x1p-48f;
+
+// an accumulator of products of two split operands -> the sum itself
+__device__ __forceinline__ float unscaled(float sum) { return sum * kSplitUnscale; }
+
 // two FP32 numbers -> the two BF16 numbers of each plane, packed
 __device__ __forceinline__ void split_pair(float x0, float x1, unsigned &hi, unsigned &mid, unsigned &lo)
 {
+    x0 *= kSplitScale; x1 *= kSplitScale;
     hi = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2){x0, x1}, bf16x2));
     const float r0 = x0 - __uint_as_float(hi << 16), r1 = x1 - __uint_as_float(hi & 0xffff0000u);
     mid = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2){r0, r1}, bf16x2));

@@ -34,6 +34,21 @@ def test_tiles_and_remainders_against_float64(a_kc, b_kc, M, N, K):
 
 
 @pytest.mark.parametrize("a_kc,b_kc", LAYOUTS)
+@pytest.mark.parametrize("M,N,K", [(100, 90, 300), (1000, 700, 97), (1500, 1501, 40), (2049, 2050, 40)])
+def test_small_operands_keep_their_bits(a_kc, b_kc, M, N, K):
+    """One operand down to FP32's subnormals, the other large or ordinary: the products are as exact as any, but for results that
+    are subnormal themselves (one rounding more, 2^-149)."""
+    A, B, _, _ = _operands(a_kc, b_kc, M, N, K, 11)
+    for at_a, at_b in ((-115, 100), (90, -126), (-140, 100), (-120, 0), (0, -146)):
+        a, b = (A.double() * 2.0 ** at_a).float(), (B.double() * 2.0 ** at_b).float()
+        C = torch.full((M, N), float("nan"), device="cuda")
+        _gemm(mb.load_library(), a_kc, b_kc, 0, M, N, K, (a if a_kc else a.t()).contiguous(), (b.t() if b_kc else b).contiguous(), C)
+        bound = 2.0 ** -23 * (-(-K // 16) + 8) * (a.double().abs() @ b.double().abs()) + 2.0 ** -149
+        inside = bool(((C.double() - a.double() @ b.double()).abs() <= bound).all())
+        assert inside, (at_a, at_b)
+
+
+@pytest.mark.parametrize("a_kc,b_kc", LAYOUTS)
 @pytest.mark.parametrize("M,N", [(100, 90), (1500, 1501), (2049, 2050)])
 def test_values_the_split_cannot_carry(a_kc, b_kc, M, N):
     K = 40

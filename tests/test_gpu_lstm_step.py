@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 
 from myea_amd import binding as mb
-from tests.common import assert_close, run_step
+from tests.common import assert_close, glorot_parameters, run_step
 from tests.test_gpu_lstm import ABS, REL, _compare, _pair
 
 pytestmark = pytest.mark.gpu
@@ -45,3 +45,36 @@ def test_infinite_weight_saturates_a_gate_as_in_fp32():
         gpu.upload_parameters(v)
         gpu.Forward_Pass(B, X)
         assert np.isfinite(gpu.download_tensor(1, mb.TENSOR["OUTPUTS"], T * B * cells)).all(), i
+
+
+@pytest.mark.parametrize("cells,B", [(9, 5), (130, 40)])
+def test_recurrent_weights_below_the_split_range_keep_their_bits(cells, B):
+    """Recurrent weights of 2^-120 between ordinary gate deltas: with no error from above at the first of two steps, dh there is
+    dG[1] Wrec alone, held against 64 bits (4 cells products: 2^-23 of their magnitudes per rounding, one per 32 k's and the sum of
+    the 16 wavefronts)."""
+    T, In = 2, 4
+    desc = mb.make_desc([dict(units=In), dict(type="lstm", units=cells), dict(units=cells, activation="LINEAR")], B, T)
+    net = mb.HipNetwork(desc, mb.default_hyper(type_loss_function=mb.LOSS["MSE"]))
+    net.set_state_propagation(mb.STATE_TRAINING)
+    w = glorot_parameters(desc, 4, bias_range=0.3)
+    layer, rows = desc.layers[1], In + cells
+    per_cell = w[layer.first_connection_index:layer.last_connection_index].reshape(cells, 4 * rows + 3)
+    # a cell's slice: its input row [In + cells], the three gates' rows from below, then their recurrent rows, the peepholes
+    recurrent = [per_cell[:, In:rows]] + [per_cell[:, rows + 3 * In + g * cells:rows + 3 * In + (g + 1) * cells] for g in range(3)]
+    for r in recurrent:
+        r *= np.float32(2.0 ** -120)
+    net.upload_parameters(w)
+    net.Clear_Training_Arrays()
+    X = np.random.default_rng(1).normal(0, 1, (B, T * In)).astype(np.float32)
+    net.Forward_Pass(B, X)
+    Y = net.download_tensor(2, mb.TENSOR["OUTPUTS"]).reshape(T, B, cells).copy()
+    Y[1] += np.random.default_rng(2).normal(0, 1, (B, cells)).astype(np.float32)
+    net.Compute__Error(B, np.ascontiguousarray(Y.transpose(1, 0, 2)).reshape(B, T * cells))
+    net.Backward_Pass(B)
+    taps = ["LSTM_DELTA_CELL_INPUT", "LSTM_DELTA_INPUT_GATE", "LSTM_DELTA_FORGET_GATE", "LSTM_DELTA_OUTPUT_GATE"]
+    dG = [net.download_tensor(1, mb.TENSOR[t], T * B * cells).reshape(T, B, cells)[1].astype(np.float64) for t in taps]
+    got = net.download_tensor(1, mb.TENSOR["ERRORS"]).reshape(T, B, cells)[0].astype(np.float64)
+    want = sum(d @ r.astype(np.float64) for d, r in zip(dG, recurrent))
+    magnitude = sum(np.abs(d) @ np.abs(r.astype(np.float64)) for d, r in zip(dG, recurrent))
+    assert np.abs(want).max() > 0
+    assert np.all(np.abs(got - want) <= 2.0 ** -23 * (cells / 8 + 20) * magnitude + 2.0 ** -149)
