@@ -739,6 +739,91 @@ int launch_short(hipStream_t stream, GemmDev d, bool a_kc, bool b_kc)
     return MYEA_OK;
 }
 
+// ---- a shallow product --------------------------------------------------------------------------------------------------
+// With few k's there is nothing to gain from the BF16 planes and something to lose: a single product or a pair of them is rounded once by
+// the FP32 instruction and a little more than once by the six (k = 1: 2.6e-8 against 2.5e-8), and a sum that one large product
+// dominates stays up to 1.7 times less exact until an instruction's 16 k's are full.  Such a product is bound by the latency of its
+// operands and the stores of C, so it can as well be exact: a wavefront owns 32 rows x 32 columns, takes its operands straight
+// from memory and multiplies with v_mfma_f64_16x16x4_f64 (as many cycles a k as the FP32 instruction's on 64-bit sums); what is
+// rounded is the result.  Infinities, NaN and subnormals need no care.
+//   operands: lane l takes k = l / 16 of every four and one row (A) or column (B) of each half of the tile
+//   result:   register i of lane l holds row 4 i + l / 16, column l % 16.  Which row of C that is is chosen by the rows that A's lanes
+//             take: with the rows below, lanes l and l ^ 16 hold each other's half of what the epilogue's layout gives them.
+constexpr int kShallow = 16;   // k's of one v_mfma_f32_32x32x16_bf16
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+
+template <bool A_KC, bool B_KC>
+__global__ __launch_bounds__(kThreads) void shallow_gemm_kernel(GemmDev p)
+{
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lane16 = lane & 15, quad = lane >> 4;
+    const int tile = (int)blockIdx.x * (kThreads / 64) + wave;   // columns first: a workgroup stores whole runs of C's rows
+    if (tile >= p.nbm * p.nbn) return;
+    const int m0 = tile / p.nbn * 32, n0 = tile % p.nbn * 32;
+    long a_row[2], b_col[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        const int i = lane16 >> 2, g = lane16 & 3;   // of the result's row 4 i + g
+        a_row[t] = min(m0 + ((g & 1) * 2 + t) * 8 + (g >> 1) * 4 + i, p.M - 1);
+        b_col[t] = min(n0 + t * 16 + lane16, p.N - 1);
+    }
+    f64x4 sum[2][2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) sum[t][u] = (f64x4){0., 0., 0., 0.};
+    float a[kShallow / 4][2], b[kShallow / 4][2];
+#pragma unroll
+    for (int e = 0; e < kShallow / 4; ++e) {
+        if (e * 4 >= p.K) break;
+        const long k = e * 4 + quad;
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            a[e][t] = b[e][t] = 0.f;
+            if (k < p.K) {
+                a[e][t] = p.A[A_KC ? a_row[t] * p.lda + k : k * p.lda + a_row[t]];
+                b[e][t] = p.B[B_KC ? b_col[t] * p.ldb + k : k * p.ldb + b_col[t]];
+            }
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < kShallow / 4; ++e) {
+        if (e * 4 >= p.K) break;
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int u = 0; u < 2; ++u) sum[t][u] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)a[e][t], (double)b[e][u], sum[t][u], 0, 0, 0);
+    }
+    f32x16 acc[1][1];
+    const bool odd = quad & 1;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float first = (float)sum[t][0][i], second = (float)sum[t][1][i];
+            const float kept = odd ? second : first, other = __shfl_xor(odd ? first : second, 16);
+            acc[0][0][t * 4 + i] = odd ? other : kept;
+            acc[0][0][8 + t * 4 + i] = odd ? kept : other;
+        }
+    const TilePlace at{m0, n0, 0, 0, lane & 31, lane >> 5, 0L};
+    if (p.M - m0 >= 32 && p.N - n0 >= 32) store_tile_kind<true, 1, 1>(p, acc, at);
+    else store_tile_kind<false, 1, 1>(p, acc, at);
+}
+
+int launch_shallow(hipStream_t stream, GemmDev d, bool a_kc, bool b_kc)
+{
+    d.nbm = (d.M + 31) / 32;
+    d.nbn = (d.N + 31) / 32;
+    const long tiles = (long)d.nbm * d.nbn;
+    if (tiles > 0x7fffffffL) { set_last_error("gemm: %ld tiles of 32 x 32 out of range", tiles); return MYEA_E_INVALID; }
+    const dim3 grid((unsigned)((tiles + kThreads / 64 - 1) / (kThreads / 64))), group(kThreads);
+    if (a_kc && b_kc) hipLaunchKernelGGL((shallow_gemm_kernel<true, true>), grid, group, 0, stream, d);
+    else if (a_kc) hipLaunchKernelGGL((shallow_gemm_kernel<true, false>), grid, group, 0, stream, d);
+    else if (b_kc) hipLaunchKernelGGL((shallow_gemm_kernel<false, true>), grid, group, 0, stream, d);
+    else hipLaunchKernelGGL((shallow_gemm_kernel<false, false>), grid, group, 0, stream, d);
+    MYEA_HIP_TRY(hipGetLastError());
+    return MYEA_OK;
+}
+
 // ---- a narrow product ---------------------------------------------------------------------------------------------------
 // C [M][N] = A B with N <= 32 and K <= 64 - a layer of an independently recurrent stack over T x batch rows, forward or backward.
 // The tiled kernel spends such a launch on its set-up and its stages: a few microseconds of instructions fetched to be run once.  Here a wavefront owns 32 rows of C: the
@@ -981,6 +1066,11 @@ int launch_gemm(hipStream_t stream, const GemmParams &p)
         MYEA_HIP_TRY(hipGetLastError());
         return MYEA_OK;
     }
+    // Fewer k's than one BF16 instruction takes: the sums in 64 bits.  Exactness decides the line, and the time is no worse than the FP32
+    // instruction's was (us, FP32 tiles / BF16 planes / this: 333 x 1201 x 10 5.2 / 8.4 / 5.3, 2049 x 2050 x 10 10.0 / 8.6 / 9.1, 4096 x
+    // 4096 x 3 20.7 / 15.1 / 15.3, 16384 x 512 x 10 13.4 / 9.7 / 12.3); at 16 k's and large outputs the planes win (16384 x 512: 9.9
+    // against 16).
+    if (p.K < kShallow && d.ksplit == 1) return launch_shallow(stream, d, a_kc, b_kc);
     // Tile choice: 128 x 128 from one workgroup per CU (256 CUs) on - its operand reuse is worth more than a second workgroup
     // (2048 x 2048 x 2048, 256 such tiles: 98 us, 512 tiles of 64 x 128: 110 us) - else 64-row tiles to keep the chip filled for
     // short-M / short-N problems.

@@ -354,8 +354,9 @@ bool aligned16(const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15u) ==
 // 5.9 + 5.3 us forward, 5.5 + 5.2 us backward as two launches), so the wavefronts of a workgroup share k in runs of 32, every
 // lane takes the operands it multiplies straight from memory (any alignment) and splits them for the BF16 matrix cores, the
 // partial tiles meet in LDS once, and 256 lanes finish a pair (example, cell) each, having asked for what the gate math reads
-// before the first run.  A pair whose sum is not finite computes it again in FP32.
-constexpr int kStepForwardWaves = 8, kStepBackwardWaves = 16;
+// before the first run.  A pair whose sum is not finite computes it again by itself, in 64 bits, and so does every pair where the sum has
+// fewer k's than a BF16 instruction (a handful of cells): the planes are no more exact than FP32 there (myea_gemm.hip, shallow products).
+constexpr int kStepForwardWaves = 8, kStepBackwardWaves = 16, kStepPlanes = 16;
 
 // Tile: 32 examples x 8 cells; column j of the tile is gate j / 8 of cell j % 8.
 __global__ __launch_bounds__(64 * kStepForwardWaves) void lstm_step_forward_kernel(LstmFusedForward p)
@@ -379,7 +380,7 @@ __global__ __launch_bounds__(64 * kStepForwardWaves) void lstm_step_forward_kern
     f32x16 acc, small;
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[r] = small[r] = 0.f;
-    for (int k0 = wave * 32; k0 < C; k0 += 32 * kStepForwardWaves) {
+    for (int k0 = wave * 32; k0 < C && C >= kStepPlanes; k0 += 32 * kStepForwardWaves) {
         float a[2][8], w[2][8];
 #pragma unroll
         for (int g = 0; g < 2; ++g) {
@@ -409,9 +410,10 @@ __global__ __launch_bounds__(64 * kStepForwardWaves) void lstm_step_forward_kern
 #pragma unroll
         for (int w = 0; w < kStepForwardWaves; ++w) s[gate] += parts[w][row >> 3][((row >> 2) & 1) * 32 + gate * 8 + cell][row & 3];
         s[gate] = unscaled(s[gate]);
-        if (!(fabsf(s[gate]) < INFINITY)) {
-            s[gate] = 0.f;
-            for (int k = 0; k < C; ++k) s[gate] = fmaf(p.h_prev[(size_t)b * C + k], p.Wrec[((size_t)gate * C + c) * C + k], s[gate]);
+        if (C < kStepPlanes || !(fabsf(s[gate]) < INFINITY)) {
+            double sum = 0.;
+            for (int k = 0; k < C; ++k) sum = fma((double)p.h_prev[(size_t)b * C + k], (double)p.Wrec[((size_t)gate * C + c) * C + k], sum);
+            s[gate] = (float)sum;
         }
         s[gate] += e_in[gate];
         s[gate] += p.bias[gate * C + c];
@@ -450,7 +452,7 @@ __global__ __launch_bounds__(64 * kStepBackwardWaves) void lstm_step_backward_ke
     const float *a_row = p.dG_next + (size_t)min(r0 + lane16, B - 1) * G;
     const float *b_col = p.Wrec + min(c0 + lane16, C - 1);
     f32x4 acc = {0.f, 0.f, 0.f, 0.f}, small = {0.f, 0.f, 0.f, 0.f};
-    for (int k0 = wave * 32; k0 < G; k0 += 32 * kStepBackwardWaves) {
+    for (int k0 = wave * 32; k0 < G && G >= kStepPlanes; k0 += 32 * kStepBackwardWaves) {
         const int k = k0 + quad * 8;
         float a[8], w[8];
         load_eight<true>(a, a_row + k, 0, k, G);
@@ -469,9 +471,10 @@ __global__ __launch_bounds__(64 * kStepBackwardWaves) void lstm_step_backward_ke
 #pragma unroll
     for (int w = 0; w < kStepBackwardWaves; ++w) s += parts[w][(row >> 2) * 16 + cell][row & 3];
     s = unscaled(s);
-    if (!(fabsf(s) < INFINITY)) {
-        s = 0.f;
-        for (int k = 0; k < G; ++k) s = fmaf(p.dG_next[(size_t)b * G + k], p.Wrec[(size_t)k * C + c], s);
+    if (G < kStepPlanes || !(fabsf(s) < INFINITY)) {
+        double sum = 0.;
+        for (int k = 0; k < G; ++k) sum = fma((double)p.dG_next[(size_t)b * G + k], (double)p.Wrec[(size_t)k * C + c], sum);
+        s = (float)sum;
     }
     const float v = dh + s, z = gate[0], gi = gate[1], gf = gate[2], go = gate[3];
     p.dh[at_c] = v;

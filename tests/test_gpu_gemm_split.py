@@ -49,6 +49,31 @@ def test_small_operands_keep_their_bits(a_kc, b_kc, M, N, K):
 
 
 @pytest.mark.parametrize("a_kc,b_kc", LAYOUTS)
+@pytest.mark.parametrize("K", [1, 2, 3, 4, 5, 11, 15])
+def test_shallow_products_are_rounded_once(a_kc, b_kc, K):
+    """Fewer k's than a BF16 instruction's 16: the sum is held in 64 bits, so a result is its FP32 neighbour (half an ulp, and 2^-50 of
+    the magnitudes for the 64-bit sums on both sides) - over heavy-tailed, subnormal, overflowing and infinite values, onto C as well."""
+    for M, N in ((1, 1), (31, 33), (32, 32), (65, 100), (300, 33), (100, 4097), (1025, 700)):
+        A, B, _, _ = _operands(a_kc, b_kc, M, N, K, M + N + K)
+        A, B = A * torch.exp(4 * A), B.clone()
+        A[0, 0], B[K - 1, N // 2] = 1e-42, -3e38
+        Ad, Bd = (A if a_kc else A.t()).contiguous(), (B.t() if b_kc else B).contiguous()
+        C = torch.full((M, N), float("nan"), device="cuda")
+        _gemm(mb.load_library(), a_kc, b_kc, 0, M, N, K, Ad, Bd, C)
+        want, magnitude = A.double() @ B.double(), A.double().abs() @ B.double().abs()
+        finite = want.abs() < 3.4e38
+        off = (C.double() - want).abs() > 2.0 ** -24 * want.abs() + 2.0 ** -50 * magnitude + 2.0 ** -150
+        assert not bool((off & finite).any()) and bool((C[want.abs() > 3.5e38].isinf()).all()), (M, N)
+        D = torch.ones((M, N), device="cuda")
+        _gemm(mb.load_library(), a_kc, b_kc, 1, M, N, K, Ad, Bd, D)
+        assert torch.equal(D, C + 1), (M, N)
+        A[M // 2, 0], B[0, 0] = float("inf"), float("nan")
+        _gemm(mb.load_library(), a_kc, b_kc, 0, M, N, K, (A if a_kc else A.t()).contiguous(), (B.t() if b_kc else B).contiguous(), C)
+        want = (A.double() @ B.double()).float()
+        assert torch.equal(C.isnan(), want.isnan()) and torch.equal(C.isinf() & (C > 0), want.isinf() & (want > 0)), (M, N)
+
+
+@pytest.mark.parametrize("a_kc,b_kc", LAYOUTS)
 @pytest.mark.parametrize("M,N", [(100, 90), (1500, 1501), (2049, 2050)])
 def test_values_the_split_cannot_carry(a_kc, b_kc, M, N):
     K = 40
