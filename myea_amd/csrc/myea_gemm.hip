@@ -1072,11 +1072,12 @@ int launch_gemm(hipStream_t stream, const GemmParams &p)
     // against 16).
     if (p.K < kShallow && d.ksplit == 1) return launch_shallow(stream, d, a_kc, b_kc);
     // Tile choice: 128 x 128 from one workgroup per CU (256 CUs) on - its operand reuse is worth more than a second workgroup
-    // (2048 x 2048 x 2048, 256 such tiles: 98 us, 512 tiles of 64 x 128: 110 us) - else 64-row tiles to keep the chip filled for
-    // short-M / short-N problems.
+    // (2048 x 2048 x 2048, 256 such tiles: 98 us, 512 tiles of 64 x 128: 110 us), unless half of it would lie outside the matrix
+    // (49152 rows, 40 columns, k = 64: 11.2 us, as 128 x 64 8.7) - else 64-row tiles to keep the chip filled for short-M / short-N
+    // problems.
     const long tiles_128 = (long)((p.M + 127) / 128) * ((p.N + 127) / 128);
     const bool pair_128 = p.pair_partials && p.pair_tickets && d.ksplit == 1 && gemm_pair_k_128(p.M, p.N, p.K);   // see below
-    if (tiles_128 * d.ksplit >= 256 && !pair_128) return launch_layout<128, 128>(stream, d, a_kc, b_kc);   // slabs of a split k count: they fill the chip like tiles do
+    if (tiles_128 * d.ksplit >= 256 && !pair_128 && p.M > 64 && p.N > 64) return launch_layout<128, 128>(stream, d, a_kc, b_kc);   // slabs of a split k count: they fill the chip like tiles do
     // At most one 64 x 64 tile per compute unit and a k worth splitting: two workgroups per tile, half of k each, combined in
     // the launch - a second wavefront per SIMD to fill the first one's waits, which such a launch otherwise lacks.
     // MYEA_GEMM_PAIR_K=0 keeps one workgroup per tile.

@@ -11,8 +11,9 @@ from tests.test_gpu_kernels import _gemm
 pytestmark = pytest.mark.gpu
 
 LAYOUTS = [(1, 1), (1, 0), (0, 0), (0, 1)]
-# tiles of 64 x 64, 64 x 128, 128 x 64 and 128 x 128; k's below, at and beyond a step of 16 or 32
-SHAPES = [(190, 1100, 1), (65, 1300, 15), (600, 640, 33), (1500, 1501, 16), (1409, 1500, 65), (3001, 700, 31), (2049, 2050, 17), (2180, 1921, 48)]
+# k's below, at and beyond a step of 16 or 32
+SHAPES = [(190, 1100, 1), (65, 1300, 15), (600, 640, 33), (1500, 1501, 16), (1409, 1500, 65), (3001, 700, 31), (2049, 2050, 17), (2180, 1921, 48),
+          (33100, 33, 65), (50, 33000, 33)]   # at least 256 tiles of 128 x 128, but half of each outside
 
 
 def _operands(a_kc, b_kc, M, N, K, seed):
