@@ -612,15 +612,16 @@ int launch_layout(hipStream_t stream, const GemmDev &d, bool a_kc, bool b_kc)
 // ---- a short product ----------------------------------------------------------------------------------------------------
 // A product with too few 64 x 64 tiles to occupy the chip - a batch of 128 in front of 256 units is 8 of them - spends the tiled
 // kernel's time in its K steps, one behind the other on a few compute units.  Here a workgroup owns 32 rows x 32 columns and its
-// kShortWaves wavefronts share k: each takes every kShortWaves-th run of 32 k's, asks for its operands straight from memory in
+// WAVES wavefronts share k: each takes every WAVES-th run of 32 k's, asks for its operands straight from memory in
 // the lanes that multiply them (A: lane l takes row l % 32, k's 8 (l / 32) .. + 7 of a group of 16; B alike), a run ahead of the
 // one it splits and multiplies; no LDS and no barrier until the wavefronts' accumulators are added, in wavefront order, by the
 // first, which runs the tiled kernel's epilogue.  What bounds it is the latency of the first operands and the splitting, which
 // every workgroup of a row or column of tiles repeats; a layer of 256 units over a batch of 128 (k = 784) went from 19 to 8 us.
-constexpr int kShortWaves = 8;
+// launch_gemm says up to where it pays.
+constexpr int kShortMost = 256;   // workgroups: one of eight wavefronts per compute unit
 constexpr int kShortRun = 32;   // k's: one 128-byte line of a k-contiguous row
 
-template <bool KC>
+template <bool KC, int WAVES>
 struct ShortOperand {
     float reg[2][2][8];   // [slot][group of 16 k's][k]
     const float *at;      // of the run that is loaded next
@@ -632,7 +633,7 @@ struct ShortOperand {
         const long r = min(row, extent - 1);
         ld = ld_; k = k0; K = K_;
         at = base + (KC ? r * ld + k : k * ld + r);
-        step = KC ? (long)kShortRun * kShortWaves : (long)kShortRun * kShortWaves * ld;
+        step = KC ? (long)kShortRun * WAVES : (long)kShortRun * WAVES * ld;
     }
     __device__ __forceinline__ void load(int slot)
     {
@@ -656,14 +657,14 @@ struct ShortOperand {
                     if (k + g * 16 + e < K) reg[slot][g][e] = at[KC ? (long)(g * 16 + e) : (g * 16 + e) * ld];
                 }
         }
-        at += step; k += kShortRun * kShortWaves;
+        at += step; k += kShortRun * WAVES;
     }
 };
 
-template <bool A_KC, bool B_KC>
-__global__ __launch_bounds__(64 * kShortWaves) void short_gemm_kernel(GemmDev p)
+template <bool A_KC, bool B_KC, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void short_gemm_kernel(GemmDev p)
 {
-    __shared__ f32x4 handed[kShortWaves - 1][4][64];   // the accumulators of the wavefronts behind the first
+    __shared__ f32x4 handed[WAVES - 1][4][64];   // the accumulators of the wavefronts behind the first
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lane32 = lane & 31, half = lane >> 5;
     const int nblocks = p.nbm * p.nbn, split = (int)blockIdx.x / nblocks, pid = (int)blockIdx.x - split * nblocks;
     const int m0 = pid % p.nbm * 32, n0 = pid / p.nbm * 32;
@@ -671,12 +672,12 @@ __global__ __launch_bounds__(64 * kShortWaves) void short_gemm_kernel(GemmDev p)
     f32x16 acc[1][1], small;   // the hi hi products; the others
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[0][0][r] = small[r] = 0.f;
-    ShortOperand<A_KC> a;
-    ShortOperand<B_KC> b;
+    ShortOperand<A_KC, WAVES> a;
+    ShortOperand<B_KC, WAVES> b;
     const int first = k_begin + wave * kShortRun;
     a.init(p.A, p.lda, m0 + lane32, p.M, first + half * 8, k_end);
     b.init(p.B, p.ldb, n0 + lane32, p.N, first + half * 8, k_end);
-    const int runs = first < k_end ? (k_end - first + kShortRun * kShortWaves - 1) / (kShortRun * kShortWaves) : 0;
+    const int runs = first < k_end ? (k_end - first + kShortRun * WAVES - 1) / (kShortRun * WAVES) : 0;
     auto multiply = [&](int slot) {
 #pragma unroll
         for (int g = 0; g < 2; ++g) {
@@ -706,7 +707,7 @@ __global__ __launch_bounds__(64 * kShortWaves) void short_gemm_kernel(GemmDev p)
     if (wave) return;
     float finite = 0.f;
 #pragma unroll
-    for (int w = 0; w < kShortWaves - 1; ++w)
+    for (int w = 0; w < WAVES - 1; ++w)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const f32x4 v = handed[w][r][lane];
@@ -724,17 +725,29 @@ __global__ __launch_bounds__(64 * kShortWaves) void short_gemm_kernel(GemmDev p)
     else store_tile_kind<false, 1, 1>(p, acc, at);
 }
 
+template <int WAVES>
+void launch_short_waves(hipStream_t stream, const GemmDev &d, bool a_kc, bool b_kc, long nblocks)
+{
+    const dim3 grid((unsigned)nblocks), group(64 * WAVES);
+    if (a_kc && b_kc) hipLaunchKernelGGL((short_gemm_kernel<true, true, WAVES>), grid, group, 0, stream, d);
+    else if (a_kc) hipLaunchKernelGGL((short_gemm_kernel<true, false, WAVES>), grid, group, 0, stream, d);
+    else if (b_kc) hipLaunchKernelGGL((short_gemm_kernel<false, true, WAVES>), grid, group, 0, stream, d);
+    else hipLaunchKernelGGL((short_gemm_kernel<false, false, WAVES>), grid, group, 0, stream, d);
+}
+
+long short_blocks(int M, int N) { return (long)((M + 31) / 32) * ((N + 31) / 32); }
+
 int launch_short(hipStream_t stream, GemmDev d, bool a_kc, bool b_kc)
 {
     d.nbm = (d.M + 31) / 32;
     d.nbn = (d.N + 31) / 32;
     const long nblocks = (long)d.nbm * d.nbn * d.ksplit;
     if (nblocks <= 0 || nblocks > 0x7fffffffL) { set_last_error("gemm: grid of %ld workgroups out of range", nblocks); return MYEA_E_INVALID; }
-    const dim3 grid((unsigned)nblocks), group(64 * kShortWaves);
-    if (a_kc && b_kc) hipLaunchKernelGGL((short_gemm_kernel<true, true>), grid, group, 0, stream, d);
-    else if (a_kc) hipLaunchKernelGGL((short_gemm_kernel<true, false>), grid, group, 0, stream, d);
-    else if (b_kc) hipLaunchKernelGGL((short_gemm_kernel<false, true>), grid, group, 0, stream, d);
-    else hipLaunchKernelGGL((short_gemm_kernel<false, false>), grid, group, 0, stream, d);
+    // The registers admit eight wavefronts a compute unit.  More workgroups than compute units: of four wavefronts each, so that two
+    // share one instead of the second waiting for the first.  us, eight -> four, 333 x 1201 (418 workgroups): k = 64 7.5 -> 5.7, 256
+    // 9.5 -> 7.8, 1000 20.9 -> 18.2; up to one per compute unit: 10 x 1000, k = 1000 9.4 against 10.8.
+    if (nblocks > kShortMost) launch_short_waves<4>(stream, d, a_kc, b_kc, nblocks);
+    else launch_short_waves<8>(stream, d, a_kc, b_kc, nblocks);
     MYEA_HIP_TRY(hipGetLastError());
     return MYEA_OK;
 }
@@ -1078,7 +1091,7 @@ int launch_gemm(hipStream_t stream, const GemmParams &p)
     const long tiles_128 = (long)((p.M + 127) / 128) * ((p.N + 127) / 128);
     const bool pair_128 = p.pair_partials && p.pair_tickets && d.ksplit == 1 && gemm_pair_k_128(p.M, p.N, p.K);   // see below
     if (tiles_128 * d.ksplit >= 256 && !pair_128 && p.M > 64 && p.N > 64) return launch_layout<128, 128>(stream, d, a_kc, b_kc);   // slabs of a split k count: they fill the chip like tiles do
-    // At most one 64 x 64 tile per compute unit and a k worth splitting: two workgroups per tile, half of k each, combined in
+    // At most one 64 x 64 tile per compute unit but enough of them, and a k worth splitting: two workgroups per tile, half of k each, combined in
     // the launch - a second wavefront per SIMD to fill the first one's waits, which such a launch otherwise lacks.
     // MYEA_GEMM_PAIR_K=0 keeps one workgroup per tile.
     static const int pair_k = [] { const char *e = std::getenv("MYEA_GEMM_PAIR_K"); return e ? std::atoi(e) : 3; }();   // bit 0: 64 x 64 tiles, bit 1: 128 x 128
@@ -1092,17 +1105,18 @@ int launch_gemm(hipStream_t stream, const GemmParams &p)
         d.pair_partials = p.pair_partials; d.pair_tickets = p.pair_tickets;
         return launch_layout<128, 128>(stream, d, a_kc, b_kc);
     }
-    // Fewer than 128 tiles of 64 x 64, slabs counted (half the compute units): the short product, whose workgroups are four times as
-    // many and keep eight wavefronts busy each.  us, tiled -> short: 128 x 256 x 784 16.0 -> 8.0, 512 x 100 x 2048 34 -> 18, 256 x
-    // 1024 x 1024 19.0 -> 12.0, 333 x 1201 x 1201 (114 tiles) 25.3 -> 22.8; at 128 tiles (512 x 1024 x 1024) 19.1 -> 21.4.
     const long tiles_64 = (long)((p.M + 63) / 64) * ((p.N + 63) / 64);
-    if (tiles_64 * d.ksplit < 128) return launch_short(stream, d, a_kc, b_kc);
     if (p.pair_partials && p.pair_tickets && !pair_k_off && d.ksplit == 1 && tiles_64 <= kGemmPairTiles && tiles_64 % 8 == 0 && tiles_64 >= 128 && p.K >= 512) {
         d.ksplit = 2;
         d.kchunk = ((p.K + 1) / 2 + kBK - 1) / kBK * kBK;
         d.pair_partials = p.pair_partials; d.pair_tickets = p.pair_tickets;
         return launch_layout<64, 64>(stream, d, a_kc, b_kc);
     }
+    // The short product while two of its workgroups a compute unit are enough, slabs counted, at any k.  us, 64 x 64 tiles -> short, k
+    // = 64, 256, 1024, 4096 (the layouts' mean): 512 x 512 (256 workgroups) 4.7 -> 4.5, 7.9 -> 5.4, 21.1 -> 10.5, 75 -> 32; 640 x 768
+    // (480) 5.6 -> 5.8, 8.3 -> 7.6, 21.6 -> 17.3, 75 -> 57; 512 x 1024 (512) 5.2 -> 5.4, 8.2 -> 7.7, 21.5 -> 17.7, 75 -> 58; with a third
+    // workgroup a unit, 700 x 900 (638), 5.6 -> 7.5, 8.6 -> 10.6, 22.4 -> 25.9, 76 -> 85.
+    if (short_blocks(p.M, p.N) * d.ksplit <= 512) return launch_short(stream, d, a_kc, b_kc);
     if (tiles_128 * 2 * d.ksplit < 256) return launch_layout<64, 64>(stream, d, a_kc, b_kc);
     if (p.M <= p.N) return launch_layout<64, 128>(stream, d, a_kc, b_kc);
     return launch_layout<128, 64>(stream, d, a_kc, b_kc);

@@ -94,9 +94,11 @@ def test_values_the_split_cannot_carry(a_kc, b_kc, M, N):
 
 
 @pytest.mark.parametrize("a_kc,b_kc", LAYOUTS)
-@pytest.mark.parametrize("M,N,K", [(1, 33, 1), (31, 1, 23), (33, 32, 24), (32, 65, 31), (64, 64, 33), (95, 100, 255), (100, 31, 257), (700, 600, 545)])
+@pytest.mark.parametrize("M,N,K", [(1, 33, 1), (31, 1, 23), (33, 32, 24), (32, 65, 31), (64, 64, 33), (95, 100, 255), (100, 31, 257), (500, 490, 545),
+                                   (257, 1000, 17), (700, 600, 33), (700, 600, 545), (512, 1024, 129), (30, 16300, 300), (520, 1000, 300)])
 def test_short_products_against_float64(a_kc, b_kc, M, N, K):
-    """Fewer than 128 tiles of 64 x 64: eight wavefronts share k in runs of 32, of which the last ones may have none or a part."""
+    """Up to 512 workgroups of 32 x 32, of eight wavefronts up to 256 and of four beyond, that share k in runs of 32, of which the last ones
+    may have none or a part; the last shape has one workgroup too many."""
     A, B, Ad, Bd = _operands(a_kc, b_kc, M, N, K, M + N + K)
     C = torch.full((M, N), float("nan"), device="cuda")
     _gemm(mb.load_library(), a_kc, b_kc, 0, M, N, K, Ad, Bd, C)
