@@ -1437,8 +1437,10 @@ static int fc_dw_slabs(size_t H, size_t In, size_t rows)
     if (rows > 0x7fffffffu) return 1;
     const int narrow = narrow_dw_slabs(H, In, rows);   // a narrow layer's kernel of its own: always through slabs
     if (narrow > 0) return narrow > 1 ? narrow : 2;    // (room for two, so that "more than one slab" still says "through slabs")
-    // Short of 1024 rows one launch is as good as slabs without the pass that adds them: each of the short product's eight wavefronts
-    // has four runs of 32 rows at most (37 x 1201 over 333 rows: 11 + 4 us through two slabs, 7 us so).
+    // Short of 1024 rows one launch is as good as slabs without the pass that adds them: a wavefront of the short product has a few runs
+    // of 32 rows (37 x 1201 over 333 rows: 11 + 4 us through two slabs, 7 us so), and 64 x 64 tiles, half as many workgroups in one
+    // launch as in two slabs, still win by what the pass costs (700 x 900 over 300, 512 and 1000 rows: 13.3 + 4.3, 15.2 + 4.4 and 24.8 +
+    // 4.3 us through two slabs, 11.7, 15.4 and 26.4 so; 1400 x 600 over 1000: 25.7 + 4.4 against 27.7).
     if (rows < 1024) return 1;
     return gemm_split_k((int)H, (int)In, (int)rows);
 }
