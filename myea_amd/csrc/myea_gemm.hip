@@ -312,8 +312,8 @@ __device__ __forceinline__ void redo_in_f32(const GemmDev &p, f32x16 (&acc)[TM][
         for (int j = 0; j < TN; ++j)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-    for (int k0 = k_begin; k0 < k_end; k0 += 2) {
-        const int k = k0 + half;
+    for (long k0 = k_begin; k0 < k_end; k0 += 2) {
+        const long k = k0 + half;
         float a[TM], b[TN];
 #pragma unroll
         for (int i = 0; i < TM; ++i) {
@@ -355,7 +355,7 @@ __device__ __forceinline__ void gemm_tile(const GemmDev &p, const int block, cha
     const int split = block / nblocks;   // split-K slab of this workgroup
     int pid = block - split * nblocks;
     if ((nblocks & 7) == 0) pid = (pid & 7) * (nblocks >> 3) + (pid >> 3);
-    const int k_begin = split * p.kchunk, k_end = min(p.K, k_begin + p.kchunk);
+    const int k_begin = split * p.kchunk, k_end = (int)min((long)p.K, (long)k_begin + p.kchunk);
     constexpr int kBand = 8;
     const int band = pid / (kBand * p.nbn);
     const int band_first = band * kBand;
@@ -626,18 +626,18 @@ struct ShortOperand {
     float reg[2][2][8];   // [slot][group of 16 k's][k]
     const float *at;      // of the run that is loaded next
     long ld, step;
-    int k, K;             // first k of this lane in that run
+    int left;             // k's from this lane's first one in that run on
 
-    __device__ __forceinline__ void init(const float *base, long ld_, int row, int extent, int k0, int K_)
+    __device__ __forceinline__ void init(const float *base, long ld_, int row, int extent, long k0, int K)
     {
         const long r = min(row, extent - 1);
-        ld = ld_; k = k0; K = K_;
-        at = base + (KC ? r * ld + k : k * ld + r);
+        ld = ld_; left = K - k0;
+        at = base + (KC ? r * ld + k0 : k0 * ld + r);
         step = KC ? (long)kShortRun * WAVES : (long)kShortRun * WAVES * ld;
     }
     __device__ __forceinline__ void load(int slot)
     {
-        if (k + 24 <= K) {   // this lane's last k of the run is k + 23
+        if (left >= 24) {   // this lane's last k of the run is the 24th
 #pragma unroll
             for (int g = 0; g < 2; ++g) {
                 if (KC) {
@@ -654,10 +654,10 @@ struct ShortOperand {
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
                     reg[slot][g][e] = 0.f;
-                    if (k + g * 16 + e < K) reg[slot][g][e] = at[KC ? (long)(g * 16 + e) : (g * 16 + e) * ld];
+                    if (g * 16 + e < left) reg[slot][g][e] = at[KC ? (long)(g * 16 + e) : (g * 16 + e) * ld];
                 }
         }
-        at += step; k += kShortRun * WAVES;
+        at += step; left -= kShortRun * WAVES;
     }
 };
 
@@ -668,7 +668,7 @@ __global__ __launch_bounds__(64 * WAVES) void short_gemm_kernel(GemmDev p)
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lane32 = lane & 31, half = lane >> 5;
     const int nblocks = p.nbm * p.nbn, split = (int)blockIdx.x / nblocks, pid = (int)blockIdx.x - split * nblocks;
     const int m0 = pid % p.nbm * 32, n0 = pid / p.nbm * 32;
-    const int k_begin = split * p.kchunk, k_end = min(p.K, k_begin + p.kchunk);
+    const int k_begin = split * p.kchunk, k_end = (int)min((long)p.K, (long)k_begin + p.kchunk);
     f32x16 acc[1][1], small;   // the hi hi products; the others
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[0][0][r] = small[r] = 0.f;
@@ -677,7 +677,7 @@ __global__ __launch_bounds__(64 * WAVES) void short_gemm_kernel(GemmDev p)
     const int first = k_begin + wave * kShortRun;
     a.init(p.A, p.lda, m0 + lane32, p.M, first + half * 8, k_end);
     b.init(p.B, p.ldb, n0 + lane32, p.N, first + half * 8, k_end);
-    const int runs = first < k_end ? (k_end - first + kShortRun * WAVES - 1) / (kShortRun * WAVES) : 0;
+    const int runs = first < k_end ? (k_end - first - 1) / (kShortRun * WAVES) + 1 : 0;
     auto multiply = [&](int slot) {
 #pragma unroll
         for (int g = 0; g < 2; ++g) {
@@ -956,7 +956,7 @@ int gemm_split_k(int M, int N, int K)
     if (want == 1) return 1;
     // the launcher rounds the chunk up to a multiple of 32: return the slab count that rounding produces
     const int chunk = (int)(((K + want - 1) / want + kBK - 1) / kBK * kBK);
-    return (K + chunk - 1) / chunk;
+    return (int)(((long)K + chunk - 1) / chunk);
 }
 
 // No k up to K takes more slabs than this: what a workspace for them is sized by.  (Fewer k's may take more of them: 16 at 4095,
@@ -1019,9 +1019,9 @@ static int prepare_gemm(const GemmParams &p, GemmDev &d)
     }
     if (p.split_k > 1) {
         if (p.epilogue != EPI_NONE || p.accumulate || p.addend) { set_last_error("gemm: split-K writes plain partial slabs"); return MYEA_E_INVALID; }
-        const int chunk = ((p.K + p.split_k - 1) / p.split_k + kBK - 1) / kBK * kBK;
+        const int chunk = (int)(((long)p.K + p.split_k - 1) / p.split_k + kBK - 1) / kBK * kBK;
         d.kchunk = chunk;
-        d.ksplit = (p.K + chunk - 1) / chunk;
+        d.ksplit = (int)(((long)p.K + chunk - 1) / chunk);
         d.slab = p.split_k_slab;
         if (d.ksplit != p.split_k) { set_last_error("gemm: split-K count %d does not divide K=%d into %d-wide chunks; use gemm_split_k()", p.split_k, p.K, chunk); return MYEA_E_INVALID; }
     }
@@ -1101,14 +1101,14 @@ int launch_gemm(hipStream_t stream, const GemmParams &p)
     // tile's operand reuse.
     if ((pair_k & 2) && pair_128) {
         d.ksplit = 2;
-        d.kchunk = ((p.K + 1) / 2 + kBK - 1) / kBK * kBK;
+        d.kchunk = (int)(((long)p.K + 1) / 2 + kBK - 1) / kBK * kBK;
         d.pair_partials = p.pair_partials; d.pair_tickets = p.pair_tickets;
         return launch_layout<128, 128>(stream, d, a_kc, b_kc);
     }
     const long tiles_64 = (long)((p.M + 63) / 64) * ((p.N + 63) / 64);
     if (p.pair_partials && p.pair_tickets && !pair_k_off && d.ksplit == 1 && tiles_64 <= kGemmPairTiles && tiles_64 % 8 == 0 && tiles_64 >= 128 && p.K >= 512) {
         d.ksplit = 2;
-        d.kchunk = ((p.K + 1) / 2 + kBK - 1) / kBK * kBK;
+        d.kchunk = (int)(((long)p.K + 1) / 2 + kBK - 1) / kBK * kBK;
         d.pair_partials = p.pair_partials; d.pair_tickets = p.pair_tickets;
         return launch_layout<64, 64>(stream, d, a_kc, b_kc);
     }

@@ -22,6 +22,7 @@ def test_split_k_never_exceeds_its_bound(M, N):
     count, most = (_function("_ZN4myea%sEiii" % n, C.c_int, C.c_int, C.c_int) for n in ("12gemm_split_k", "17gemm_split_k_most"))
     reached, ks = 0, list(range(1, 700)) + list(range(700, 20000, 53)) + [4063, 4064, 4065, 4095, 4096, 4097, 16383, 16384, 100000, 10 ** 7, 2 ** 31 - 1]
     for k in sorted(ks):
+        assert count(M, N, k) >= 1, k
         reached = max(reached, count(M, N, k))
         assert reached <= most(M, N, k), k
     assert most(M, N, 2 ** 31 - 1) <= 32
