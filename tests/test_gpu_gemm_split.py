@@ -11,9 +11,14 @@ from tests.test_gpu_kernels import _gemm
 pytestmark = pytest.mark.gpu
 
 LAYOUTS = [(1, 1), (1, 0), (0, 0), (0, 1)]
-# k's below, at and beyond a step of 16 or 32
-SHAPES = [(190, 1100, 1), (65, 1300, 15), (600, 640, 33), (1500, 1501, 16), (1409, 1500, 65), (3001, 700, 31), (2049, 2050, 17), (2180, 1921, 48),
-          (33100, 33, 65), (50, 33000, 33)]   # at least 256 tiles of 128 x 128, but half of each outside
+# the tiled kernel, a shape per tile: more than 512 tiles of 32 x 32 (below it is the short product's) and
+TILE_64 = [(700, 1000), (1001, 777), (1025, 1030)]   # fewer than 128 of 128 x 128
+TILE_64_128, TILE_128_64 = [(1500, 1501), (1409, 1500)], [(3001, 700), (1600, 1500)]   # up to 255 of them
+TILE_128 = [(2049, 2050), (2180, 1921)]
+# k's at, around and beyond a step of 16 or 32, and for the 64 x 64 tile around the four steps that it keeps in registers
+SHAPES = ([t + (k,) for t in TILE_64 for k in (16, 31, 33, 65, 127, 161, 257, 545)] + [t + (k,) for t in TILE_64_128 + TILE_128_64 for k in (16, 31, 65, 97)] +
+          [t + (k,) for t in TILE_128 for k in (17, 48, 95)] + [(33100, 33, 65), (50, 33000, 33)] +   # thin: 128 x 64 and 64 x 128
+          [(190, 1100, 1), (65, 1300, 15), (600, 640, 33)])   # shallow, shallow, short
 
 
 def _operands(a_kc, b_kc, M, N, K, seed):
@@ -32,6 +37,21 @@ def test_tiles_and_remainders_against_float64(a_kc, b_kc, M, N, K):
     _gemm(mb.load_library(), a_kc, b_kc, 0, M, N, K, Ad, Bd, C)
     bound = 2.0 ** -23 * (-(-K // 16) + 8) * (A.double().abs() @ B.double().abs())
     assert bool(((C.double() - A.double() @ B.double()).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("M,N", [(96, 100), (640, 768), (1030, 1000), (2049, 2050)])   # short (eight and four wavefronts), 64 x 64, 128 x 128
+def test_error_over_many_products(M, N):
+    """2-norm of the error over that of the result at k = 4096: what myea_gemm.hip states for the tiled kernel is 4.0e-7 for normal operands
+    (two planes of BF16 would leave 3.5e-6, emulated) and 3.1e-7 for positive ones (a unit that cut its sums off where this one rounds them
+    would leave 5.7e-6, emulated); the FP32 instruction has 1.15e-6 and 8.4e-7.  The short product adds
+    four or eight shorter sums and is below both."""
+    K = 4096
+    A, B, _, _ = _operands(1, 1, M, N, K, M)
+    for a, b, most in ((A, B, 5e-7), (A.abs(), B.abs(), 4e-7)):
+        C = torch.empty((M, N), device="cuda")
+        _gemm(mb.load_library(), 1, 1, 0, M, N, K, a, b.t().contiguous(), C)
+        want = a.double() @ b.double()
+        assert ((C.double() - want).norm() / want.norm()).item() <= most
 
 
 @pytest.mark.parametrize("a_kc,b_kc", LAYOUTS)
@@ -75,7 +95,7 @@ def test_shallow_products_are_rounded_once(a_kc, b_kc, K):
 
 
 @pytest.mark.parametrize("a_kc,b_kc", LAYOUTS)
-@pytest.mark.parametrize("M,N", [(100, 90), (1500, 1501), (2049, 2050)])
+@pytest.mark.parametrize("M,N", [(100, 90), (700, 1000), (1500, 1501), (1600, 1500), (2049, 2050)])
 def test_values_the_split_cannot_carry(a_kc, b_kc, M, N):
     K = 40
     A, B, _, _ = _operands(a_kc, b_kc, M, N, K, 3)

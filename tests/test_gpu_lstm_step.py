@@ -30,9 +30,9 @@ def test_step_of_any_width(cells, B, Bmax, monkeypatch):
     assert_close(g, two.download_gradient(), REL, ABS * max(1.0, float(np.abs(want).max())), what="gradient, one launch against two")
 
 
-def test_infinite_weight_saturates_a_gate_as_in_fp32():
+def test_infinite_weight_saturates_a_gate_as_in_fp32(monkeypatch):
     """One weight of infinity at a time, recurrent ones and peepholes among them: a gate's sum is an infinity (not NaN) wherever
-    what the weight meets is not zero, and the activations of an infinity are finite."""
+    what the weight meets is not zero, and the activations of an infinity are finite - the same as through the two launches."""
     T, B, cells = 2, 5, 9
     desc, gpu, _ = _pair([dict(units=4), dict(type="lstm", units=cells), dict(units=cells, activation="LINEAR")], B, T, {}, seed=3)
     w = gpu.download_parameters()
@@ -43,8 +43,13 @@ def test_infinite_weight_saturates_a_gate_as_in_fp32():
         v = w.copy()
         v[i] = np.inf
         gpu.upload_parameters(v)
-        gpu.Forward_Pass(B, X)
-        assert np.isfinite(gpu.download_tensor(1, mb.TENSOR["OUTPUTS"], T * B * cells)).all(), i
+        out = []
+        for fused in ("1", "0"):
+            monkeypatch.setenv("MYEA_LSTM_FUSED", fused)
+            gpu.Forward_Pass(B, X)
+            out.append(gpu.download_tensor(1, mb.TENSOR["OUTPUTS"], T * B * cells))
+        assert np.isfinite(out[0]).all(), i
+        assert_close(out[0], out[1], REL, ABS, what="weight %d" % i)
 
 
 @pytest.mark.parametrize("cells,B", [(9, 5), (130, 40)])
