@@ -31,6 +31,9 @@
 // compiler's order, 98 us so).  An operand's place in LDS
 // does not depend on its orientation in memory:
 //   [plane][k / 8][row][8 k's]     a fragment (row l % 32, k's 8 (l / 32) .. + 7 of lane l) is one conflict-free ds_read_b128
+// Counted (1024 x 4096 x 4096, two workgroups a tile): the matrix unit is busy 56 % of the clocks, 5 vector instructions a matrix
+// instruction, no bank conflicts; 64 x 64 tiles (1024 x 1000 x 4096) 37 %, and a k-contiguous operand's stores, four chunks of a row at a
+// time, lose a sixth of the clocks to conflicts there.
 // A k-contiguous operand is read as two 16-byte loads per lane, the other kind as eight 4-byte loads that are coalesced over
 // the rows; neither needs more than 4-byte alignment, so odd widths and leading dimensions take the same path.
 //
@@ -1143,10 +1146,6 @@ int launch_gemm_pair(hipStream_t stream, const GemmParams &a, const GemmParams &
     };
     constexpr size_t lds_b = 2 * stage_bytes<128, 128>();
     if (fits(128)) {
-        // beside a long dX of 128 x 128 tiles adds at the L2 and stores take the same time (4096-wide layers at a batch of 1024:
-        // 27.45 and 27.35 ms for eight steps); everywhere else a store onto known zeros wins
-        static const int store128 = [] { const char *e = std::getenv("MYEA_DW_STORE_PAIR128"); return e ? std::atoi(e) : 0; }();
-        if (b.accumulate && !store128) db.accumulate = 1;
         da.nbm = (a.M + 127) / 128; da.nbn = (a.N + 127) / 128;
         const long na = (long)da.nbm * da.nbn;
         constexpr size_t lds_bytes = lds_b;
