@@ -7,7 +7,8 @@ stack 4096-4096-4096-4096-4096-1000 (ReLU, softmax + cross-entropy, Adam) at bat
 
 Prints ONE JSON line.  The timed block of exactly `steps` steps is run `--repeats` times; `value` and `ms_per_step` are the
 median block's, every block's figure is listed (`ms_per_step_blocks`).  `roofline` covers the dominant kernel family — the
-FP32 MFMA contractions (forward X W^T, dX = delta W, dW += delta^T X): algorithmic FLOPs of all their launches over their
+FP32 contractions (forward X W^T, dX = delta W, dW += delta^T X), which run as six BF16 products each on the matrix cores, so that
+their peak is a sixth of the BF16 one (`of_fp32_peak` divides by the FP32 matrix peak instead): algorithmic FLOPs of all their launches over their
 summed HIP-event durations on the stream they run on, taken in a second pass of `steps` steps (`events_pass`), because a
 pair of timing events around every launch slows the step it measures.  `cpu_baseline` times the CPU restatement of the
 reference (oracle/, OpenMP) on this host on a bounded sample of the same workload.
@@ -25,14 +26,16 @@ if ROOT not in sys.path:
 # HBM bytes per contraction launch (mean over the launches of one step): NOT measured by this script's run.  Recorded
 # from rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE runs of this script, scaled by what the same counters read for copies of
 # known size (FETCH_SIZE x2, WRITE_SIZE x1); the line names the file the figure comes from.
-RECORDED_TRAFFIC = {"fc4096x4_b1024_adam": dict(bytes_per_launch=2951372 * 1024 / 10,
+RECORDED_TRAFFIC = {"fc4096x4_b1024_adam": dict(bytes_per_launch=2934498 * 1024 / 10,
                                                 source="recorded constant, not measured in this run: profiles/hbm_traffic__fc4096x4_b1024_adam__pmc.txt"),
                     # the two resident time loops of one layer (forward + backward launch), mean per launch
                     "lstm512x2_t64_b256_amsgrad": dict(bytes_per_launch=(2 * 98055.1 + 230411.5 + 2 * 203936.9 + 197795.6) * 1024 / 2,
                                                        source="recorded constant, not measured in this run: profiles/lstm_resident__lstm512x2_t64_b256_amsgrad__pmc.txt")}
 from myea_amd.synthetic import simple_debug_layers  # noqa: E402  (no device is touched by the import)
 
-PEAK_FP32_MFMA_TFLOPS = 157.3   # MI355X dense FP32 matrix
+PEAK_FP32_MFMA_TFLOPS = 157.3   # MI355X dense FP32 matrix: the resident LSTM time loops
+PEAK_CONTRACTION_TFLOPS = 2516.6 / 6   # MI355X dense BF16 matrix, six products a multiplication: the contractions
+SUSTAINED_CONTRACTION_TFLOPS = 1143.0 / 6   # the rate a large BF16 product of the vendor's library was measured to sustain, over six
 PEAK_HBM_GBS = 8000.0           # MI355X HBM3E
 
 WORKLOADS = {
@@ -172,6 +175,7 @@ def cpu_baseline(wl, sample_rows, threads):
 FAMILIES = (("forward", "flop"), ("dx", "flop"), ("dw", "flop"), ("update", "byte"), ("dx_dw_pair", "flop"),
             ("lstm_forward_loop", "flop"), ("lstm_backward_loop", "flop"),
             ("normalization", "byte"), ("bias_gradient", "byte"), ("output_error", "byte"), ("softmax", "byte"))
+TIME_LOOPS = ("lstm_forward_loop", "lstm_backward_loop")
 KERNEL_NAMES = {"forward": "gemm_forward", "dx": "gemm_dx", "dw": "gemm_dw", "dx_dw_pair": "gemm_dx_dw_pair", "update": "optimizer_update"}
 
 
@@ -253,17 +257,18 @@ def run_workload(name, steps, warmup, separate_update=False, repeats=1):
         rate = work / max(ms * 1e-3, 1e-12)
         entry = dict(launches=n, avg_ms=ms / n, ms_per_step=ms / steps)
         if unit == "flop":
-            entry.update(tflops=rate / 1e12, frac_mfma_peak=rate / 1e12 / PEAK_FP32_MFMA_TFLOPS)
+            peak = PEAK_FP32_MFMA_TFLOPS if fname in TIME_LOOPS else PEAK_CONTRACTION_TFLOPS
+            entry.update(tflops=rate / 1e12, frac_mfma_peak=rate / 1e12 / peak)
         else:
             entry.update(gbs=rate / 1e9, frac_hbm_peak=rate / 1e9 / PEAK_HBM_GBS)
         kernels[KERNEL_NAMES.get(fname, fname)] = entry
 
-    def mfma_aggregate(names, fam=fam):
+    def mfma_aggregate(names, fam=fam, peak=PEAK_CONTRACTION_TFLOPS):
         n = sum(fam[k][0] for k in names)
         ms = sum(fam[k][1] for k in names)
         flop = sum(fam[k][2] for k in names)
         achieved = flop / (ms * 1e-3) / 1e12 if ms > 0 else 0.0
-        return dict(bound="mfma", achieved=achieved, peak=PEAK_FP32_MFMA_TFLOPS, unit="TFLOP/s", frac=achieved / PEAK_FP32_MFMA_TFLOPS,
+        return dict(bound="mfma", achieved=achieved, peak=peak, unit="TFLOP/s", frac=achieved / peak, of_fp32_peak=achieved / PEAK_FP32_MFMA_TFLOPS,
                     launches=n, avg_launch_ms=ms / max(n, 1), flops_per_launch=flop / max(n, 1), ms_per_step=ms / steps)
 
     return dict(workload=name, wl=wl, desc_parameters=int(desc.total_parameters), batch=B, ms_per_step=ms_per_step, value=B / (ms_per_step * 1e-3),
@@ -273,7 +278,7 @@ def run_workload(name, steps, warmup, separate_update=False, repeats=1):
                 contractions=mfma_aggregate(("forward", "dx", "dw", "dx_dw_pair")),
                 contractions_alone=mfma_aggregate(("forward", "dx", "dw", "dx_dw_pair"), fam_alone) if fam_alone else None,
                 ms_per_step_events_alone=ms_per_step_alone,
-                time_loops=mfma_aggregate(("lstm_forward_loop", "lstm_backward_loop")))
+                time_loops=mfma_aggregate(TIME_LOOPS, peak=PEAK_FP32_MFMA_TFLOPS))
 
 
 def config_of(r):
@@ -375,7 +380,8 @@ def main():
     has_loops = r["time_loops"]["launches"] > 0
     alone = r["contractions_alone"]
     roofline = dict(alone or r["contractions"])
-    roofline["kernel"] = "gemm_f32_mfma_kernel / gemm_pair_kernel (forward, dX, dW and paired dX + dW launches)"
+    roofline["kernel"] = "gemm_f32_kernel / gemm_pair_kernel (forward, dX, dW and paired dX + dW launches)"
+    roofline["sustained_peak"] = SUSTAINED_CONTRACTION_TFLOPS
     roofline["gemm_ms_per_step"] = roofline.pop("ms_per_step")
     roofline["measured_in"] = "events_pass"
     if alone:

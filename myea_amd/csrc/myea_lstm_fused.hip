@@ -564,8 +564,11 @@ int launch_transpose(hipStream_t s, size_t rows, size_t cols, const float *src, 
     return MYEA_OK;
 }
 
-// One workgroup per compute unit at most in either direction: beyond that the operands that every tile reads for itself cost more
-// than the launch that is saved (512 examples of 1000 cells would read 1 GB a step).
+// One workgroup per compute unit at most in either direction: a second round costs its own latency again, and every tile reads its
+// operands for itself.  us for 12 steps, two launches a step -> one, forward and forward with backward: 200 cells, 60 examples 167 -> 78
+// and 314 -> 157; 100, 570 164 -> 100 and 332 -> 203; 500, 128 211 -> 128 and 401 -> 271; 1001, 64 345 -> 193 and 654 -> 452; 2039, 32 571 ->
+// 290 and 1267 -> 737.  Beyond the line: 100, 1000 338 -> 272 with backward, 500, 256 485 -> 442, but 1001, 128 622 -> 767 and 2039, 64 980 ->
+// 1316.
 bool lstm_step_fits(size_t C, size_t cells_per_block, size_t B)
 {
     return cells_per_block == 1 && C > 0 && B > 0 && (B + 31) / 32 * ((C + 7) / 8) <= 256 && (B + 15) / 16 * ((C + 15) / 16) <= 256;

@@ -122,7 +122,8 @@ def test_c2_shape_relu_softmax_ce_shrunk(optimizer, extra):
 
 @pytest.mark.parametrize("B,Bmax", [(1, 1), (5, 8), (33, 33)])
 def test_ragged_shapes_use_the_guarded_path(B, Bmax):
-    """widths that are not multiples of 4 (unaligned weight slices), batch smaller than the allocated batch"""
+    """widths that are not multiples of 4 (unaligned weight slices; whole loads need 4-byte alignment only, tails are guarded), batch smaller
+    than the allocated batch"""
     specs = [dict(units=13), dict(units=31, activation="SIGMOID"), dict(units=7, activation="LEAKY_RELU"),
              dict(units=66, activation="ELLIOT_SYMMETRIC"), dict(units=3, activation="LINEAR")]
     desc, gpu, cpu = _pair(specs, Bmax, dict(type_optimizer_function=mb.OPTIMIZER["ADAM"], type_loss_function=mb.LOSS["MSE"]), seed=5)

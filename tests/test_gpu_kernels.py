@@ -1,4 +1,4 @@
-"""Kernel-level GPU checks through the C ABI: the FP32 MFMA contraction in all operand layouts against float64
+"""Kernel-level GPU checks through the C ABI: the FP32 contraction in all operand layouts against float64
 matmul (brute force) on ragged shapes, at BASELINE config 2's full shapes against torch.matmul (library routine)
 and through linearity; the fused optimizer kernel at an odd length against a float64 restatement."""
 import ctypes as C
