@@ -26,7 +26,7 @@ if ROOT not in sys.path:
 # HBM bytes per contraction launch (mean over the launches of one step): NOT measured by this script's run.  Recorded
 # from rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE runs of this script, scaled by what the same counters read for copies of
 # known size (FETCH_SIZE x2, WRITE_SIZE x1); the line names the file the figure comes from.
-RECORDED_TRAFFIC = {"fc4096x4_b1024_adam": dict(bytes_per_launch=2934498 * 1024 / 10,
+RECORDED_TRAFFIC = {"fc4096x4_b1024_adam": dict(bytes_per_launch=2958506 * 1024 / 10,
                                                 source="recorded constant, not measured in this run: profiles/hbm_traffic__fc4096x4_b1024_adam__pmc.txt"),
                     # the two resident time loops of one layer (forward + backward launch), mean per launch
                     "lstm512x2_t64_b256_amsgrad": dict(bytes_per_launch=(2 * 98055.1 + 230411.5 + 2 * 203936.9 + 197795.6) * 1024 / 2,

@@ -7,18 +7,20 @@
 //   weights  dW += delta^T X     (A m-contiguous, B n-contiguous)   Update_Derivative_Weight__FC,
 //            Neural_Network__Update_Derivative_Weight__OpenMP.cpp:178-216
 //
-// Arithmetic.  gfx950 multiplies FP32 at 157 TFLOP/s and BF16 at 2.5 PFLOP/s.  An FP32 number below 2^103 is the sum of three BF16
-// numbers, but for a power of two that keeps the smallest of them normal (myea_split.h): hi = x rounded to BF16, mid = (x - hi)
-// rounded to BF16, lo = what is left (8 + 8 + 8 significant bits, signs included, cover the 24 of x; both differences are exact in FP32).  Of the nine products of two such sums the six with a weight above 2^-24 are
-// formed - hi hi, hi mid, mid hi, mid mid, hi lo, lo hi - each exact in the matrix unit, all accumulated in FP32.  What is left
-// out is below 2^-25 of a product.  The five smaller products have an accumulator of their own, added at the end: an accumulator
-// as large as the result is rounded once per 16 k's, where v_mfma_f32_32x32x2_f32 rounds it at every second k, and the measured
-// error against 64-bit sums is smaller than that instruction's (normal operands, 2-norm: 4e-7 against 1.15e-6 at k = 4096,
-// 1.3e-7 against 4.1e-7 at k = 512; positive ones: 6.0e-7 against 1.7e-6 at k = 16384).  Six BF16 instructions for 16 k's
-// take 6 x 32 cycles of a SIMD's matrix unit where the FP32 ones take 8 x 64: the ceiling moves from 157 to 419 TFLOP/s, and to
-// 190 at the 1.14 PFLOP/s that a large BF16 product was measured to sustain on this card.  Measured, FP32 instruction -> this:
-// 1024 x 4096 x 4096 forward 314 -> 221 us, its weight gradient 304 -> 197 us (174 TFLOP/s), 16384 x 2048 x 512 269 -> 193 us
-// (178 TFLOP/s); 333 x 1201 x 1201, whose rows are no 16-byte multiples, 50 -> 25 us.
+// Arithmetic.  gfx950 multiplies FP32 at 157 TFLOP/s and BF16 at 2.5 PFLOP/s.  An FP32 number below 2^103 is the sum of three
+// BF16 numbers, but for a power of two that keeps the smallest of them normal (myea_split.h): hi = x rounded to BF16, mid = (x
+// - hi) rounded to BF16, lo = what is left (8 + 8 + 8 significant bits, signs included, cover the 24 of x; both differences
+// are exact in FP32).  Of the nine products of two such sums the six with a weight above 2^-24 are formed - hi hi, hi mid, mid
+// hi, mid mid, hi lo, lo hi - each exact in the matrix unit, all accumulated in FP32.  What is left out is below 2^-25 of a
+// product.  The five smaller products have an accumulator of their own, added at the end: an accumulator as large as the
+// result is rounded (to nearest, as measured) once per 16 k's, where v_mfma_f32_32x32x2_f32 rounds it at every second k, and
+// from 16 k's on (fewer are another kernel's) the measured error against 64-bit sums is smaller than that instruction's
+// (normal operands, 2-norm: 4e-7 against 1.15e-6 at k = 4096, 1.3e-7 against 4.1e-7 at k = 512; positive ones: 3.1e-7 against
+// 8.4e-7 at k = 4096, 6.0e-7 against 1.7e-6 at k = 16384).  Six BF16 instructions for 16 k's take 6 x 32 cycles of a SIMD's
+// matrix unit where the FP32 ones take 8 x 64: the ceiling moves from 157 to 419 TFLOP/s, and to 190 at the 1.14 PFLOP/s that
+// a large BF16 product was measured to sustain on this card.  Measured, FP32 instruction -> this: 1024 x 4096 x 4096 forward
+// 296 -> 197 us, its weight gradient 303 -> 196 us (176 TFLOP/s), 16384 x 2048 x 512 307 -> 199 us, 512 x 2048 x 2048 44.5 ->
+// 37.4; 333 x 1201 x 1201, whose rows are no 16-byte multiples and which is a short product now, 50 -> 21 us.
 // Infinities and NaN do not survive the split (inf - inf), nor do finite values whose scaled hi is a BF16 infinity: such a product
 // always leaves a non-finite accumulator, and a wavefront that finds one computes its accumulators again with the FP32
 // instruction (redo_in_f32), so the results are those of FP32 arithmetic there too.
@@ -28,8 +30,7 @@
 // two steps ahead or four), split there once, three BF16 planes -> LDS (two stages, one barrier per step).  What bounds a step is
 // issue: per 16 k's of a 128 x 128 tile a wavefront has 24 matrix instructions (768 cycles) and about 120 vector ones (480), so
 // the splitting of the next step is spread between the matrix instructions of this one (2048 x 2048 x 2048: 114 us with the
-// compiler's order, 98 us so).  An operand's place in LDS
-// does not depend on its orientation in memory:
+// compiler's order, 98 us so).  An operand's place in LDS does not depend on its orientation in memory:
 //   [plane][k / 8][row][8 k's]     a fragment (row l % 32, k's 8 (l / 32) .. + 7 of lane l) is one conflict-free ds_read_b128
 // Counted (1024 x 4096 x 4096, two workgroups a tile): the matrix unit is busy 56 % of the clocks, 5 vector instructions a matrix
 // instruction, no bank conflicts; 64 x 64 tiles (1024 x 1000 x 4096) 37 %, and a k-contiguous operand's stores, four chunks of a row at a

@@ -24,7 +24,7 @@ EXTRA = {
     "pooling_member_wide": ([fc(48), fc(64, "RELU"), res(3, normalization="BATCH_NORMALIZATION"), fc(96, "RELU", normalization="BATCH_NORMALIZATION"),
                              dict(type="max_pooling", kernel=3, stride=2, padding=1, dilation=2), fc(64, "TANH", dropout="BERNOULLI_INVERTED", keep=0.5),
                              fc(10, "SOFTMAX")], 32),
-    # odd widths: guarded scalar-load contraction path, shortcut wider and narrower in consecutive blocks
+    # odd widths: guarded tails and 4-byte-aligned rows of the contractions, shortcut wider and narrower in consecutive blocks
     "odd_widths": ([fc(19), res(2), fc(31, "TANH"), fc(27, "LEAKY_RELU"), res(1), fc(13, "SIGMOID"), fc(7, "LINEAR")], 11),
 }
 ALL = dict(CASES, **EXTRA)
