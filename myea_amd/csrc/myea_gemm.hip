@@ -739,8 +739,6 @@ void launch_short_waves(hipStream_t stream, const GemmDev &d, bool a_kc, bool b_
     else hipLaunchKernelGGL((short_gemm_kernel<false, false, WAVES>), grid, group, 0, stream, d);
 }
 
-long short_blocks(int M, int N) { return (long)((M + 31) / 32) * ((N + 31) / 32); }
-
 int launch_short(hipStream_t stream, GemmDev d, bool a_kc, bool b_kc)
 {
     d.nbm = (d.M + 31) / 32;
@@ -1116,11 +1114,12 @@ int launch_gemm(hipStream_t stream, const GemmParams &p)
         d.pair_partials = p.pair_partials; d.pair_tickets = p.pair_tickets;
         return launch_layout<64, 64>(stream, d, a_kc, b_kc);
     }
-    // The short product while two of its workgroups a compute unit are enough, slabs counted, at any k.  us, 64 x 64 tiles -> short, k
-    // = 64, 256, 1024, 4096 (the layouts' mean): 512 x 512 (256 workgroups) 4.7 -> 4.5, 7.9 -> 5.4, 21.1 -> 10.5, 75 -> 32; 640 x 768
-    // (480) 5.6 -> 5.8, 8.3 -> 7.6, 21.6 -> 17.3, 75 -> 57; 512 x 1024 (512) 5.2 -> 5.4, 8.2 -> 7.7, 21.5 -> 17.7, 75 -> 58; with a third
-    // workgroup a unit, 700 x 900 (638), 5.6 -> 7.5, 8.6 -> 10.6, 22.4 -> 25.9, 76 -> 85.
-    if (short_blocks(p.M, p.N) * d.ksplit <= 512) return launch_short(stream, d, a_kc, b_kc);
+    // The short product below 128 tiles of 64 x 64, slabs counted, at any k: two of its workgroups a compute unit are enough there.  us, 64 x
+    // 64 tiles -> short, k = 64, 256, 1024, 4096 (the layouts' mean): 512 x 512 (256 workgroups) 4.7 -> 4.5, 7.9 -> 5.4, 21.1 -> 10.5, 75 ->
+    // 32; 640 x 768 (480) 5.6 -> 5.8, 8.3 -> 7.6, 21.6 -> 17.3, 75 -> 57; with a third workgroup a unit, 700 x 900 (638), 5.6 -> 7.5, 8.6 ->
+    // 10.6, 22.4 -> 25.9, 76 -> 85.  (128 tiles exactly, 512 x 1024, would gain as well, 21.5 -> 17.7 at k = 1024, but are what a paired launch
+    // takes as tiles, and a product has the same bits there and alone.)
+    if (tiles_64 * d.ksplit < 128) return launch_short(stream, d, a_kc, b_kc);
     if (tiles_128 * 2 * d.ksplit < 256) return launch_layout<64, 64>(stream, d, a_kc, b_kc);
     if (p.M <= p.N) return launch_layout<64, 128>(stream, d, a_kc, b_kc);
     return launch_layout<128, 64>(stream, d, a_kc, b_kc);
@@ -1128,9 +1127,11 @@ int launch_gemm(hipStream_t stream, const GemmParams &p)
 
 // `a` = (A k-contiguous, B n-contiguous), `b` = (both k-strided), neither split along k, any alignment, and `a` no
 // more than about one 128 x 128 tile per CU: both in ONE launch (gemm_pair_kernel).  Returns MYEA_OK when launched, 1 when the pair form does not apply (the caller launches the two one after the other), a negative code on an error.
+// Either product has the bits that launch_gemm gives it: what that sends to a kernel of other sums (fewer than 16 k's) does not pair.
 int launch_gemm_pair(hipStream_t stream, const GemmParams &a, const GemmParams &b)
 {
     if (!a.a_k_contiguous || a.b_k_contiguous || b.a_k_contiguous || b.b_k_contiguous || a.split_k > 1 || b.split_k > 1) return 1;
+    if (a.K < kShallow || b.K < kShallow) return 1;
     GemmDev da, db;
     int rc = prepare_gemm(a, da);
     if (rc != MYEA_OK) return rc;

@@ -11,7 +11,7 @@ from tests.test_gpu_kernels import _gemm
 pytestmark = pytest.mark.gpu
 
 LAYOUTS = [(1, 1), (1, 0), (0, 0), (0, 1)]
-# the tiled kernel, a shape per tile: more than 512 tiles of 32 x 32 (below it is the short product's) and
+# the tiled kernel, a shape per tile: at least 128 tiles of 64 x 64 (below it is the short product's) and
 TILE_64 = [(700, 1000), (1001, 777), (1025, 1030)]   # fewer than 128 of 128 x 128
 TILE_64_128, TILE_128_64 = [(1500, 1501), (1409, 1500)], [(3001, 700), (1600, 1500)]   # up to 255 of them
 TILE_128 = [(2049, 2050), (2180, 1921)]
@@ -117,8 +117,8 @@ def test_values_the_split_cannot_carry(a_kc, b_kc, M, N):
 @pytest.mark.parametrize("M,N,K", [(1, 33, 1), (31, 1, 23), (33, 32, 24), (32, 65, 31), (64, 64, 33), (95, 100, 255), (100, 31, 257), (500, 490, 545),
                                    (257, 1000, 17), (700, 600, 33), (700, 600, 545), (512, 1024, 129), (30, 16300, 300), (520, 1000, 300)])
 def test_short_products_against_float64(a_kc, b_kc, M, N, K):
-    """Up to 512 workgroups of 32 x 32, of eight wavefronts up to 256 and of four beyond, that share k in runs of 32, of which the last ones
-    may have none or a part; the last shape has one workgroup too many."""
+    """Fewer than 128 tiles of 64 x 64: workgroups of 32 x 32, of eight wavefronts up to 256 of them and of four beyond, that share k in runs
+    of 32, of which the last ones may have none or a part; the last three shapes are the tiled kernel's."""
     A, B, Ad, Bd = _operands(a_kc, b_kc, M, N, K, M + N + K)
     C = torch.full((M, N), float("nan"), device="cuda")
     _gemm(mb.load_library(), a_kc, b_kc, 0, M, N, K, Ad, Bd, C)

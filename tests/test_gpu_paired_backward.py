@@ -108,3 +108,20 @@ def test_weight_gradient_rides_with_the_delta_at_batch_512(B):
     want = 2.0 * (delta[:, :48].T @ x)
     got = a.download_gradient()[l.first_connection_index:l.first_connection_index + 48 * 2048].reshape(48, 2048)
     assert_close(got, want, 1e-4, 1e-5 * float(np.abs(want).max()), what="dW rows 0..47 of layer 2")
+
+
+@pytest.mark.parametrize("specs,B", [
+    ([dict(units=64), dict(units=1024, activation="RELU"), dict(units=2048, activation="TANH"), dict(units=5, activation="LINEAR")], 512),
+    ([dict(units=8), dict(units=16384, activation="TANH"), dict(units=6, activation="TANH"), dict(units=6, activation="LINEAR")], 10),
+    ([dict(units=8), dict(units=16384, activation="TANH"), dict(units=24, activation="TANH"), dict(units=6, activation="LINEAR")], 28),
+], ids=["128-tiles", "fewer-than-16-k", "few-k"])
+def test_paired_launches_at_the_lines_of_the_other_kernels(specs, B):
+    """What rides in one launch with the weight gradient gives the bits of its own launch: 128 tiles of 64 x 64, one more than the short
+    product takes, and products over fewer k's than the paired kernel is for."""
+    desc, (a, b), X, Y, _ = _pair(specs, B)
+    for step in range(2):
+        _step(a, B, X, Y, fused=False)
+        _step(b, B, X, Y, fused=True)
+    assert np.array_equal(a.download_gradient(), b.download_gradient())
+    for li in range(1, desc.n_layers):
+        assert np.array_equal(a.download_tensor(li, mb.TENSOR["ERRORS"]), b.download_tensor(li, mb.TENSOR["ERRORS"]))
