@@ -72,3 +72,18 @@ def test_smaller_batch_with_more_slabs(layers, Bmax, batches):
 def test_small_lstm_over_many_rows():
     """Four gates of 16 cells over 32 inputs are one 64 x 64 tile: 18 slabs over 2 x 2304 rows."""
     _gradients([dict(units=32), dict(type="lstm", units=16), dict(units=16, activation="LINEAR")], 2304, 2, 2304, 5)
+
+
+@pytest.mark.gpu
+def test_call_without_allocations_sizes_its_pieces_for_the_batch():
+    """16 slabs at 3000 rows, 4 at 5000, in front of a second layer whose LSTM slabs lie behind them: bit for bit the ordinary call."""
+    from tests.test_zz_no_alloc import _gradients as both
+    desc = mb.make_desc([dict(units=256), dict(units=256, activation="TANH"), dict(type="lstm", units=16), dict(units=16, activation="LINEAR")], 5000)
+    net = mb.HipNetwork(desc, mb.default_hyper(type_optimizer_function=mb.OPTIMIZER["ADAM"], type_loss_function=mb.LOSS["MSE"]))
+    net.set_state_propagation(mb.STATE_TRAINING)
+    net.upload_parameters(glorot_parameters(desc, 9))
+    rng = np.random.default_rng(9)
+    for B in (5000, 3000):
+        X, Y = (rng.normal(0, 1, (B, n)).astype(np.float32) for n in (256, 16))
+        got, want = both(net, B, X, Y)
+        assert np.abs(want).max() > 0 and np.array_equal(got, want)
