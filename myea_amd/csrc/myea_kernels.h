@@ -300,7 +300,7 @@ int launch_lstm_step_forward(hipStream_t s, const LstmFusedForward &p);
 int launch_lstm_step_backward(hipStream_t s, const LstmFusedBackward &p);
 int launch_transpose(hipStream_t s, size_t rows, size_t cols, const float *src, float *dst);
 
-// ---- LSTM time loop as one resident launch (one cell per block, C in {128, 256, 512, 1024}) --------------------------
+// ---- LSTM time loop as one resident launch (one cell per block) -------------------------------------------------------
 // one direction of a layer: packed parameters and the layer's [T][Bmax][..] tensors
 struct LstmResidentDir {
     const float *Wrec;     // [4C][C] packed recurrent weights, rows z | i | f | o (forward)
@@ -316,25 +316,38 @@ struct LstmResidentDir {
     size_t zone_stride;
     int reverse;           // walks time from T - 1 down to 0
 };
+// The FP32 matrix instruction: 1024 cells, and the backward loop of 512 (myea_lstm_resident.hip).
 struct LstmResidentPlan {
     bool ok = false;       // the resident form applies
     bool agent = false;    // groups wider than one XCD: device-scope exchange
-    bool backward = false; // the backward loop has a resident form too
-    bool ksplit = false;   // ... and it is the one split along k, which needs the exchange buffer
-    bool ksplit_available = false;   // the k form exists for this layer (a caller may set ksplit when other work shares the device)
-    int cells = 0, members = 0, rs = 0, row_groups = 0, grid = 0, cus = 0;
+    int members = 0, row_groups = 0, grid = 0;
 };
-int lstm_resident_plan(size_t C, size_t cells_per_block, size_t B, int dirs, LstmResidentPlan *plan);
+int lstm_resident_plan(size_t C, size_t cells_per_block, size_t B, int dirs, bool backward, LstmResidentPlan *plan);
 size_t lstm_resident_sync_words();
 // sync: lstm_resident_sync_words() unsigneds of device memory (cleared by the call); host_flag: a pinned host word the
 // kernel sets when a bounded wait gave up (1) or the members of a group did not share an XCD (2); fault: a device word set
 // to 1 on the same occasions and never cleared by these calls (null: none)
 int launch_lstm_resident_forward(hipStream_t s, const LstmResidentPlan &plan, size_t T, size_t B, size_t Bmax, size_t C, int dirs,
                                  const LstmResidentDir *dir, unsigned *sync, unsigned *host_flag, unsigned *fault);
-// dh must hold the delta from the layers above for every time step.  exchange: device memory of at least
-// lstm_resident_exchange_floats(C, B, dirs) floats, 16-byte aligned, when plan.ksplit (its contents do not matter); else unused
-size_t lstm_resident_exchange_floats(size_t C, size_t B, int dirs);
+// dh must hold the delta from the layers above for every time step
 int launch_lstm_resident_backward(hipStream_t s, const LstmResidentPlan &plan, size_t T, size_t B, size_t Bmax, size_t C, int dirs,
-                                  const LstmResidentDir *dir, unsigned *sync, unsigned *host_flag, unsigned *fault, float *exchange, size_t exchange_floats);
+                                  const LstmResidentDir *dir, unsigned *sync, unsigned *host_flag, unsigned *fault);
+// The BF16 matrix cores: any width of 16 .. 512 cells (myea_lstm_planes.hip); sync, host_flag and fault as above.
+struct LstmPlanesPlan {
+    bool ok = false;
+    bool backward = false;  // the backward loop too
+    int members = 0, rs = 0, row_tiles = 0, row_groups = 0, grid = 0, cus = 0;
+};
+int lstm_planes_plan(size_t C, size_t cells_per_block, size_t B, size_t Bmax, int dirs, LstmPlanesPlan *plan);
+size_t lstm_planes_sync_words();
+// floats of the forward loop's exchange buffer (16-byte aligned, cleared by the call) for up to B examples per direction
+size_t lstm_planes_exchange_floats(size_t C, size_t B, int dirs);
+int launch_lstm_planes_forward(hipStream_t s, const LstmPlanesPlan &plan, size_t T, size_t B, size_t Bmax, size_t C, int dirs, const LstmResidentDir *dir,
+                               unsigned *sync, unsigned *host_flag, unsigned *fault, float *exchange, size_t exchange_floats);
+// floats of the backward loop's buffer (16-byte aligned): absent - every bit set - before the first launch, and again after every one that
+// ran to its end
+size_t lstm_planes_shares_floats(size_t C, size_t B, int dirs);
+int launch_lstm_planes_backward(hipStream_t s, const LstmPlanesPlan &plan, size_t T, size_t B, size_t Bmax, size_t C, int dirs, const LstmResidentDir *dir,
+                                unsigned *sync, unsigned *host_flag, unsigned *fault, float *shares, size_t shares_floats);
 
 }  // namespace myea

@@ -17,6 +17,7 @@
 //
 // NN/ = Neural_Network_Library_Windows/Source_Files/Neural_Network/.
 #include <cstdlib>
+#include <mutex>
 #include <type_traits>
 
 #include "myea_device_af.h"
@@ -1208,7 +1209,7 @@ int Net::lstm_create_layer(size_t li)
         q->renorm = l.type_normalization == MYEA_NORMALIZATION_BATCH_RENORMALIZATION;
         q->fused = !q->norm && lstm_fused_supported(q->C, q->cpb) && !fused_lstm_disabled();
         if (q->fused) MYEA_TRY(dev_alloc_zero(&q->WrecT, q->C * q->G));
-        if (q->fused) MYEA_TRY(dev_alloc_zero(&q->sums, (B + 31) / 32 * 7 * q->C));
+        if (!q->norm && q->cpb == 1) MYEA_TRY(dev_alloc_zero(&q->sums, (B + 15) / 16 * 7 * q->C));
         MYEA_TRY(dev_alloc_zero(&q->gWin, gradient_slabs(q->G, q->In, T * B) * q->G * q->In));   // split-K slabs of the weight-gradient contractions
         MYEA_TRY(dev_alloc_zero(&q->gWrec, gradient_slabs(q->G, q->C, T * B) * q->G * q->C));
         q->gWin_own = q->gWin; q->gWrec_own = q->gWrec;
@@ -1239,9 +1240,11 @@ int Net::lstm_create_layer(size_t li)
             MYEA_HIP_TRY(hipDeviceSynchronize());
         }
     }
-    // the widest layer sizes the buffer the members of a resident backward loop hand each other partial sums through
-    if (o.lstm->fused && o.lstm->cpb == 1)
-        resident_exchange_floats = std::max(resident_exchange_floats, lstm_resident_exchange_floats(o.lstm->C, B, (int)dirs));
+    // the widest layer sizes the buffers the members of a resident loop hand each other their results through
+    if (!o.lstm->norm && o.lstm->cpb == 1 && T > 1) {
+        planes_exchange_floats = std::max(planes_exchange_floats, lstm_planes_exchange_floats(o.lstm->C, B, (int)dirs));
+        planes_shares_floats = std::max(planes_shares_floats, lstm_planes_shares_floats(o.lstm->C, B, (int)dirs));
+    }
     return MYEA_OK;
 }
 
@@ -1557,12 +1560,79 @@ int Net::lstm_backward_step_norm(LstmLayer &q, size_t B, size_t s)
     return MYEA_OK;
 }
 
+// Two resident loops at once may each hold compute units that the other's workgroups wait for.  So while more than one network of the
+// process has such layers on a device, a loop waits (on the device) for the loop launched before it on another network's stream; a
+// stream that is being captured is left alone.
+namespace {
+
+struct LoopOrder {
+    std::mutex mutex;
+    int networks = 0;
+    hipEvent_t last = nullptr;         // behind the last loop launched
+    const void *owner = nullptr;       // the network that launched it
+};
+LoopOrder g_loop_order[64];
+
+struct LoopTurn {
+    LoopOrder *order = nullptr;
+    const void *net;
+    hipStream_t stream;
+    LoopTurn(const void *n, int device, hipStream_t s) : net(n), stream(s)
+    {
+        if (device < 0) return;
+        LoopOrder &o = g_loop_order[device];
+        o.mutex.lock();
+        order = &o;
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        if (o.networks < 2 || hipStreamIsCapturing(stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) { leave(); return; }
+        if (!o.last && hipEventCreateWithFlags(&o.last, hipEventDisableTiming) != hipSuccess) { o.last = nullptr; leave(); return; }
+        if (o.owner && o.owner != net) (void)hipStreamWaitEvent(stream, o.last, 0);
+    }
+    void leave()
+    {
+        if (order) order->mutex.unlock();
+        order = nullptr;
+    }
+    ~LoopTurn()
+    {
+        if (!order) return;
+        if (hipEventRecord(order->last, stream) == hipSuccess) order->owner = net;
+        leave();
+    }
+    LoopTurn(const LoopTurn &) = delete;
+    LoopTurn &operator=(const LoopTurn &) = delete;
+};
+
+}  // namespace
+
+int Net::loop_order_join()
+{
+    int dev = -1;
+    MYEA_HIP_TRY(hipGetDevice(&dev));
+    if (dev < 0 || dev >= 64 || loop_device >= 0) return MYEA_OK;
+    LoopOrder &o = g_loop_order[dev];
+    std::lock_guard<std::mutex> lock(o.mutex);
+    loop_device = dev;
+    if (++o.networks == 2) (void)hipDeviceSynchronize();   // the first network's loops so far have left no event behind
+    return MYEA_OK;
+}
+
+void Net::loop_order_leave()
+{
+    if (loop_device < 0) return;
+    LoopOrder &o = g_loop_order[loop_device];
+    std::lock_guard<std::mutex> lock(o.mutex);
+    --o.networks;
+    if (o.owner == this) o.owner = nullptr;
+    loop_device = -1;
+}
+
 bool Net::lstm_backward_loop_leaves_room(size_t li, size_t B)
 {
     const DevLayer &o = L[li];
     if (!o.lstm) return false;
-    LstmResidentPlan plan;
-    if (lstm_resident_plan(o.lstm->C, o.lstm->cpb, B, o.lstm2 ? 2 : 1, &plan) != MYEA_OK || !plan.ok || !plan.backward) return false;
+    LstmPlanesPlan plan;
+    if (o.lstm->norm || lstm_planes_plan(o.lstm->C, o.lstm->cpb, B, d.batch_size, o.lstm2 ? 2 : 1, &plan) != MYEA_OK || !plan.ok || !plan.backward) return false;
     return 2 * plan.grid <= plan.cus;
 }
 
@@ -1607,18 +1677,41 @@ int Net::lstm_forward_layer(size_t li, size_t B)
     DevLayer &o = L[li];
     const size_t T = d.number_recurrent_depth;
     const double loop_work = 2.0 * (double)(T - 1) * (double)B * (double)o.lstm->G * (double)o.lstm->C;   // the recurrent contractions of steps 1 .. T-1
-    if (T > 1 && o.lstm->fused && !resident_off && resident_sync) {
-        // the whole time loop (both directions) as one launch when the layer's shape and the device allow it
-        LstmResidentPlan plan;
+    if (T > 1 && !o.lstm->norm && !fused_lstm_disabled() && !resident_off && planes_sync) {
+        LstmPlanesPlan plan;
         const int dirs = o.lstm2 ? 2 : 1;
-        MYEA_TRY(lstm_resident_plan(o.lstm->C, o.lstm->cpb, B, dirs, &plan));
+        MYEA_TRY(lstm_planes_plan(o.lstm->C, o.lstm->cpb, B, d.batch_size, dirs, &plan));
         if (plan.ok) {
             MYEA_TRY(lstm_forward_inputs(li, *o.lstm, B));
             if (o.lstm2) MYEA_TRY(lstm_forward_inputs(li, *o.lstm2, B));
             LstmResidentDir rd[2];
             lstm_resident_dirs(o, rd);
             prof_begin(kProfLstmForwardLoop);
-            MYEA_TRY(launch_lstm_resident_forward(stream, plan, T, B, d.batch_size, o.lstm->C, dirs, rd, resident_sync, resident_flag, fault));
+            {
+                LoopTurn turn(this, loop_device, stream);
+                MYEA_TRY(launch_lstm_planes_forward(stream, plan, T, B, d.batch_size, o.lstm->C, dirs, rd, planes_sync, resident_flag, fault, planes_exchange, planes_exchange_floats));
+            }
+            prof_end(dirs * loop_work, 1);
+            if (!o.lstm2) return MYEA_OK;
+            const size_t rows = (size_t)d.number_recurrent_depth * d.batch_size;
+            return launch_padded_add(stream, rows, o.H, o.lstm->h, o.H, 0, o.lstm2->h, o.H, 0, o.values);  // output = h_forward + h_backward
+        }
+    }
+    if (T > 1 && o.lstm->fused && !resident_off && resident_sync) {
+        // the whole time loop (both directions) as one launch when the layer's shape and the device allow it
+        LstmResidentPlan plan;
+        const int dirs = o.lstm2 ? 2 : 1;
+        MYEA_TRY(lstm_resident_plan(o.lstm->C, o.lstm->cpb, B, dirs, false, &plan));
+        if (plan.ok) {
+            MYEA_TRY(lstm_forward_inputs(li, *o.lstm, B));
+            if (o.lstm2) MYEA_TRY(lstm_forward_inputs(li, *o.lstm2, B));
+            LstmResidentDir rd[2];
+            lstm_resident_dirs(o, rd);
+            prof_begin(kProfLstmForwardLoop);
+            {
+                LoopTurn turn(this, loop_device, stream);
+                MYEA_TRY(launch_lstm_resident_forward(stream, plan, T, B, d.batch_size, o.lstm->C, dirs, rd, resident_sync, resident_flag, fault));
+            }
             prof_end(dirs * loop_work, 1);
             if (!o.lstm2) return MYEA_OK;
             const size_t rows = (size_t)d.number_recurrent_depth * d.batch_size;
@@ -1714,19 +1807,40 @@ int Net::lstm_backward_layer(size_t li, size_t B)
     };
     for (LstmLayer *q : {o.lstm, o.lstm2})
         if (q) q->sums_groups = 0;   // the gate deltas are about to change
-    if (T > 1 && o.lstm->fused && !resident_off && resident_sync) {
-        LstmResidentPlan plan;
+    if (T > 1 && !o.lstm->norm && !fused_lstm_disabled() && !resident_off && planes_sync) {
+        LstmPlanesPlan plan;
         const int dirs = o.lstm2 ? 2 : 1;
-        MYEA_TRY(lstm_resident_plan(o.lstm->C, o.lstm->cpb, B, dirs, &plan));
-        if (plan.ok && plan.backward) {   // the whole backward time loop (both directions) as one launch
-            // weight contractions are about to run beside this loop: the form that leaves them room in LDS
-            if (loop_shares_device && plan.ksplit_available) plan.ksplit = true;
+        MYEA_TRY(lstm_planes_plan(o.lstm->C, o.lstm->cpb, B, d.batch_size, dirs, &plan));
+        if (plan.ok && plan.backward) {
             MYEA_TRY(seed(*o.lstm));
             if (o.lstm2) MYEA_TRY(seed(*o.lstm2));
             LstmResidentDir rd[2];
             lstm_resident_dirs(o, rd);
             prof_begin(kProfLstmBackwardLoop);
-            MYEA_TRY(launch_lstm_resident_backward(stream, plan, T, B, d.batch_size, o.lstm->C, dirs, rd, resident_sync, resident_flag, fault, resident_exchange, resident_exchange_floats));
+            {
+                LoopTurn turn(this, loop_device, stream);
+                MYEA_TRY(launch_lstm_planes_backward(stream, plan, T, B, d.batch_size, o.lstm->C, dirs, rd, planes_sync, resident_flag, fault, planes_shares, planes_shares_floats));
+            }
+            prof_end(dirs * loop_work, 1);
+            for (LstmLayer *q : {o.lstm, o.lstm2})
+                if (q && q->sums) { q->sums_groups = (size_t)plan.row_groups; q->sums_batch = B; }
+            return MYEA_OK;
+        }
+    }
+    if (T > 1 && o.lstm->fused && !resident_off && resident_sync) {
+        LstmResidentPlan plan;
+        const int dirs = o.lstm2 ? 2 : 1;
+        MYEA_TRY(lstm_resident_plan(o.lstm->C, o.lstm->cpb, B, dirs, true, &plan));
+        if (plan.ok) {   // the whole backward time loop (both directions) as one launch
+            MYEA_TRY(seed(*o.lstm));
+            if (o.lstm2) MYEA_TRY(seed(*o.lstm2));
+            LstmResidentDir rd[2];
+            lstm_resident_dirs(o, rd);
+            prof_begin(kProfLstmBackwardLoop);
+            {
+                LoopTurn turn(this, loop_device, stream);
+                MYEA_TRY(launch_lstm_resident_backward(stream, plan, T, B, d.batch_size, o.lstm->C, dirs, rd, resident_sync, resident_flag, fault));
+            }
             prof_end(dirs * loop_work, 1);
             for (LstmLayer *q : {o.lstm, o.lstm2})
                 if (q && q->sums) { q->sums_groups = (size_t)plan.row_groups; q->sums_batch = B; }

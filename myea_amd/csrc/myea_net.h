@@ -140,8 +140,12 @@ struct Net {
     void pair_buffers(GemmParams *g, float *partials, unsigned *tickets) const;   // a contraction's meeting place and fault words
     float *gemm_pair_partials = nullptr;       // scratch of the contractions that split a tile's k between two workgroups
     unsigned *gemm_pair_tickets = nullptr;
-    float *resident_exchange = nullptr;   // partial sums the members of a group hand each other in the backward loop
-    size_t resident_exchange_floats = 0;
+    unsigned *planes_sync = nullptr;      // words and buffers of the time loops on the BF16 matrix cores (myea_lstm_planes.hip)
+    float *planes_exchange = nullptr, *planes_shares = nullptr;
+    size_t planes_exchange_floats = 0, planes_shares_floats = 0;
+    int loop_device = -1;             // the device whose order of loops this network is part of, -1: none
+    int loop_order_join();
+    void loop_order_leave();
     bool resident_off = false;
     int resident_check();   // MYEA_E_DEVICE (once) after a resident launch reported a give-up
     unsigned long long *index_stage = nullptr;   // [Bmax] example indices of a gathered batch
@@ -203,7 +207,6 @@ struct Net {
     int update_derivative_weight_contraction(size_t li, size_t B);   // the weight contraction(s) of one layer
     bool dw_beside_loop_allowed(size_t gi, size_t li, size_t B);
     bool dw_beside_loop = false;       // this pass put weight contractions on the side stream beside a time loop: join before returning
-    bool loop_shares_device = false;   // set around a time loop that weight contractions will run beside
     // the same call with every scratch buffer of its kernels taken from the library's static device array
     int update_derivative_weight_no_alloc(size_t B, size_t first, size_t end);
     int update_parameter(size_t B, size_t training_size);

@@ -377,7 +377,14 @@ int Net::create(const myea_net_desc &desc)
             void *q = nullptr;
             MYEA_HIP_TRY(hipMalloc(&q, lstm_resident_sync_words() * sizeof(unsigned)));
             resident_sync = static_cast<unsigned *>(q);
-            if (resident_exchange_floats) MYEA_TRY(dev_alloc(&resident_exchange, resident_exchange_floats));
+            if (T > 1) MYEA_TRY(loop_order_join());
+            if (planes_exchange_floats) {
+                MYEA_HIP_TRY(hipMalloc(&q, lstm_planes_sync_words() * sizeof(unsigned)));
+                planes_sync = static_cast<unsigned *>(q);
+                MYEA_TRY(dev_alloc(&planes_exchange, planes_exchange_floats));
+                MYEA_TRY(dev_alloc(&planes_shares, planes_shares_floats));
+                MYEA_HIP_TRY(hipMemset(planes_shares, 0xff, planes_shares_floats * sizeof(float)));
+            }
         }
     }
     MYEA_TRY(dev_alloc(&tmp1, T * B * max_h));
@@ -449,6 +456,7 @@ int Net::create(const myea_net_desc &desc)
 
 Net::~Net()
 {
+    loop_order_leave();
     if (side_stream) {
         (void)hipStreamSynchronize(side_stream);
         (void)hipStreamDestroy(side_stream);
@@ -467,7 +475,7 @@ Net::~Net()
         lstm_destroy_layer(o);
     }
     fr(resident_sync);
-    fr(resident_exchange);
+    fr(planes_sync); fr(planes_exchange); fr(planes_shares);
     fr(gemm_pair_partials); fr(gemm_pair_tickets); fr(fault);
     if (resident_flag) (void)hipHostFree(resident_flag);
     fr(bn_shares); fr(bn_jobs); fr(narrow_slabs); fr(fold_jobs); fr(clip_ranges);
@@ -1406,10 +1414,7 @@ int Net::backward_pass(size_t B)
             // its workgroups are placed first.  MYEA_DW_BESIDE_LOOP=0 keeps them behind the loop on the one stream.
             const bool beside = pairing && dw_beside_loop_allowed(gi, li, B);
             if (beside) MYEA_HIP_TRY(hipEventRecord(fork_event, stream));
-            loop_shares_device = beside;
-            const int loop_rc = lstm_backward_layer(li, B);
-            loop_shares_device = false;
-            MYEA_TRY(loop_rc);
+            MYEA_TRY(lstm_backward_layer(li, B));
             if (beside) {
                 MYEA_HIP_TRY(hipStreamWaitEvent(side_stream, fork_event, 0));
                 std::swap(stream, side_stream);

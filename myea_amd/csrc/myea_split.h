@@ -19,6 +19,7 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));   // a 16-byte load from any element's address
 
 // the smaller five of the six products a_x b_y, in this order; hi hi has an accumulator of its own

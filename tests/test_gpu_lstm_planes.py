@@ -1,0 +1,93 @@
+"""The LSTM time loops on the BF16 matrix cores (16 .. 512 cells, any width) where they can go wrong: an odd number of members (half a
+block of k's without an owner), one member, a last member of one cell, one and several row tiles per group, a last group with fewer of
+them, examples missing from the last tile, more steps than the exchange buffer has slots, two directions, zoneout, a smaller batch
+behind a larger one - against one launch per time step (MYEA_LSTM_RESIDENT=0; the two paths sum in another order and round their gate
+functions differently by a few ulp: rel 1e-4 / abs 1e-5 as for the other LSTM paths) - and what the planes cannot hold."""
+import numpy as np
+import pytest
+import torch
+
+from myea_amd import binding as mb
+from tests.common import assert_close, environment, run_step
+from tests.test_gpu_lstm_resident import ABS, REL, _compare, _loop_launches, _net, _setup, lstm, zone
+
+pytestmark = pytest.mark.gpu
+
+# cells, two directions, zoneout, T, B, Bmax
+CASES = [(16, False, False, 9, 1, 1), (17, False, False, 5, 16, 16), (47, False, False, 6, 17, 20), (257, True, False, 6, 33, 40),
+         (200, False, True, 7, 60, 60), (256, False, False, 5, 520, 520), (512, False, True, 6, 129, 136), (511, True, False, 5, 70, 70),
+         (500, False, False, 5, 300, 300), (64, True, True, 12, 3, 4)]
+
+
+@pytest.mark.parametrize("cells,both,zoned,T,B,Bmax", CASES)
+def test_loop_of_any_width(cells, both, zoned, T, B, Bmax):
+    specs = [dict(units=7), (zone if zoned else lstm)(cells, **(dict(bidirectional=True) if both else {})), dict(units=cells, activation="LINEAR")]
+    desc, h, w, masks, X, Y = _setup(specs, T, B, Bmax, seed=cells)
+    loop, steps = _net(desc, h, w, masks), _net(desc, h, w, masks)
+    for b in (B, (B + 1) // 2):
+        with environment(MYEA_LSTM_RESIDENT="0"):
+            steps.Clear_Training_Arrays()
+            run_step(steps, b, X[:b], Y[:b], update=False)
+        loop.Clear_Training_Arrays()
+        loop.profile_enable(True)
+        run_step(loop, b, X[:b], Y[:b], update=False)
+        launches = _loop_launches(loop)
+        loop.profile_enable(False)
+        assert launches == (1, 1), "the time loops did not run as one launch each"
+        _compare(desc, loop, steps, b, T, "%d examples" % b)
+
+
+@pytest.mark.parametrize("cells,B", [(40, 20), (300, 200)])
+def test_weights_beyond_the_planes(cells, B):
+    """Recurrent weights of 2^110 next to ordinary ones: the planes of such a weight are an infinity and NaNs, so every sum it is part of
+    is computed again; forward, the gates saturate (or not, where a weight meets an h of zero) as with one launch per step; backward, the
+    share of a member that holds one is finite or an infinity as there."""
+    T = 4
+    specs = [dict(units=5), lstm(cells), dict(units=cells, activation="LINEAR")]
+    desc, h, w, masks, X, Y = _setup(specs, T, B, B, seed=3)
+    layer = desc.layers[1]
+    rng = np.random.default_rng(5)
+    at = rng.choice(np.arange(layer.first_connection_index, layer.last_connection_index), 40, replace=False)
+    for value in (2.0 ** 110, np.inf):
+        v = w.copy()
+        v[at] = np.float32(value)
+        out = []
+        for resident in ("1", "0"):
+            net = _net(desc, h, v, masks)
+            with environment(MYEA_LSTM_RESIDENT=resident):
+                net.Forward_Pass(B, X)
+                out.append(net.download_tensor(1, mb.TENSOR["OUTPUTS"], T * B * cells).copy())
+                if np.isfinite(value):
+                    net.Compute__Error(B, Y)
+                    net.Backward_Pass(B)
+                    out[-1] = (out[-1], net.download_tensor(1, mb.TENSOR["ERRORS"], T * B * cells).copy())
+                else:
+                    out[-1] = (out[-1],)
+        for a, b in zip(*out):
+            same = np.isfinite(a) & np.isfinite(b)
+            assert np.array_equal(np.isnan(a), np.isnan(b)) and np.array_equal(a[~same], b[~same], equal_nan=True)
+            scale = float(np.abs(b[same]).max())
+            assert_close(a[same] / scale, b[same] / scale, REL, ABS, what="weights of %g" % value)
+
+
+def test_two_networks_on_two_streams_take_turns():
+    """each loop fills the device by itself: launched side by side, their workgroups would wait for compute units the other's hold"""
+    T, B, cells = 24, 256, 500
+    specs = [dict(units=5), lstm(cells), dict(units=cells, activation="LINEAR")]
+    desc, h, w, masks, X, Y = _setup(specs, T, B, B, seed=11)
+    nets = [_net(desc, h, w, masks) for _ in range(2)]
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    x, y = torch.from_numpy(X).cuda(), torch.from_numpy(Y).cuda()
+    torch.cuda.synchronize()
+    for n, s in zip(nets, streams):
+        n.set_stream(s.cuda_stream)
+    for _ in range(6):
+        for n in nets:
+            n.Clear_Training_Arrays()
+            n.Forward_Pass(B, x, on_device=True)
+            n.Compute__Error(B, y, on_device=True)
+            n.Backward_Pass(B)
+    for n in nets:
+        n.synchronize()   # a wait that gave up is reported here
+    a, b = (n.download_tensor(1, mb.TENSOR["ERRORS"], T * B * cells) for n in nets)
+    assert np.array_equal(a, b)
