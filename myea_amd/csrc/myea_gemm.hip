@@ -616,41 +616,138 @@ int launch_layout(hipStream_t stream, const GemmDev &d, bool a_kc, bool b_kc)
 // ---- a short product ----------------------------------------------------------------------------------------------------
 // A product with too few 64 x 64 tiles to occupy the chip - a batch of 128 in front of 256 units is 8 of them - spends the tiled
 // kernel's time in its K steps, one behind the other on a few compute units.  Here a workgroup owns 32 rows x 32 columns and its
-// WAVES wavefronts share k: each takes every WAVES-th run of 32 k's, asks for its operands straight from memory in
-// the lanes that multiply them (A: lane l takes row l % 32, k's 8 (l / 32) .. + 7 of a group of 16; B alike), a run ahead of the
-// one it splits and multiplies; no LDS and no barrier until the wavefronts' accumulators are added, in wavefront order, by the
-// first, which runs the tiled kernel's epilogue.  What bounds it is the latency of the first operands and the splitting, which
-// every workgroup of a row or column of tiles repeats; a layer of 256 units over a batch of 128 (k = 784) went from 19 to 8 us.
+// WAVES wavefronts share k: each takes every WAVES-th run of 32 k's, a run ahead of the one it splits and multiplies; no barrier until the
+// wavefronts' accumulators are added, in wavefront order, by the first, which runs the tiled kernel's epilogue.  What bounds it is
+// the latency of the first operands and the splitting, which every workgroup of a row or column of tiles repeats.  Loading a k-contiguous
+// operand in whole lines and turning it round in LDS, and addresses that are scalar but for a lane's constant, took (us) 256 x 1024, k =
+// 1024 forward 11.8 -> 10.4, backward 11.0 -> 9.3; 512 x 100, k = 2048 18.2 -> 14.5; 64 x 512, k = 512 7.4 -> 6.0; 333 x 1201, k = 1201 20.9
+// -> 20.7 and 21.4 -> 19.2 (three runs in registers instead of two: no better at long k, 0.3 - 0.9 worse at short).
 // launch_gemm says up to where it pays.
 constexpr int kShortMost = 256;   // workgroups: one of eight wavefronts per compute unit
 constexpr int kShortRun = 32;   // k's: one 128-byte line of a k-contiguous row
 
-template <bool KC, int WAVES>
+// Operands are read through buffer instructions: the lane's part of an address is set up once, a run's part is scalar, and the range ends
+// where this workgroup's k's do.  short_fits: offsets are 32 bits wide.
+inline bool short_fits(const GemmDev &d, bool a_kc, bool b_kc)
+{
+    const long most = 0x1c000000L;   // floats
+    auto fits = [&](bool kc, long ld, long rows) { return kc ? 32 * ld + d.K < most : ((long)d.K + 2 * kShortRun * 8) * ld + rows < most; };
+    return fits(a_kc, d.lda, d.M) && fits(b_kc, d.ldb, d.N);
+}
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t short_range(const float *base, long floats)
+{
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(base), 0, (int)(floats * (long)sizeof(float)), 0x00020000);
+}
+
+// An operand whose k's are not contiguous: a lane's eight k's are eight loads, 32 columns - a line - each; k's beyond the last lie beyond
+// the range and read as zeros.
+template <bool KC, int WAVES, bool TURN>
 struct ShortOperand {
     float reg[2][2][8];   // [slot][group of 16 k's][k]
-    const float *at;      // of the run that is loaded next
-    long ld, step;
-    int left;             // k's from this lane's first one in that run on
+    __amdgpu_buffer_rsrc_t range;
+    int lane_at, run_at, ld;   // bytes
 
-    __device__ __forceinline__ void init(const float *base, long ld_, int row, int extent, long k0, int K)
+    // rows (columns) from `first` on, k's from k_begin to k_end; the wavefront's first run is `run` k's further on
+    __device__ __forceinline__ void init(const float *base, long ld_, int first, int extent, int k_begin, int k_end, int run, float *)
     {
-        const long r = min(row, extent - 1);
-        ld = ld_; left = K - k0;
-        at = base + (KC ? r * ld + k0 : k0 * ld + r);
-        step = KC ? (long)kShortRun * WAVES : (long)kShortRun * WAVES * ld;
+        const int lane = threadIdx.x & 63;
+        range = short_range(base + (long)k_begin * ld_ + first, (long)(k_end - k_begin - 1) * ld_ + (extent - first));
+        ld = (int)ld_ * 4;
+        lane_at = (lane >> 5) * 8 * ld + min(lane & 31, extent - 1 - first) * 4;
+        run_at = run * ld;
     }
-    __device__ __forceinline__ void load(int slot)
+    __device__ __forceinline__ void load(int slot, int)
     {
-        if (left >= 24) {   // this lane's last k of the run is the 24th
+#pragma unroll
+        for (int g = 0; g < 2; ++g)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) reg[slot][g][e] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(range, lane_at, run_at + (g * 16 + e) * ld, 0));
+        run_at += kShortRun * WAVES * ld;
+    }
+    __device__ __forceinline__ void place(int) {}
+    __device__ __forceinline__ void fetch(int slot, int g, float (&x)[8]) const
+    {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = reg[slot][g][e];
+    }
+};
+
+// An operand whose k's are contiguous.  The matrix instruction wants a lane to hold eight k's of one row: loaded so, every load instruction
+// touches 32 rows' lines for 16 bytes each, and the address path takes a line at a time.  So eight lanes bring a row's 128 bytes - any
+// alignment - and the wavefront turns them round in 4 KiB of LDS of its own: 16-byte chunks, XOR-swizzled by row, no barrier.
+template <int WAVES>
+struct ShortOperand<true, WAVES, true> {
+    u32x4 reg[2][4];   // [slot][rows 8 q + lane / 8]
+    __amdgpu_buffer_rsrc_t range;
+    int lane_at[4], run_at;   // bytes
+    float *tile;          // [32 rows][32 k's]
+
+    static __device__ __forceinline__ int chunk(int row, int c) { return row * 32 + ((c ^ ((row >> 1) & 7)) << 2); }
+    __device__ __forceinline__ void init(const float *base, long ld, int first, int extent, int k_begin, int k_end, int run, float *tile_)
+    {
+        const int lane = threadIdx.x & 63, last = min(31, extent - 1 - first);
+        tile = tile_;
+        range = short_range(base + first * ld + k_begin, last * ld + (k_end - k_begin));
+#pragma unroll
+        for (int q = 0; q < 4; ++q) lane_at[q] = (min(q * 8 + (lane >> 3), last) * (int)ld + (lane & 7) * 4) * 4;
+        run_at = run * 4;
+    }
+    __device__ __forceinline__ void load(int slot, int left)   // left: k's from the run's first on
+    {
+        if (left >= kShortRun) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) reg[slot][q] = __builtin_amdgcn_raw_buffer_load_b128(range, lane_at[q], run_at, 0);
+        } else {   // the rest of a row: word by word, the row's last in the place of those beyond it, and zeros in their place
+            const int mine = left - (int)(threadIdx.x & 7) * 4;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int back = (e - min(e, mine - 1)) * 4;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const unsigned v = __builtin_amdgcn_raw_buffer_load_b32(range, lane_at[q] + e * 4 - back, run_at, 0);
+                    reg[slot][q][e] = e < mine ? v : 0u;
+                }
+            }
+        }
+        run_at += kShortRun * WAVES * 4;
+    }
+    __device__ __forceinline__ void place(int slot)
+    {
+        const int lane = threadIdx.x & 63;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) *reinterpret_cast<u32x4 *>(tile + chunk(q * 8 + (lane >> 3), lane & 7)) = reg[slot][q];
+    }
+    __device__ __forceinline__ void fetch(int, int g, float (&x)[8]) const
+    {
+        const int lane = threadIdx.x & 63, row = lane & 31, c = g * 4 + (lane >> 5) * 2;
+        *reinterpret_cast<f32x4 *>(x) = *reinterpret_cast<const f32x4 *>(tile + chunk(row, c));
+        *reinterpret_cast<f32x4 *>(x + 4) = *reinterpret_cast<const f32x4 *>(tile + chunk(row, c + 1));
+    }
+};
+
+// The same in the lanes that multiply it.  Where A has only a few rows, all lanes of an instruction are in their lines, and the trip through
+// LDS and the set-up of the ranges are what remains (1 x 256, k = 784: 7.3 us against 7.6; 8 x 1000, k = 1000 9.0 against 9.9; 16 x 1000 9.3
+// against 9.1; 24 x 2048, k = 2048 17.3 against 14.5).
+constexpr int kShortDirectRows = 8;
+template <int WAVES>
+struct ShortOperand<true, WAVES, false> {
+    float reg[2][2][8];   // [slot][group of 16 k's][k]
+    const float *at;      // of the run that is loaded next
+    int mine;             // k's from this lane's first one in that run on
+
+    __device__ __forceinline__ void init(const float *base, long ld, int first, int extent, int k_begin, int k_end, int run, float *)
+    {
+        const int lane = threadIdx.x & 63, k0 = k_begin + run + (lane >> 5) * 8;
+        at = base + min(first + (lane & 31), extent - 1) * ld + k0;
+        mine = k_end - k0;
+    }
+    __device__ __forceinline__ void load(int slot, int)
+    {
+        if (mine >= 24) {   // this lane's last k of the run is the 24th
 #pragma unroll
             for (int g = 0; g < 2; ++g) {
-                if (KC) {
-                    *reinterpret_cast<f32x4 *>(reg[slot][g]) = *reinterpret_cast<const f32x4_any *>(at + g * 16);
-                    *reinterpret_cast<f32x4 *>(reg[slot][g] + 4) = *reinterpret_cast<const f32x4_any *>(at + g * 16 + 4);
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) reg[slot][g][e] = at[(g * 16 + e) * ld];
-                }
+                *reinterpret_cast<f32x4 *>(reg[slot][g]) = *reinterpret_cast<const f32x4_any *>(at + g * 16);
+                *reinterpret_cast<f32x4 *>(reg[slot][g] + 4) = *reinterpret_cast<const f32x4_any *>(at + g * 16 + 4);
             }
         } else {
 #pragma unroll
@@ -658,54 +755,70 @@ struct ShortOperand {
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
                     reg[slot][g][e] = 0.f;
-                    if (g * 16 + e < left) reg[slot][g][e] = at[KC ? (long)(g * 16 + e) : (g * 16 + e) * ld];
+                    if (g * 16 + e < mine) reg[slot][g][e] = at[g * 16 + e];
                 }
         }
-        at += step; left -= kShortRun * WAVES;
+        at += kShortRun * WAVES; mine -= kShortRun * WAVES;
+    }
+    __device__ __forceinline__ void place(int) {}
+    __device__ __forceinline__ void fetch(int slot, int g, float (&x)[8]) const
+    {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = reg[slot][g][e];
     }
 };
 
-template <bool A_KC, bool B_KC, int WAVES>
+template <bool A_KC, bool B_KC, int WAVES, bool TURN>
 __global__ __launch_bounds__(64 * WAVES) void short_gemm_kernel(GemmDev p)
 {
-    __shared__ f32x4 handed[WAVES - 1][4][64];   // the accumulators of the wavefronts behind the first
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lane32 = lane & 31, half = lane >> 5;
+    // a wavefront's tiles of its operands, 4 KiB each; the accumulators of those behind the first take their place
+    constexpr int kTiles = A_KC && B_KC ? 2 : 1;
+    __shared__ __attribute__((aligned(16))) float tiles[WAVES][kTiles][1024];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane32 = lane & 31, half = lane >> 5;
     const int nblocks = p.nbm * p.nbn, split = (int)blockIdx.x / nblocks, pid = (int)blockIdx.x - split * nblocks;
     const int m0 = pid % p.nbm * 32, n0 = pid / p.nbm * 32;
     const int k_begin = split * p.kchunk, k_end = (int)min((long)p.K, (long)k_begin + p.kchunk);
     f32x16 acc[1][1], small;   // the hi hi products; the others
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[0][0][r] = small[r] = 0.f;
-    ShortOperand<A_KC, WAVES> a;
-    ShortOperand<B_KC, WAVES> b;
+    ShortOperand<A_KC, WAVES, TURN> a;
+    ShortOperand<B_KC, WAVES, TURN> b;
     const int first = k_begin + wave * kShortRun;
-    a.init(p.A, p.lda, m0 + lane32, p.M, first + half * 8, k_end);
-    b.init(p.B, p.ldb, n0 + lane32, p.N, first + half * 8, k_end);
+    a.init(p.A, p.lda, m0, p.M, k_begin, k_end, wave * kShortRun, tiles[wave][0]);
+    b.init(p.B, p.ldb, n0, p.N, k_begin, k_end, wave * kShortRun, tiles[wave][kTiles - 1]);
     const int runs = first < k_end ? (k_end - first - 1) / (kShortRun * WAVES) + 1 : 0;
+    int left = k_end - first;
+    auto load = [&](int slot) {
+        a.load(slot, left); b.load(slot, left);
+        left -= kShortRun * WAVES;
+    };
     auto multiply = [&](int slot) {
+        a.place(slot); b.place(slot);
 #pragma unroll
         for (int g = 0; g < 2; ++g) {
             bf16x8 pa[3], pb[3];
-            split_eight(a.reg[slot][g], pa);
-            split_eight(b.reg[slot][g], pb);
+            float xa[8], xb[8];
+            a.fetch(slot, g, xa); b.fetch(slot, g, xb);
+            split_eight(xa, pa);
+            split_eight(xb, pb);
 #pragma unroll
             for (int q = 0; q < 5; ++q) small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pa[kSmallA[q]], pb[kSmallB[q]], small, 0, 0, 0);
             acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pa[0], pb[0], acc[0][0], 0, 0, 0);
         }
     };
-    if (runs > 0) { a.load(0); b.load(0); }
+    if (runs > 0) load(0);
     for (int r = 0; r < runs; r += 2) {
-        if (r + 1 < runs) { a.load(1); b.load(1); }
+        if (r + 1 < runs) load(1);
         multiply(0);
         if (r + 1 >= runs) break;
-        if (r + 2 < runs) { a.load(0); b.load(0); }
+        if (r + 2 < runs) load(0);
         multiply(1);
     }
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[0][0][r] += small[r];
     if (wave) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) handed[wave - 1][r][lane] = (f32x4){acc[0][0][r * 4], acc[0][0][r * 4 + 1], acc[0][0][r * 4 + 2], acc[0][0][r * 4 + 3]};
+        for (int r = 0; r < 4; ++r) *reinterpret_cast<f32x4 *>(&tiles[wave][0][(r * 64 + lane) * 4]) = (f32x4){acc[0][0][r * 4], acc[0][0][r * 4 + 1], acc[0][0][r * 4 + 2], acc[0][0][r * 4 + 3]};
     }
     __syncthreads();
     if (wave) return;
@@ -714,7 +827,7 @@ __global__ __launch_bounds__(64 * WAVES) void short_gemm_kernel(GemmDev p)
     for (int w = 0; w < WAVES - 1; ++w)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const f32x4 v = handed[w][r][lane];
+            const f32x4 v = *reinterpret_cast<const f32x4 *>(&tiles[w + 1][0][(r * 64 + lane) * 4]);
 #pragma unroll
             for (int e = 0; e < 4; ++e) acc[0][0][r * 4 + e] += v[e];
         }
@@ -733,10 +846,10 @@ template <int WAVES>
 void launch_short_waves(hipStream_t stream, const GemmDev &d, bool a_kc, bool b_kc, long nblocks)
 {
     const dim3 grid((unsigned)nblocks), group(64 * WAVES);
-    if (a_kc && b_kc) hipLaunchKernelGGL((short_gemm_kernel<true, true, WAVES>), grid, group, 0, stream, d);
-    else if (a_kc) hipLaunchKernelGGL((short_gemm_kernel<true, false, WAVES>), grid, group, 0, stream, d);
-    else if (b_kc) hipLaunchKernelGGL((short_gemm_kernel<false, true, WAVES>), grid, group, 0, stream, d);
-    else hipLaunchKernelGGL((short_gemm_kernel<false, false, WAVES>), grid, group, 0, stream, d);
+    if (a_kc && b_kc) hipLaunchKernelGGL((short_gemm_kernel<true, true, WAVES, true>), grid, group, 0, stream, d);
+    else if (a_kc) hipLaunchKernelGGL((short_gemm_kernel<true, false, WAVES, true>), grid, group, 0, stream, d);
+    else if (b_kc) hipLaunchKernelGGL((short_gemm_kernel<false, true, WAVES, true>), grid, group, 0, stream, d);
+    else hipLaunchKernelGGL((short_gemm_kernel<false, false, WAVES, true>), grid, group, 0, stream, d);
 }
 
 int launch_short(hipStream_t stream, GemmDev d, bool a_kc, bool b_kc)
@@ -749,6 +862,7 @@ int launch_short(hipStream_t stream, GemmDev d, bool a_kc, bool b_kc)
     // share one instead of the second waiting for the first.  us, eight -> four, 333 x 1201 (418 workgroups): k = 64 7.5 -> 5.7, 256
     // 9.5 -> 7.8, 1000 20.9 -> 18.2; up to one per compute unit: 10 x 1000, k = 1000 9.4 against 10.8.
     if (nblocks > kShortMost) launch_short_waves<4>(stream, d, a_kc, b_kc, nblocks);
+    else if (a_kc && b_kc && d.M <= kShortDirectRows) hipLaunchKernelGGL((short_gemm_kernel<true, true, 8, false>), dim3((unsigned)nblocks), dim3(64 * 8), 0, stream, d);
     else launch_short_waves<8>(stream, d, a_kc, b_kc, nblocks);
     MYEA_HIP_TRY(hipGetLastError());
     return MYEA_OK;
@@ -1119,7 +1233,7 @@ int launch_gemm(hipStream_t stream, const GemmParams &p)
     // 32; 640 x 768 (480) 5.6 -> 5.8, 8.3 -> 7.6, 21.6 -> 17.3, 75 -> 57; with a third workgroup a unit, 700 x 900 (638), 5.6 -> 7.5, 8.6 ->
     // 10.6, 22.4 -> 25.9, 76 -> 85.  (128 tiles exactly, 512 x 1024, would gain as well, 21.5 -> 17.7 at k = 1024, but are what a paired launch
     // takes as tiles, and a product has the same bits there and alone.)
-    if (tiles_64 * d.ksplit < 128) return launch_short(stream, d, a_kc, b_kc);
+    if (tiles_64 * d.ksplit < 128 && short_fits(d, a_kc, b_kc)) return launch_short(stream, d, a_kc, b_kc);
     if (tiles_128 * 2 * d.ksplit < 256) return launch_layout<64, 64>(stream, d, a_kc, b_kc);
     if (p.M <= p.N) return launch_layout<64, 128>(stream, d, a_kc, b_kc);
     return launch_layout<128, 64>(stream, d, a_kc, b_kc);
