@@ -1488,7 +1488,8 @@ __global__ __launch_bounds__(kBlock) void bn_backward_sequence_kernel(BnBackward
     {   // wavefront q finishes sum q: the scale's and the shift's shares of this time step go out, the two others to the second pass
         const double total = norm_sum_partials<CW, NP>(red[wave], lane);
         if (keeper) {
-            if (wave < 2) partial[(t * 2 + wave) * p.H + fj] = (float)total;
+            if (wave < 2 && partial) partial[(t * 2 + wave) * p.H + fj] = (float)total;
+            else if (wave < 2) (wave ? p.dshift : p.dscale)[fj] += (float)total;   // a single time step
             else s_d[wave - 2][fc] = (float)total;
         }
     }
@@ -1571,6 +1572,7 @@ int launch_bn_backward_sequence(hipStream_t s, const BnBackwardParams &p, size_t
 {
     if (p.H == 0 || p.rows == 0 || T == 0) return MYEA_OK;
     if (p.rows > Bmax || T > 65535) { set_last_error("bn_backward_sequence: %zu rows of %zu, %zu time steps", p.rows, Bmax, T); return MYEA_E_INVALID; }
+    if (!scratch && (T != 1 || fold_now)) { set_last_error("bn_backward_sequence: no room for the shares of %zu time steps", T); return MYEA_E_INVALID; }
     const int cw = sequence_columns(p.H, T);
     const size_t blocks = (p.H + cw - 1) / cw;
     if (cw == 4) hipLaunchKernelGGL(bn_backward_sequence_kernel<4>, dim3((unsigned)blocks, (unsigned)T), dim3(kBlock), 0, s, p, Bmax, scratch);

@@ -530,6 +530,13 @@ static bool bn_sequence_allowed()
     return on;
 }
 
+// A single time step through the same launch instead of three (column sums, their finish, the rows): a workgroup owns four columns of all
+// rows, which pays while the rows are few and the launches are what counts.  us for four steps of three residual blocks (7 normalisations
+// a pass, activations in the same launch on both sides), three launches -> one: 128 units x 32 examples 1025 -> 797; 512 x 128 1568 -> 1262;
+// 1024 x 256 2464 -> 2250; 1000 x 333 3017 -> 2813; 1024 x 512 3248 -> 3194; 2048 x 256 6258 -> 6217; beyond the lines 128 x 1024 1446 ->
+// 1555; 1500 x 700 6356 -> 6498; 2048 x 1024 9190 -> 10255.
+static bool bn_in_one_launch(size_t rows, size_t H) { return rows <= 512 && rows * H <= (size_t)1 << 19; }
+
 int Net::forward_fc_layer(size_t li, size_t B)
 {
     const myea_layer_desc &l = d.layers[li];
@@ -658,7 +665,7 @@ int Net::bn_forward_all(size_t li, size_t B, const float *x, bool training, floa
     const myea_layer_desc &l = d.layers[li];
     DevLayer &o = L[li];
     const size_t T = d.number_recurrent_depth, Bmax = d.batch_size, H = o.NH;
-    if (T == 1 || !bn_sequence_allowed() || 2 * T * H > scratch_floats) {
+    if ((T == 1 && !bn_in_one_launch(B, H)) || !bn_sequence_allowed() || 2 * T * H > scratch_floats) {
         for (size_t t = 0; t < T; ++t)
             MYEA_TRY(bn_forward(li, t, B, x + t * Bmax * H, training, act_out ? act_out + t * Bmax * H : nullptr, colscale ? colscale + t * H : nullptr));
         return MYEA_OK;
@@ -684,7 +691,8 @@ int Net::bn_backward_all(size_t li, size_t B, const float *x, const float *dy, f
     const myea_layer_desc &l = d.layers[li];
     DevLayer &o = L[li];
     const size_t T = d.number_recurrent_depth, Bmax = d.batch_size, H = o.NH;
-    if (T == 1 || !bn_sequence_allowed() || 2 * T * H > scratch_floats || bn_share_at[li] == SIZE_MAX) {
+    const bool alone = T == 1 && bn_in_one_launch(B, H);
+    if ((!alone && (T == 1 || bn_share_at[li] == SIZE_MAX)) || !bn_sequence_allowed() || 2 * T * H > scratch_floats) {
         for (size_t t = T; t-- > 0;) MYEA_TRY(bn_backward(li, t, B, x + t * Bmax * H, dy + t * Bmax * H, dx + t * Bmax * H));
         return MYEA_OK;
     }
@@ -695,11 +703,12 @@ int Net::bn_backward_all(size_t li, size_t B, const float *x, const float *dy, f
     p.dx = dx;
     p.renorm = l.type_normalization == MYEA_NORMALIZATION_BATCH_RENORMALIZATION;
     prof_begin(kProfNormalization);
-    // the shares of the scale's and the shift's gradient stay in the layer's slice until the end of the pass: flush_bn_shares
-    float *shares = bn_shares + bn_share_at[li];
+    // the shares of the scale's and the shift's gradient stay in the layer's slice until the end of the pass: flush_bn_shares (a single
+    // time step's go straight onto the gradient)
+    float *shares = alone ? nullptr : bn_shares + bn_share_at[li];
     const int rc = launch_bn_backward_sequence(stream, p, T, Bmax, shares, false);
     prof_end((double)T * (double)B * (double)H * sizeof(float) * 3.0);
-    if (rc == MYEA_OK) bn_jobs_pending.push_back(BnFoldJob{shares, p.dscale, p.dshift, (unsigned)H, (unsigned)T});
+    if (rc == MYEA_OK && shares) bn_jobs_pending.push_back(BnFoldJob{shares, p.dscale, p.dshift, (unsigned)H, (unsigned)T});
     return rc;
 }
 
@@ -904,7 +913,11 @@ int Net::forward_residual_block(size_t ri, size_t B)
         bool drop = false;
         if (o.group == 2) MYEA_TRY(refresh_colscale(m, &drop));
         const bool norm = layer_uses_norm(l), ind = o.group == 2 && layer_is_ind_rnn(l);
-        if (norm) MYEA_TRY(bn_forward_all(m, B, x, training));
+        if (norm) {   // training: the activation (and the dropout multiplier) of a member rides in the normalisation's last pass
+            const bool af_in_bn = o.group == 2 && !ind && training && !o.unit_act;
+            MYEA_TRY(bn_forward_all(m, B, x, training, af_in_bn ? o.values : nullptr, af_in_bn && drop ? o.colscale : nullptr));
+            values_ready = values_ready || af_in_bn;
+        }
         const float *in = norm ? o.normalizes : x;
         if (ind) {   // the recurrence and the activation over the whole sequence; Bernoulli dropout in place on what the next step reads
             IndRnnParams p{};
