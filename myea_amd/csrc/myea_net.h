@@ -115,6 +115,10 @@ struct Net {
     std::vector<size_t> narrow_slab_at;        // per layer, SIZE_MAX without a slice
     SlabFoldJob *fold_jobs = nullptr, *fold_jobs_staging = nullptr;   // device; pinned host
     std::vector<SlabFoldJob> fold_pending, fold_uploaded;
+    // ... and the contractions that write those slabs are one launch too, in front of it
+    NarrowDwJob *narrow_jobs = nullptr, *narrow_jobs_staging = nullptr;   // device; pinned host
+    std::vector<NarrowDwJob> narrow_pending, narrow_uploaded;
+    double narrow_work = 0;
     int flush_slab_folds();
     // the bounds of the independently recurrent layers' self weights, clipped behind every update in one launch; built at the first update
     ClipRange *clip_ranges = nullptr;

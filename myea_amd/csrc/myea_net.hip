@@ -437,6 +437,10 @@ int Net::create(const myea_net_desc &desc)
             fold_jobs = static_cast<SlabFoldJob *>(q);
             MYEA_HIP_TRY(hipHostMalloc(&q, count * sizeof(SlabFoldJob), hipHostMallocDefault));
             fold_jobs_staging = static_cast<SlabFoldJob *>(q);
+            MYEA_HIP_TRY(hipMalloc(&q, count * sizeof(NarrowDwJob)));
+            narrow_jobs = static_cast<NarrowDwJob *>(q);
+            MYEA_HIP_TRY(hipHostMalloc(&q, count * sizeof(NarrowDwJob), hipHostMallocDefault));
+            narrow_jobs_staging = static_cast<NarrowDwJob *>(q);
         }
     }
     MYEA_TRY(static_scratch_address(&static_scratch));   // set-up: this device's address of the static array
@@ -478,7 +482,8 @@ Net::~Net()
     fr(planes_sync); fr(planes_exchange); fr(planes_shares);
     fr(gemm_pair_partials); fr(gemm_pair_tickets); fr(fault);
     if (resident_flag) (void)hipHostFree(resident_flag);
-    fr(bn_shares); fr(bn_jobs); fr(narrow_slabs); fr(fold_jobs); fr(clip_ranges);
+    fr(bn_shares); fr(bn_jobs); fr(narrow_slabs); fr(fold_jobs); fr(narrow_jobs); fr(clip_ranges);
+    if (narrow_jobs_staging) (void)hipHostFree(narrow_jobs_staging);
     if (fold_jobs_staging) (void)hipHostFree(fold_jobs_staging);
     if (bn_jobs_staging) (void)hipHostFree(bn_jobs_staging);
     fr(tmp1); fr(tmp2); fr(scratch); fr(stage_in); fr(stage_out); fr(loss_acc); fr(index_stage); fr(dw_slabs);
@@ -712,20 +717,40 @@ int Net::bn_backward_all(size_t li, size_t B, const float *x, const float *dy, f
     return rc;
 }
 
+// A launch's table onto the device, unless what lies there is the same: the first call, or one over other layers or buffers than the last,
+// uploads it again.
+template <class Job>
+static int upload_jobs(hipStream_t stream, const std::vector<Job> &pending, std::vector<Job> *uploaded, Job *staging, Job *jobs)
+{
+    const size_t count = pending.size();
+    bool same = uploaded->size() == count;
+    for (size_t i = 0; same && i < count; ++i) same = std::memcmp(&pending[i], &(*uploaded)[i], sizeof(Job)) == 0;
+    if (same) return MYEA_OK;
+    MYEA_HIP_TRY(hipStreamSynchronize(stream));   // no earlier launch still reads the table
+    std::memcpy(staging, pending.data(), count * sizeof(Job));
+    MYEA_HIP_TRY(hipMemcpyAsync(jobs, staging, count * sizeof(Job), hipMemcpyHostToDevice, stream));
+    MYEA_HIP_TRY(hipStreamSynchronize(stream));   // the staging words are free again
+    *uploaded = pending;
+    return MYEA_OK;
+}
+
 // The slabs the narrow layers' weight gradients of this call left are added onto the gradient: one launch for all layers.
 int Net::flush_slab_folds()
 {
     if (fold_pending.empty()) return MYEA_OK;
-    const size_t count = fold_pending.size();
-    bool same = fold_uploaded.size() == count;
-    for (size_t i = 0; same && i < count; ++i) same = std::memcmp(&fold_pending[i], &fold_uploaded[i], sizeof(SlabFoldJob)) == 0;
-    if (!same) {   // the first call, or one over other layers or buffers than the last: the table goes up again
-        MYEA_HIP_TRY(hipStreamSynchronize(stream));   // no earlier launch still reads the table
-        std::memcpy(fold_jobs_staging, fold_pending.data(), count * sizeof(SlabFoldJob));
-        MYEA_HIP_TRY(hipMemcpyAsync(fold_jobs, fold_jobs_staging, count * sizeof(SlabFoldJob), hipMemcpyHostToDevice, stream));
-        MYEA_HIP_TRY(hipStreamSynchronize(stream));   // the staging words are free again
-        fold_uploaded = fold_pending;
+    if (!narrow_pending.empty()) {
+        MYEA_TRY(upload_jobs(stream, narrow_pending, &narrow_uploaded, narrow_jobs_staging, narrow_jobs));
+        unsigned most = 0;
+        for (const NarrowDwJob &j : narrow_pending) most = std::max(most, j.slab_count);
+        const size_t layers = narrow_pending.size();
+        narrow_pending.clear();
+        prof_begin(2);
+        MYEA_TRY(launch_narrow_dw_jobs(stream, narrow_jobs, layers, most));
+        prof_end(narrow_work);
+        narrow_work = 0;
     }
+    const size_t count = fold_pending.size();
+    MYEA_TRY(upload_jobs(stream, fold_pending, &fold_uploaded, fold_jobs_staging, fold_jobs));
     size_t widest = 0;
     for (const SlabFoldJob &j : fold_pending) widest = std::max(widest, (size_t)j.n);
     fold_pending.clear();
@@ -740,15 +765,7 @@ int Net::flush_bn_shares()
 {
     if (bn_jobs_pending.empty()) return MYEA_OK;
     const size_t count = bn_jobs_pending.size();
-    bool same = bn_jobs_uploaded.size() == count;
-    for (size_t i = 0; same && i < count; ++i) same = std::memcmp(&bn_jobs_pending[i], &bn_jobs_uploaded[i], sizeof(BnFoldJob)) == 0;
-    if (!same) {   // the first pass, or one over other layers than the last (another batch size): the table goes up again
-        MYEA_HIP_TRY(hipStreamSynchronize(stream));   // no earlier launch still reads the table
-        std::memcpy(bn_jobs_staging, bn_jobs_pending.data(), count * sizeof(BnFoldJob));
-        MYEA_HIP_TRY(hipMemcpyAsync(bn_jobs, bn_jobs_staging, count * sizeof(BnFoldJob), hipMemcpyHostToDevice, stream));
-        MYEA_HIP_TRY(hipStreamSynchronize(stream));   // the staging words are free again
-        bn_jobs_uploaded = bn_jobs_pending;
-    }
+    MYEA_TRY(upload_jobs(stream, bn_jobs_pending, &bn_jobs_uploaded, bn_jobs_staging, bn_jobs));
     size_t widest = 0;
     for (const BnFoldJob &j : bn_jobs_pending) widest = std::max(widest, (size_t)j.H);
     bn_jobs_pending.clear();
@@ -1548,10 +1565,16 @@ int Net::update_derivative_weight_contraction(size_t li, size_t B)
         // a narrow layer over all of its rows: the slabs wait in the layer's slice for the one launch that adds every layer's
         const bool later = defer_folds && narrow > 0 && chunks == 1 && narrow_slabs && narrow_slab_at[li] != SIZE_MAX;
         float *const slabs_at = later ? narrow_slabs + narrow_slab_at[li] : dw_slabs;
+        if (later) {   // with the other narrow layers' in one launch: flush_slab_folds
+            prof_cancel();
+            narrow_pending.push_back(narrow_dw_job(g.A, g.B, slabs_at, H, In, rows));
+            narrow_work += 2.0 * (double)rows * (double)H * (double)In;
+            fold_pending.push_back(SlabFoldJob{slabs_at, gradient + l.first_connection_index, (unsigned)(H * In), (unsigned)narrow});
+            continue;
+        }
         if (narrow > 0) { slabs = narrow; MYEA_TRY(launch_narrow_dw(stream, g.A, g.B, slabs_at, H, In, rows)); }
         else MYEA_TRY(launch_gemm(stream, g));
-        if (later) fold_pending.push_back(SlabFoldJob{slabs_at, gradient + l.first_connection_index, (unsigned)(H * In), (unsigned)slabs});
-        else if (slabs > 1 || narrow > 0) MYEA_TRY(launch_slab_sum_add(stream, H * In, slabs, dw_slabs, gradient + l.first_connection_index, narrow > 0));
+        if (slabs > 1 || narrow > 0) MYEA_TRY(launch_slab_sum_add(stream, H * In, slabs, dw_slabs, gradient + l.first_connection_index, narrow > 0));
         prof_end(2.0 * (double)rows * (double)H * (double)In);
     }
 
@@ -1582,6 +1605,7 @@ int Net::update_derivative_weight(size_t B, size_t first, size_t end)
     const bool per_t = T > 1 && B != Bmax;
     const size_t chunks = per_t ? T : 1, rows = per_t ? B : (T > 1 ? T * B : B);
     fold_pending.clear();
+    narrow_pending.clear(); narrow_work = 0;
     // The column reductions (biases, LSTM peepholes, self weights of independently recurrent layers) read deltas that
     // are complete before this call and write gradient slots no contraction touches; slots shared between layers (the
     // LSTM bias addressing reaches into the next layers' biases) are added to in the layers' order, on one stream.
@@ -1613,23 +1637,10 @@ int Net::update_derivative_weight(size_t B, size_t first, size_t end)
         }
         return MYEA_OK;
     };
-    // alternate: narrow layers, whose slabs wait in slices of their own, take turns on the two streams - each is a launch of a few
-    // dozen workgroups and a chain of them on one stream leaves most of the device idle
-    auto contractions = [&](bool alternate) -> int {
-        bool on_side = false;
+    auto contractions = [&]() -> int {
         for (size_t li = first; li < end; ++li) {
             const bool done_before = li < dw_done.size() && dw_done[li];
-            const bool own_slice = alternate && !done_before && chunks == 1 && defer_folds && narrow_slabs && li < narrow_slab_at.size() &&
-                                   narrow_slab_at[li] != SIZE_MAX && layer_is_dense(d.layers[li]) && narrow_dw_slabs(L[li].H, L[li].In, rows) > 0;
-            if (own_slice && on_side) {
-                std::swap(stream, side_stream);
-                const int rc = update_derivative_weight_contraction(li, B);
-                std::swap(stream, side_stream);
-                MYEA_TRY(rc);
-            } else {
-                MYEA_TRY(update_derivative_weight_contraction(li, B));
-            }
-            if (own_slice) on_side = !on_side;
+            MYEA_TRY(update_derivative_weight_contraction(li, B));
             // the combined call: every delta has been handed down by now, so the layer's weights may take their step beside the
             // contractions of the layers that follow
             if (early_update && !done_before) MYEA_TRY(early_update_layer(li));
@@ -1641,17 +1652,17 @@ int Net::update_derivative_weight(size_t B, size_t first, size_t end)
     if (any_lstm || !side_stream) {
         // beside the split-K contractions of LSTM layers the long reductions over T x batch rows were measured to cost
         // more than they hide: one stream, contractions first
-        MYEA_TRY(contractions(false));
+        MYEA_TRY(contractions());
         MYEA_TRY(reductions());
         return flush_slab_folds();
     }
-    // memory-bound reductions on the side stream beside the matrix-pipe-bound contractions, and every other narrow contraction
+    // memory-bound reductions on the side stream beside the matrix-pipe-bound contractions
     MYEA_HIP_TRY(hipEventRecord(fork_event, stream));
     MYEA_HIP_TRY(hipStreamWaitEvent(side_stream, fork_event, 0));
     std::swap(stream, side_stream);
     int rc = reductions();
     std::swap(stream, side_stream);
-    if (rc == MYEA_OK) rc = contractions(true);
+    if (rc == MYEA_OK) rc = contractions();
     const hipError_t e = hipEventRecord(join_event, side_stream);   // the main stream goes on behind the side stream, whatever else happened
     const int joined = e == hipSuccess ? side_stream_join() : MYEA_E_DEVICE;
     if (e != hipSuccess && rc == MYEA_OK) set_last_error("hipEventRecord: %s", hipGetErrorString(e));
