@@ -1045,7 +1045,7 @@ __global__ __launch_bounds__(64 * kNarrowWaves) void narrow_dw_kernel(const floa
 }
 
 // The same for a table of layers, grid (most slabs of one, layers): as launches of their own they were 5.6 us each, a few dozen workgroups
-// at a time (29 layers of at most 32 x 32 over 7168 rows: 162 us in turns on two streams, 11 us here).
+// at a time (29 layers of at most 32 x 32 over 7168 rows: 161 us of launches in turns on two streams, 15 us here).
 __global__ __launch_bounds__(64 * kNarrowWaves) void narrow_dw_jobs_kernel(const NarrowDwJob *__restrict__ jobs)
 {
     const NarrowDwJob job = jobs[blockIdx.y];

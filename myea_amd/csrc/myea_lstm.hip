@@ -49,7 +49,7 @@ struct LstmLayer {
     float *dG = nullptr;    // [T][Bmax][G] deltas dz | di | df | do
     float *dc = nullptr;    // [T][Bmax][C]
     float *part = nullptr;  // split-K slabs of the per-step recurrent contractions, 16 x [Bmax][G]
-    // [ceil(Bmax / 32)][7][C]: what the resident backward loop sums of its gate deltas as it goes (bias and peephole gradients
+    // [ceil(Bmax / 16)][7][C]: what the resident backward loop sums of its gate deltas as it goes (bias and peephole gradients
     // per group of examples); sums_groups > 0 while they belong to the deltas in dG, of a pass over sums_batch examples
     float *sums = nullptr;
     size_t sums_groups = 0, sums_batch = 0;

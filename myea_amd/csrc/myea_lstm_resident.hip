@@ -8,7 +8,7 @@
 // the previous step produced for the SAME examples: workgroups that own different examples never talk.
 //
 // Shape of the work (one cell per block, C cells, gate rows z | i | f | o of the packed matrices):
-//   * a workgroup owns CELLS cells (16, or 8 when C > 512).  Forward: the 4 CELLS gate columns of those cells, its four wavefronts split
+//   * a workgroup owns CELLS = 16 cells.  Forward: the 4 CELLS gate columns of those cells, its four wavefronts split
 //     k = C into contiguous quarters; backward: the CELLS columns of dh, wavefront w takes the k range of gate w.  Either
 //     way a wavefront holds its [columns][k range] slice of Wrec (WrecT) in registers for the whole launch (at most 128
 //     registers per lane) in the operand layout of v_mfma_f32_16x16x4_f32;
@@ -34,7 +34,7 @@
 //     checks that with a probe launch once per process, and in every launch the members of a group compare their XCC
 //     ids).  The XCD's L2 is then the point of coherence: plain stores, a counter bumped by an atomic performed in L2 and
 //     polled with loads that bypass the compute unit's L1 (sc1), as do the loads of the exchanged tensor;
-//   * AGENT (groups wider than an XCD, C = 1024, forward only): device-scope stores of h, device-scope counter, sc1 loads.
+//   * AGENT (groups wider than an XCD, C = 1024): device-scope stores of h, device-scope counter, sc1 loads.
 // A wavefront arrives once its own stores are complete (vmcnt(0)); the last of the four - counted in LDS - bumps the
 // chain's counter.  A wait is bounded: after `spin_polls` polls the waiting wavefront raises the give-up flag, every
 // wavefront sees it at its next poll and leaves, the kernel ends normally and the host reports MYEA_E_DEVICE.
@@ -251,7 +251,7 @@ namespace {
 using Chain0 = std::integral_constant<int, 0>;
 using Chain1 = std::integral_constant<int, 1>;
 
-template <int KW, int CELLS, int RS, bool AGENT>
+template <int KW, int CELLS, int RS>
 __global__ __launch_bounds__(kThreads, 1) void lstm_resident_forward_kernel(ResidentGeometry g, LstmResidentDir d0, LstmResidentDir d1, SyncWords w)
 {
     constexpr int C = 4 * KW, G = 4 * C;
@@ -259,17 +259,13 @@ __global__ __launch_bounds__(kThreads, 1) void lstm_resident_forward_kernel(Resi
     constexpr int LPT = ROWS / 8;                 // direct loads per tile
     constexpr int PAIRS = ROWS * CELLS / kThreads;
     constexpr int NSTORE = 7 * PAIRS;             // stores of a unit
-    constexpr int A1 = NT >= 4 ? NT / 4 : 1;      // tiles whose MFMAs run before the previous unit's arrival is signalled
-    constexpr int P1 = NT >= 4 ? (3 * NT) / 4 : NT - 1;   // tile before which the next unit's counter is read
+    constexpr int A1 = NT / 4;      // tiles whose MFMAs run before the previous unit's arrival is signalled
     constexpr int kStride = NB + 8;               // floats per row of a wavefront's partial tile
-    constexpr bool HALF = !AGENT && NT == 4 && RS == 1;   // 512 cells: a unit's four tiles are requested in two halves, each two tiles of MFMAs ahead
-    constexpr int SLOTS = NT;
-    constexpr int kAhead = HALF ? NT / 2 : NT;    // tiles of a unit that the other chain requests for it
-    constexpr int kStage = SLOTS * ROWS * 32, kPart = 4 * ROWS * kStride;
-    constexpr int kAux = AGENT ? 16 : kLocalAux;
-    constexpr bool DB = AGENT;                    // the other chain's tiles are requested during this chain's last MFMAs, into the slots those have left
-    constexpr int S1 = (5 * NT) / 8, X1 = (3 * NT) / 4;   // DB: tile behind which the other chain's counter is read / behind which its value is looked at
-    static_assert(!DB || (NT >= 8 && X1 > S1 && X1 < NT && X1 % (NT - X1) == 0), "tiles left to spread the requests over");
+    constexpr int kStage = NT * ROWS * 32, kPart = 4 * ROWS * kStride;
+    constexpr int kAux = 16;
+    // the other chain's tiles are requested during this chain's last MFMAs, into the slots those have left
+    constexpr int S1 = (5 * NT) / 8, X1 = (3 * NT) / 4;   // tile behind which the other chain's counter is read / behind which its value is looked at
+    static_assert(NT >= 8 && X1 > S1 && X1 < NT && X1 % (NT - X1) == 0, "tiles left to spread the requests over");
     static_assert(PAIRS >= 1 && ROWS * CELLS % kThreads == 0, "every lane has the same number of pairs");
     static_assert(NT * LPT + NSTORE < 64, "vmcnt has 6 bits");
     extern __shared__ __attribute__((aligned(16))) float smem[];
@@ -277,14 +273,13 @@ __global__ __launch_bounds__(kThreads, 1) void lstm_resident_forward_kernel(Resi
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col16 = lane & 15, quad = lane >> 4;
 
     int group, member;
-    if (!place<AGENT>(blockIdx.x, g.members, g.dirs * g.row_groups, group, member)) return;
+    if (!place<true>(blockIdx.x, g.members, g.dirs * g.row_groups, group, member)) return;
     const int dir = group % g.dirs, rg = group / g.dirs;
     const LstmResidentDir &d = dir ? d1 : d0;
     const int c0 = member * CELLS, B = g.B, T = g.T;
     const size_t Bmax = (size_t)g.Bmax;
     unsigned *const counters = w.counters + (size_t)group * 2 * kSyncStride;   // chain c: counters + c * kSyncStride
     const unsigned members = (unsigned)g.arrivals;
-    if (!AGENT) check_same_xcd(w, group);
     if (threadIdx.x < 2) s_arrive[threadIdx.x] = 0u;
     __syncthreads();
 
@@ -386,17 +381,17 @@ __global__ __launch_bounds__(kThreads, 1) void lstm_resident_forward_kernel(Resi
 #pragma unroll
             for (int q = 0; q < LPT; ++q)
                 __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(p_tile[c][q] + i * 32),
-                                                 (__attribute__((address_space(3))) void *)(stage + (i % SLOTS) * ROWS * 32 + q * 256), 16, 0, kAux);
+                                                 (__attribute__((address_space(3))) void *)(stage + i * ROWS * 32 + q * 256), 16, 0, kAux);
         if (decltype(advance)::value) {
 #pragma unroll
             for (int q = 0; q < LPT; ++q) p_tile[c][q] += step_c;
         }
     };
-    auto load_tiles = [&](auto ch) { load_tile_range(ch, std::integral_constant<int, 0>{}, std::integral_constant<int, kAhead>{}, std::integral_constant<bool, !HALF>{}); };
+    auto load_tiles = [&](auto ch) { load_tile_range(ch, std::integral_constant<int, 0>{}, std::integral_constant<int, NT>{}, std::true_type{}); };
     auto mfma_tiles = [&](auto ch, auto first, auto last) {
 #pragma unroll
         for (int i = decltype(first)::value; i < decltype(last)::value; ++i) {
-            const float *tile = stage + (i % SLOTS) * ROWS * 32;
+            const float *tile = stage + i * ROWS * 32;
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 f32x4 fa[RS];
@@ -414,7 +409,6 @@ __global__ __launch_bounds__(kThreads, 1) void lstm_resident_forward_kernel(Resi
     };
     using I0 = std::integral_constant<int, 0>;
     using IA = std::integral_constant<int, A1>;
-    using IP = std::integral_constant<int, (P1 > A1 ? P1 : A1)>;
     using IN = std::integral_constant<int, NT>;
 
     // The first part of a unit with a recurrent term: its tiles have landed when only the previous unit's stores can be
@@ -427,21 +421,10 @@ __global__ __launch_bounds__(kThreads, 1) void lstm_resident_forward_kernel(Resi
 #pragma unroll
             for (int ct = 0; ct < NCT; ++ct) acc[rs][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
         if (decltype(all_landed)::value) wait_vm<0>(); else wait_vm<NSTORE>();
-        if constexpr (HALF) {   // the unit's second half: the third tile now, the fourth behind the first tile's MFMAs - two tiles of MFMAs ahead each
-            __builtin_amdgcn_sched_barrier(0);
-            load_tile_range(ch, std::integral_constant<int, 2>{}, std::integral_constant<int, 3>{}, std::false_type{});
-            __builtin_amdgcn_sched_barrier(0);
-        }
         mfma_tiles(ch, I0{}, IA{});
         __builtin_amdgcn_sched_barrier(0);   // keeps the MFMAs above in front of the wait
-        if constexpr (HALF) {   // the stores of the unit before are older than the two requests
-            load_tile_range(ch, std::integral_constant<int, 3>{}, IN{}, std::true_type{});
-            __builtin_amdgcn_sched_barrier(0);
-            wait_vm<2 * LPT>();
-        } else {
-            wait_vm<0>();
-        }
-        wave_arrive<AGENT>(counters + (1 - c) * kSyncStride, &s_arrive[1 - c]);
+        wait_vm<0>();
+        wave_arrive<true>(counters + (1 - c) * kSyncStride, &s_arrive[1 - c]);
     };
     // The rest of the unit.  FIRST: the chain's first step (no recurrent term, no forget gate, no peephole into the input
     // gate).  wait_for: the other chain's units that must have arrived before its next unit's tiles are requested (0: that
@@ -451,43 +434,7 @@ __global__ __launch_bounds__(kThreads, 1) void lstm_resident_forward_kernel(Resi
         constexpr bool FIRST = decltype(first_tag)::value;
         load_inputs(ch);
         bool requested = false;   // the other chain's tiles are on their way already
-        if constexpr (!FIRST && HALF) {
-            // A unit's four tiles are requested two at a time (its first two behind the last two MFMA tiles of the unit before, if
-            // the chain's counter is complete by then; the third and the fourth in the unit's head, around its first tile's
-            // MFMAs), so a wavefront never issues more than two loads in a row - eight in a row, four wavefronts at once, keep
-            // the compute unit's address path busy for 512 clocks during which the issuing wavefronts stand still - and every tile
-            // has two tiles of MFMAs to arrive (with one, the wait for it cost 500 clocks a tile).  The first wait counts what
-            // was issued behind the tile it waits for: the fourth tile, the counter, and the unit's inputs, counted as four loads,
-            // the fewest there can be (two more with zoneout masks: it then asks for a little more than it needs).  The second leaves nothing in flight - the inputs too, requested two
-            // tiles of MFMAs ago - so that the compiler has no load left to wait for in front of the gate math: it would
-            // wait for everything there, the next unit's tiles included.
-            constexpr int kIn = 4 * PAIRS;
-            using I1 = std::integral_constant<int, 1>;
-            using I2 = std::integral_constant<int, 2>;
-            using I3 = std::integral_constant<int, 3>;
-            using Other = std::integral_constant<int, 1 - c>;
-            __builtin_amdgcn_sched_barrier(0);
-            mfma_tiles(ch, I1{}, I2{});
-            __builtin_amdgcn_sched_barrier(0);
-            asm volatile("global_load_dword %0, %1, off sc1" : "=v"(seen) : "v"(counters + (1 - c) * kSyncStride) : "memory");
-            __builtin_amdgcn_sched_barrier(0);
-            wait_vm<LPT + 1 + kIn>();              // the third tile has landed: behind it came the inputs, the fourth tile, the counter
-            mfma_tiles(ch, I2{}, I3{});
-            __builtin_amdgcn_sched_barrier(0);
-            wait_vm<0>();                          // the fourth, the counter's value, the inputs
-            asm volatile("" : "+v"(seen));         // looked at behind the wait, not before
-            if (wait_for && !g.never_early && (int)(__builtin_amdgcn_readfirstlane(seen) - wait_for * members) >= 0) {
-                load_tile_range(Other{}, I0{}, I1{}, std::false_type{});
-                __builtin_amdgcn_sched_barrier(0);
-                mfma_tiles(ch, I3{}, IN{});
-                __builtin_amdgcn_sched_barrier(0);
-                load_tile_range(Other{}, I1{}, I2{}, std::false_type{});
-                requested = true;
-            } else {
-                mfma_tiles(ch, I3{}, IN{});
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        } else if constexpr (!FIRST && DB) {
+        if constexpr (!FIRST) {
             // The other chain's counter is read five eighths into the MFMAs, when its step is normally complete, and looked at an
             // eighth later; its tiles are then requested between the last quarter's MFMAs, into the slots whose tiles those
             // MFMAs no longer need (a tile's own slot right behind its MFMAs) - they have those MFMAs and the gate math to
@@ -519,16 +466,9 @@ __global__ __launch_bounds__(kThreads, 1) void lstm_resident_forward_kernel(Resi
                 mfma_tiles(ch, IX{}, IN{});
             }
             __builtin_amdgcn_sched_barrier(0);
-        } else if (!FIRST) {
-            mfma_tiles(ch, IA{}, IP{});
-            if (wait_for) seen = __hip_atomic_load(counters + (1 - c) * kSyncStride, __ATOMIC_RELAXED, MYEA_SCOPE_AGENT);
-            mfma_tiles(ch, IP{}, IN{});
-            __builtin_amdgcn_sched_barrier(0);   // the counter's value is looked at after the MFMAs, not right behind its load
         }
         if (wait_for && !requested) {
-            const unsigned target = wait_for * members;
-            const bool there = !FIRST && !DB && !HALF && (int)(__builtin_amdgcn_readfirstlane(seen) - target) >= 0;
-            if (!there && !wave_wait(w, counters + (1 - c) * kSyncStride, target, g.spin_polls)) return false;
+            if (!wave_wait(w, counters + (1 - c) * kSyncStride, wait_for * members, g.spin_polls)) return false;
             load_tiles(std::integral_constant<int, 1 - c>{});   // every wavefront's reads of this unit's tiles have been issued and waited for by its MFMAs
         }
         float *part = parts + c * kPart;
@@ -574,8 +514,7 @@ __global__ __launch_bounds__(kThreads, 1) void lstm_resident_forward_kernel(Resi
             float hv = a * go;
             hv = keep_h[q] ? hv : h_prev[c][q];
             c_prev[c][q] = cs; h_prev[c][q] = hv;
-            if (AGENT) __hip_atomic_store(p_h[c][q], hv, __ATOMIC_RELAXED, MYEA_SCOPE_AGENT);
-            else *p_h[c][q] = hv;
+            __hip_atomic_store(p_h[c][q], hv, __ATOMIC_RELAXED, MYEA_SCOPE_AGENT);   // read by members on another XCD
             float *arow = p_acts_out[c][q];
             arow[0] = z; arow[C] = gi; arow[2 * C] = gf; arow[3 * C] = go;
             *p_c[c][q] = cs; *p_ca[c][q] = a;
@@ -594,7 +533,7 @@ __global__ __launch_bounds__(kThreads, 1) void lstm_resident_forward_kernel(Resi
     // units in program order: (0,0) (1,0) (0,1) (1,1) ... ; unit (c, s) needs every member's h of unit (c, s - 1)
     if (!tail(Chain0{}, First{}, 0u)) return;
     wait_vm<0>();
-    wave_arrive<AGENT>(counters, &s_arrive[0]);          // unit (0, 0)
+    wave_arrive<true>(counters, &s_arrive[0]);          // unit (0, 0)
     if (!tail(Chain1{}, First{}, 1u)) return;            // requests the tiles of unit (0, 1)
     head(Chain0{}, std::true_type{});                    // signals unit (1, 0)
     for (int s = 1; s + 1 < T; ++s) {
@@ -1404,11 +1343,11 @@ struct KernelInfo {
     int per_cu = 0;   // workgroups of this kernel a compute unit can hold
 };
 
-template <int KW, int CELLS, int RS, bool AGENT>
+template <int KW, int CELLS, int RS>
 KernelInfo forward_info()
 {
     KernelInfo k;
-    k.fn = lstm_resident_forward_kernel<KW, CELLS, RS, AGENT>;
+    k.fn = lstm_resident_forward_kernel<KW, CELLS, RS>;
     k.lds = forward_lds(KW, CELLS, RS);
     k.cells = CELLS;
     return k;
@@ -1437,7 +1376,7 @@ KernelInfo sets_info()
 // What the loops of myea_lstm_planes.hip leave to these: both passes at 1024 cells, whose members span two XCDs, and the backward pass at
 // 512 cells and more than one row of 16 examples a group (256 examples, 64 time steps: 454 us here, 619 there; up to 128 examples 460
 // here, 237 there).
-KernelInfo g_forward_1024 = forward_info<256, 16, 1, true>();
+KernelInfo g_forward_1024 = forward_info<256, 16, 1>();
 KernelInfo g_backward_512 = backward_info<512, 1>(), g_backward_1024 = backward_info<1024, 1>();
 // the 512-cell backward loop with one chain per set of four wavefronts
 KernelInfo g_sets_512 = sets_info<512>();

@@ -1591,9 +1591,9 @@ bool Net::dw_beside_loop_allowed(size_t gi, size_t li, size_t B)
     if (off || !side_stream || d.number_recurrent_depth < 2 || B != d.batch_size) return false;
     if (L[li].lstm2 || L[gi].lstm2 || (gi < dw_done.size() && dw_done[gi])) return false;
     if (d.layers[gi].type_layer != MYEA_LAYER_LSTM || !L[li].lstm) return false;
-    // ... and a loop that leaves at least half of the compute units without a workgroup.  One that fills the device is faster
-    // alone in its column form than in the k form beside the contractions, by more than those then hide (2 x LSTM-512 at a
-    // batch of 256: 3.66 against 3.70 ms per step).
+    // ... and a loop that leaves at least half of the compute units without a workgroup: beside one that fills the device, every time
+    // step waits for the member whose compute unit a contraction shares (2 x LSTM-512 at a batch of 256, on the FP32 instruction: 3.66 ms
+    // per step with the contractions behind the loop, 3.70 with them beside the best loop for that).
     return lstm_backward_loop_leaves_room(li, B);
 }
 
