@@ -91,3 +91,20 @@ def test_two_networks_on_two_streams_take_turns():
         n.synchronize()   # a wait that gave up is reported here
     a, b = (n.download_tensor(1, mb.TENSOR["ERRORS"], T * B * cells) for n in nets)
     assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("switches", [dict(), dict(MYEA_LSTM_BACKWARD_SETS="0"),
+                                      dict(MYEA_LSTM_BACKWARD_SETS="0", MYEA_LSTM_RESIDENT_TEST_NEVER_EARLY="1")], ids=["sets", "one-stream", "one-stream-late"])
+def test_512_cells_beyond_a_row_tile_per_group(switches):
+    """where the backward pass is the FP32 loop's: both of its forms behind this forward loop, with a ragged last group"""
+    T, B, cells = 5, 141, 512
+    specs = [dict(units=7), lstm(cells), dict(units=cells, activation="LINEAR")]
+    desc, h, w, masks, X, Y = _setup(specs, T, B, 150, seed=17)
+    loop, steps = _net(desc, h, w, masks), _net(desc, h, w, masks)
+    with environment(MYEA_LSTM_RESIDENT="0"):
+        run_step(steps, B, X, Y, update=False)
+    with environment(**switches):
+        loop.profile_enable(True)
+        run_step(loop, B, X, Y, update=False)
+        assert _loop_launches(loop) == (1, 1)
+    _compare(desc, loop, steps, B, T, "512 cells")
