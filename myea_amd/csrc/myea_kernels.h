@@ -106,7 +106,7 @@ bool gemm_can_fuse_activation(int act);
 // (wa, wb) and B may be null: the zero-padded identity shortcut (narrower operand shifted by -padding) and its gradient
 // (wider operand cropped at +padding).  out may alias neither operand unless the shifts are zero.
 int launch_padded_add(hipStream_t s, size_t rows, size_t wo, const float *a, size_t wa, long sa,
-                      const float *b, size_t wb, long sb, float *out);
+                      const float *b, size_t wb, long sb, float *out, float *cropped = nullptr, size_t wc = 0, long sc = 0);
 // y = AF(x) * colscale[j]  (colscale may be null); x and y may alias.
 int launch_activation(hipStream_t s, int act, size_t rows, size_t H, const float *x, float *y, const float *colscale, const int *unit_act = nullptr);
 // row softmax (max-subtracted) then * colscale

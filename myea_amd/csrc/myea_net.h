@@ -24,6 +24,7 @@ struct DevLayer {
     // a block member carries both on its input side (In wide, no activation units on the first member); a residual
     // layer keeps its basic units in values / neuron_errors (H wide) and normalises the block's last member (NH wide)
     size_t AH = 0, NH = 0;
+    bool delta_handed_down = false;   // residual layer: this pass's errors went to its block's last member as they were written
     size_t pad = 0;   // residual layer: column offset of the narrower shortcut operand (pooling_values[2])
     // [T][Bmax][H] (summations, neuron_errors), [T][Bmax][AH] (values), [T][Bmax][NH] (hats, normalizes)
     float *summations = nullptr, *values = nullptr, *hats = nullptr, *normalizes = nullptr, *neuron_errors = nullptr;
@@ -192,6 +193,7 @@ struct Net {
     int pool_backward_with_shortcut(size_t gi, size_t rows, size_t roff, const DevLayer *shortcut, long crop, float *dst);
     int forward_residual_block(size_t ri, size_t B);
     int backward_residual_block(size_t ri, size_t B);
+    float *block_delta(size_t ri, size_t *width);
 
     int forward_pass(size_t B, const float *inputs, int on_device);
     int compute_error(size_t B, const float *desired, int on_device);

@@ -1119,6 +1119,15 @@ int Net::pool_backward_with_shortcut(size_t gi, size_t rows, size_t roff, const 
     return MYEA_OK;
 }
 
+// Where residual layer ri's errors, cropped to its block's width, go: to the block-level normalisation, or the last member's delta.
+float *Net::block_delta(size_t ri, size_t *width)
+{
+    const size_t last = ri + d.layers[ri].block_depth;
+    const bool norm = layer_uses_norm(d.layers[ri]);
+    *width = norm ? L[ri].NH : L[last].H;   // (the same width: the block's last member's)
+    return norm ? tmp1 : L[last].neuron_errors;
+}
+
 // FF__Backward_Pass_Batch (NN/Neural_Network__Backward_Pass__OpenMP.cpp:24-155): for every layer below the
 // output layer, dX = delta_next * W_next (Backward_Pass__FC, :1044-1082) and then
 // Backward_Pass__Gradient__FC (:544-709): [BN after] -> act' -> [BN before].  The act' multiply is fused
@@ -1128,6 +1137,7 @@ int Net::backward_into_layer(size_t li, size_t B)
     const myea_layer_desc &l = d.layers[li];
     DevLayer &o = L[li];
     const size_t T = d.number_recurrent_depth, Bmax = d.batch_size, H = o.H;
+    o.delta_handed_down = false;
     // next_connected_layers (Organize__Next_Layers_Connected, NN/Neural_Network.cpp:59-102): the layer after this one (after
     // this block, for a residual layer); when that is a residual layer, its shortcut AND its block's first member consume
     // this layer.  The shortcut's share (Backward_Pass__Residual, NN/Neural_Network__Backward_Pass__OpenMP.cpp:1155-1215:
@@ -1185,7 +1195,17 @@ int Net::backward_into_layer(size_t li, size_t B)
             g.C = o.neuron_errors + roff * H;
             g.epilogue = EPI_NONE;
             if (pool_consumer) { MYEA_TRY(pool_backward_with_shortcut(gi, rows, roff, shortcut, crop, g.C)); continue; }
-            if (!have_gemm) { MYEA_TRY(launch_padded_add(stream, rows, H, shortcut->neuron_errors + roff * shortcut->H, shortcut->H, crop, identity + roff * H, H, 0, g.C)); continue; }
+            if (!have_gemm) {   // a residual layer's errors go to its block's last member in the same launch
+                float *cropped = nullptr;
+                size_t wide = 0;
+                if (l.type_layer == MYEA_LAYER_RESIDUAL) {
+                    cropped = block_delta(li, &wide) + roff * wide;
+                    o.delta_handed_down = true;
+                }
+                MYEA_TRY(launch_padded_add(stream, rows, H, shortcut->neuron_errors + roff * shortcut->H, shortcut->H, crop, identity + roff * H, H, 0, g.C,
+                                           cropped, wide, o.H > o.NH ? (long)o.pad : 0));
+                continue;
+            }
             prof_begin(1);
             MYEA_TRY(launch_gemm(stream, g));
             prof_end(2.0 * (double)rows * (double)H * (double)Out);
@@ -1302,10 +1322,10 @@ int Net::backward_residual_block(size_t ri, size_t B)
     const bool shake = r.type_dropout == MYEA_DROPOUT_SHAKEDROP;
     {
         const bool norm = layer_uses_norm(r);
-        float *to = norm ? tmp1 : L[last].neuron_errors;
-        const size_t W = norm ? ro.NH : L[last].H;   // (the same width: the block's last member's)
+        size_t W = 0;
+        float *to = block_delta(ri, &W);
         MYEA_TRY(chunked([&](size_t roff, size_t rows) -> int {
-            MYEA_TRY(launch_padded_add(stream, rows, ro.NH, ro.neuron_errors + roff * ro.H, ro.H, crop, nullptr, 0, 0, to + roff * W));
+            if (!ro.delta_handed_down) MYEA_TRY(launch_padded_add(stream, rows, ro.NH, ro.neuron_errors + roff * ro.H, ro.H, crop, nullptr, 0, 0, to + roff * W));
             if (shake) MYEA_TRY(launch_shakedrop_apply(stream, rows, ro.NH, to + roff * W, ro.noise + roff, ro.noise + T * Bmax + T * Bmax * ro.NH + roff * ro.NH, 1.f));
             return MYEA_OK;
         }));
