@@ -324,7 +324,7 @@ struct LstmResidentDir {
 struct LstmResidentPlan {
     bool ok = false;       // the resident form applies
     bool agent = false;    // groups wider than one XCD: device-scope exchange
-    int members = 0, row_groups = 0, grid = 0;
+    int members = 0, row_groups = 0, grid = 0, cus = 0;
 };
 int lstm_resident_plan(size_t C, size_t cells_per_block, size_t B, int dirs, bool backward, LstmResidentPlan *plan);
 size_t lstm_resident_sync_words();
@@ -353,5 +353,7 @@ int launch_lstm_planes_forward(hipStream_t s, const LstmPlanesPlan &plan, size_t
 size_t lstm_planes_shares_floats(size_t C, size_t B, int dirs);
 int launch_lstm_planes_backward(hipStream_t s, const LstmPlanesPlan &plan, size_t T, size_t B, size_t Bmax, size_t C, int dirs, const LstmResidentDir *dir,
                                 unsigned *sync, unsigned *host_flag, unsigned *fault, float *shares, size_t shares_floats);
+// a layer's backward time loop is one launch that leaves at least half of the compute units without a workgroup
+bool lstm_backward_leaves_room(size_t C, size_t cells_per_block, size_t B, size_t Bmax, int dirs);
 
 }  // namespace myea

@@ -1627,13 +1627,19 @@ void Net::loop_order_leave()
     loop_device = -1;
 }
 
+bool lstm_backward_leaves_room(size_t C, size_t cells_per_block, size_t B, size_t Bmax, int dirs)
+{
+    LstmPlanesPlan planes;
+    if (lstm_planes_plan(C, cells_per_block, B, Bmax, dirs, &planes) != MYEA_OK) return false;
+    if (planes.ok && planes.backward) return 2 * planes.grid <= planes.cus;
+    LstmResidentPlan plan;   // (512 cells fill the device here; 1024 leave half of it up to 64 examples)
+    return lstm_resident_plan(C, cells_per_block, B, dirs, true, &plan) == MYEA_OK && plan.ok && 2 * plan.grid <= plan.cus;
+}
+
 bool Net::lstm_backward_loop_leaves_room(size_t li, size_t B)
 {
     const DevLayer &o = L[li];
-    if (!o.lstm) return false;
-    LstmPlanesPlan plan;
-    if (o.lstm->norm || lstm_planes_plan(o.lstm->C, o.lstm->cpb, B, d.batch_size, o.lstm2 ? 2 : 1, &plan) != MYEA_OK || !plan.ok || !plan.backward) return false;
-    return 2 * plan.grid <= plan.cus;
+    return o.lstm && !o.lstm->norm && lstm_backward_leaves_room(o.lstm->C, o.lstm->cpb, B, d.batch_size, o.lstm2 ? 2 : 1);
 }
 
 int Net::side_stream_create()

@@ -1506,7 +1506,7 @@ int lstm_resident_plan(size_t C, size_t cells_per_block, size_t B, int dirs, boo
     int grid = 0;
     if (agent != (C > 512) || !place_groups(*dev, *k, members, agent, row_groups * dirs, &grid)) return MYEA_OK;
     plan->ok = true; plan->agent = agent;
-    plan->members = members; plan->row_groups = row_groups; plan->grid = grid;
+    plan->members = members; plan->row_groups = row_groups; plan->grid = grid; plan->cus = dev->cus;
     return MYEA_OK;
 }
 

@@ -2,7 +2,7 @@
 C ABI: against the same library with one launch per time step (MYEA_LSTM_RESIDENT=0), against the CPU oracle, and the
 bounded wait's give-up path.  Tolerance rel 1e-4 / abs 1e-5 (the resident kernels use the exp2 and reciprocal
 instructions in the gate functions, the per-step kernels expf and a division: a few ulp apart)."""
-import os
+import ctypes as C
 
 import numpy as np
 import pytest
@@ -260,11 +260,21 @@ def test_a_backward_wait_that_gives_up_is_reported_too(cells, ksplit):
     _compare(desc, gpu, cpu, B, T, "after the backward give-up")
 
 
-def test_weight_contractions_beside_the_backward_loop_change_nothing():
+# a layer's backward loop leaves half of the 256 compute units: groups of 16 examples on the BF16 matrix cores (one to an XCD until they
+# are more than eight), of 32 at 1024 cells (64 workgroups each)
+@pytest.mark.parametrize("cells,B,dirs,room", [(1024, 1, 1, True), (1024, 64, 1, True), (1024, 65, 1, False), (256, 128, 1, True), (256, 129, 1, False),
+                                               (200, 60, 1, True), (512, 16, 1, False), (512, 141, 1, False), (1000, 16, 1, False)])
+def test_which_loops_leave_room_for_contractions_beside_them(cells, B, dirs, room):
+    leaves_room = getattr(mb.load_library(), "_ZN4myea25lstm_backward_leaves_roomEmmmmi")
+    leaves_room.argtypes, leaves_room.restype = [C.c_size_t] * 4 + [C.c_int], C.c_bool
+    assert leaves_room(cells, 1, B, B, dirs) == room
+
+
+@pytest.mark.parametrize("cells", [128, 1024])
+def test_weight_contractions_beside_the_backward_loop_change_nothing(cells):
     """the combined backward + weight-gradient call runs the weight contractions of the layer above on a second stream beside an
-    LSTM layer's backward time loop (and picks the loop's form that leaves them room): same gradient as the two separate calls
-    within the tolerance the two resident forms are held to, and the same as the oracle"""
-    specs = [dict(units=16), lstm(128), lstm(128), dict(units=128, activation="LINEAR")]
+    LSTM layer's backward time loop: same gradient as the two separate calls, and the same as the oracle"""
+    specs = [dict(units=16), lstm(cells), lstm(cells), dict(units=cells, activation="LINEAR")]
     T, B = 6, 64
     desc, h, w, masks, X, Y = _setup(specs, T, B, B, seed=13)
     combined, separate = _net(desc, h, w, None), _net(desc, h, w, None)
