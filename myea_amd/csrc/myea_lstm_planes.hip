@@ -667,6 +667,26 @@ bool flag_set(const char *name, char value)
     return e && e[0] == value;
 }
 
+// Row tiles a group at which one launch a step is not the faster form yet, both sides measured over 16 time steps, us.  A loop's step costs
+// the members' shares, tile by tile, and more than that once a XCD's shares of two steps (2 members^2 KiB a tile) outgrow its 4 MiB of L2; a launch a
+// step costs its launch, and less the better its width fills tiles (multiples of 32 have a kernel of their own).
+// Backward, loop against launches, up to the line and beyond it: 128 cells 8 tiles (4093 examples) 340 | 374, 100 cells 310 | 311, 12 tiles
+// 462 | 424; 160 x 2301 (6) 283 | 298, 2309 (7) 310 | 297; 256 x 1277 (5) 285 | 298, 1533 (6) 343 | 318; 384 x 509 (4) 228 | 248, 637 (5) 289 |
+// 263; 480 x 509 (4) 304 | 316, 517 (5) 349 | 322; 300 x 773 (7) 280 | 326, 1021 (8) 388 | 373; 200 x 1541 (7) 298 | 316, 2045 (8) 383 | 339; 500
+// x 765 (6) 523 | 538, 1021 (8) 697 | 566.  Two directions' launches share the device: 100 x 2045 (8) 307 | 314; 128 x 1277 (5) 193 | 218, 1533
+// (6) 259 | 247; 160 x 957 (5) 216 | 226, 1149 (6) 280 | 250; 256 x 509 (4) 208 | 210, 637 (5) 283 | 248; 448 x 189 (3) 167 | 208, 253 (4) 279 |
+// 245; 300 x 381 (6) 249 | 313; 500 x 317 (5) 433 | 481, 381 (6) 524 | 506.  512 cells and more than one tile: the loop of
+// myea_lstm_resident.hip is the faster one (figures there), or one launch a step where that does not hold the batch (512 examples, 30 steps:
+// 642 us against 670).
+size_t backward_most_tiles(size_t C, int dirs)
+{
+    if (C == 512) return 1;
+    if (C % 32 != 0) return dirs == 1 ? (C <= 128 ? 8 : C <= 320 ? 7 : 6) : (C <= 128 ? 8 : C <= 320 ? 6 : 5);
+    return dirs == 1 ? (C <= 128 ? 8 : C <= 224 ? 6 : C <= 320 ? 5 : 4) : (C <= 224 ? 5 : C <= 320 ? 4 : 3);
+}
+// Forward: 480 x 3712 (29 tiles) 894 | 1743, 300 x 3712 790 | 832, 200 x 7424 839 | 867; 100 x 8189 (16) 450 | 515, 14848 (29) 836 | 756.
+size_t forward_most_tiles(size_t C) { return C <= 128 ? 16 : 29; }
+
 }  // namespace
 
 int lstm_planes_plan(size_t C, size_t cells_per_block, size_t B, size_t Bmax, int dirs, LstmPlanesPlan *plan)
@@ -681,19 +701,17 @@ int lstm_planes_plan(size_t C, size_t cells_per_block, size_t B, size_t Bmax, in
     const size_t most = (size_t)(cus / 8 / members * 8) / (size_t)dirs;   // groups of one direction that fit
     if (most == 0) return MYEA_OK;
     const size_t tiles = (B + kRows - 1) / kRows, rs = (tiles + most - 1) / most;
-    // offsets into a group's exchange and into a time step's rows are 32 bits wide
-    if (rs > 32 || rs * ((C + 31) / 32) * 3072 * kSlots > 0x7fffffffu || Bmax * 4 * C > 0x3fffffffu) return MYEA_OK;
+    // offsets into a time step's rows are 32 bits wide (a group's exchange: 29 tiles x 192 KiB forward, 8 x 2 MiB backward)
+    if (rs > forward_most_tiles(C) || Bmax * 4 * C > 0x3fffffffu) return MYEA_OK;
     PlaneKernelInfo *k = forward_kernel(C);
-    if (!k || !backward_kernel(members) || forward_lds(k->waves, (int)rs) > kMaxLds || backward_lds((int)rs) > kMaxLds) return MYEA_OK;
+    if (!k || !backward_kernel(members) || forward_lds(k->waves, (int)rs) > kMaxLds) return MYEA_OK;
     plan->ok = true; plan->members = members; plan->rs = (int)rs; plan->row_tiles = (int)tiles;
     plan->row_groups = (int)((tiles + rs - 1) / rs);
     const int groups = plan->row_groups * dirs;
     if (groups > kMaxPlaneGroups) { plan->ok = false; return MYEA_OK; }
     plan->grid = 8 * ((groups + 7) / 8) * members;
     plan->cus = cus;
-    // 512 cells and more than one row tile a group: the loop of myea_lstm_resident.hip is the faster one (figures there), or one launch a step
-    // where that does not hold the batch (512 examples, 30 steps: 642 us against 670)
-    plan->backward = C < 512 || rs == 1;
+    plan->backward = rs <= backward_most_tiles(C, dirs) && backward_lds((int)rs) <= kMaxLds;
     return MYEA_OK;
 }
 

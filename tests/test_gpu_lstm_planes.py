@@ -37,6 +37,32 @@ def test_loop_of_any_width(cells, both, zoned, T, B, Bmax):
         _compare(desc, loop, steps, b, T, "%d examples" % b)
 
 
+# the last batch of the backward loop and the first of one launch a step, where the forward pass stays a loop; the first batch without either
+LINES = [(16, False, 32768, 32769, None), (100, False, 4096, 4097, 8193), (256, False, 1280, 1281, None), (480, False, 512, 513, None), (500, False, 768, 769, 3713),
+         (200, True, 768, 769, None), (224, True, 640, 641, None), (448, True, 192, 193, None)]
+
+
+@pytest.mark.parametrize("cells,both,loop,beyond,without", LINES)
+def test_lines_between_the_backward_loop_and_one_launch_a_step(cells, both, loop, beyond, without):
+    """values of both passes and the gradient against one launch a step throughout"""
+    T, directions = 3, 2 if both else 1
+    specs = [dict(units=3), lstm(cells, **(dict(bidirectional=True) if both else {})), dict(units=cells, activation="LINEAR")]
+    launches = {loop: (1, 1), beyond: (1, directions * (T - 1)), without: (directions * (T - 1),) * 2}
+    Bmax = without or beyond
+    desc, h, w, masks, X, Y = _setup(specs, T, Bmax, Bmax, seed=cells)
+    net, steps = _net(desc, h, w, masks), _net(desc, h, w, masks)
+    for B in sorted((b for b in launches if b), reverse=True):
+        with environment(MYEA_LSTM_RESIDENT="0"):
+            steps.Clear_Training_Arrays()
+            run_step(steps, B, X[:B], Y[:B], update=False)
+        net.Clear_Training_Arrays()
+        net.profile_enable(True)
+        run_step(net, B, X[:B], Y[:B], update=False)
+        assert _loop_launches(net) == launches[B], "%d examples" % B
+        net.profile_enable(False)
+        _compare(desc, net, steps, B, T, "%d examples" % B)
+
+
 @pytest.mark.parametrize("cells,B", [(40, 20), (300, 200)])
 def test_weights_beyond_the_planes(cells, B):
     """Recurrent weights of 2^110 next to ordinary ones: the planes of such a weight are an infinity and NaNs, so every sum it is part of
