@@ -1044,13 +1044,12 @@ __global__ __launch_bounds__(64 * kNarrowWaves) void narrow_dw_kernel(const floa
     narrow_dw(delta, x, slabs, H, In, rows, rows_per_wave);
 }
 
-// The same for a table of layers, grid (most slabs of one, layers): as launches of their own they were 5.6 us each, a few dozen workgroups
+// The same for a table of layers, grid (slabs, layers): as launches of their own they were 5.6 us each, a few dozen workgroups
 // at a time (29 layers of at most 32 x 32 over 7168 rows: 161 us of launches in turns on two streams, 15 us here).
-__global__ __launch_bounds__(64 * kNarrowWaves) void narrow_dw_jobs_kernel(const NarrowDwJob *__restrict__ jobs)
+__global__ __launch_bounds__(64 * kNarrowWaves) void narrow_dw_jobs_kernel(const NarrowDwJob *__restrict__ jobs, long rows, long rows_per_wave)
 {
     const NarrowDwJob job = jobs[blockIdx.y];
-    if (blockIdx.x >= job.slab_count) return;
-    narrow_dw(job.delta, job.x, job.slabs, (int)job.H, (int)job.In, (long)job.rows, (long)job.rows_per_wave);
+    narrow_dw(job.delta, job.x, job.slabs, (int)job.H, (int)job.In, rows, rows_per_wave);
 }
 
 }  // namespace
@@ -1192,17 +1191,12 @@ int launch_narrow_dw(hipStream_t stream, const float *delta, const float *x, flo
     return MYEA_OK;
 }
 
-NarrowDwJob narrow_dw_job(const float *delta, const float *x, float *slabs, size_t H, size_t In, size_t rows)
-{
-    const int S = narrow_dw_slabs(H, In, rows);
-    return NarrowDwJob{delta, x, slabs, (unsigned)H, (unsigned)In, (unsigned)rows, (unsigned)narrow_rows_per_wave(rows, S), (unsigned)S, 0u};
-}
-
-int launch_narrow_dw_jobs(hipStream_t stream, const NarrowDwJob *jobs, size_t count, unsigned most_slabs)
+int launch_narrow_dw_jobs(hipStream_t stream, const NarrowDwJob *jobs, size_t count, size_t rows)
 {
     if (count == 0) return MYEA_OK;
-    if (count > 65535 || most_slabs == 0) { set_last_error("narrow weight gradients: %zu layers in one launch", count); return MYEA_E_INVALID; }
-    hipLaunchKernelGGL(narrow_dw_jobs_kernel, dim3(most_slabs, (unsigned)count), dim3(64 * kNarrowWaves), 0, stream, jobs);
+    const int S = narrow_dw_slabs(1, 1, rows);   // the same for every layer that is narrow
+    if (count > 65535 || S <= 0) { set_last_error("narrow weight gradients: %zu layers over %zu rows in one launch", count, rows); return MYEA_E_INVALID; }
+    hipLaunchKernelGGL(narrow_dw_jobs_kernel, dim3((unsigned)S, (unsigned)count), dim3(64 * kNarrowWaves), 0, stream, jobs, (long)rows, narrow_rows_per_wave(rows, S));
     MYEA_HIP_TRY(hipGetLastError());
     return MYEA_OK;
 }

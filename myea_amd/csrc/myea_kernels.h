@@ -88,10 +88,11 @@ int launch_gemm(hipStream_t stream, const GemmParams &p);
 // narrow_dw_slabs gives their number (0: not this kernel's shape), launch_narrow_dw writes them.
 int narrow_dw_slabs(size_t H, size_t In, size_t rows);
 int narrow_dw_slabs_most(size_t H, size_t In, size_t rows);   // the largest of any number of rows up to this one
-// ... and the same for a table of layers in one launch (jobs: device memory; narrow_dw_slabs > 0 for each of them)
-struct NarrowDwJob { const float *delta, *x; float *slabs; unsigned H, In, rows, rows_per_wave, slab_count, unused; };
-NarrowDwJob narrow_dw_job(const float *delta, const float *x, float *slabs, size_t H, size_t In, size_t rows);
-int launch_narrow_dw_jobs(hipStream_t stream, const NarrowDwJob *jobs, size_t count, unsigned most_slabs);
+// ... and the same for a table of layers in one launch (jobs: device memory; narrow_dw_slabs > 0 for each of them).  What changes with the
+// number of rows is no part of the table: a batch of another size uses the one that lies there (uploading it again costs a step of three
+// narrow layers 20 of 100 us).
+struct NarrowDwJob { const float *delta, *x; float *slabs; unsigned H, In; };
+int launch_narrow_dw_jobs(hipStream_t stream, const NarrowDwJob *jobs, size_t count, size_t rows);
 int launch_narrow_dw(hipStream_t stream, const float *delta, const float *x, float *slabs, size_t H, size_t In, size_t rows);
 // dX = delta W (`a`) and dW += delta^T X (`b`) in one launch when their shapes suit it; MYEA_OK = launched, 1 = does not
 // apply (launch them one after the other), negative = error

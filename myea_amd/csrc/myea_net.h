@@ -120,6 +120,7 @@ struct Net {
     NarrowDwJob *narrow_jobs = nullptr, *narrow_jobs_staging = nullptr;   // device; pinned host
     std::vector<NarrowDwJob> narrow_pending, narrow_uploaded;
     double narrow_work = 0;
+    size_t narrow_rows = 0;                    // of every layer in narrow_pending
     int flush_slab_folds();
     // the bounds of the independently recurrent layers' self weights, clipped behind every update in one launch; built at the first update
     ClipRange *clip_ranges = nullptr;

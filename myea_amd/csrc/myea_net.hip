@@ -740,12 +740,10 @@ int Net::flush_slab_folds()
     if (fold_pending.empty()) return MYEA_OK;
     if (!narrow_pending.empty()) {
         MYEA_TRY(upload_jobs(stream, narrow_pending, &narrow_uploaded, narrow_jobs_staging, narrow_jobs));
-        unsigned most = 0;
-        for (const NarrowDwJob &j : narrow_pending) most = std::max(most, j.slab_count);
         const size_t layers = narrow_pending.size();
         narrow_pending.clear();
         prof_begin(2);
-        MYEA_TRY(launch_narrow_dw_jobs(stream, narrow_jobs, layers, most));
+        MYEA_TRY(launch_narrow_dw_jobs(stream, narrow_jobs, layers, narrow_rows));
         prof_end(narrow_work);
         narrow_work = 0;
     }
@@ -1587,7 +1585,8 @@ int Net::update_derivative_weight_contraction(size_t li, size_t B)
         float *const slabs_at = later ? narrow_slabs + narrow_slab_at[li] : dw_slabs;
         if (later) {   // with the other narrow layers' in one launch: flush_slab_folds
             prof_cancel();
-            narrow_pending.push_back(narrow_dw_job(g.A, g.B, slabs_at, H, In, rows));
+            narrow_pending.push_back(NarrowDwJob{g.A, g.B, slabs_at, (unsigned)H, (unsigned)In});
+            narrow_rows = rows;
             narrow_work += 2.0 * (double)rows * (double)H * (double)In;
             fold_pending.push_back(SlabFoldJob{slabs_at, gradient + l.first_connection_index, (unsigned)(H * In), (unsigned)narrow});
             continue;

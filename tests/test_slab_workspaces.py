@@ -5,6 +5,7 @@ import ctypes as C
 
 import numpy as np
 import pytest
+import torch
 
 from myea_amd import binding as mb
 from tests.common import assert_close, glorot_parameters
@@ -87,3 +88,41 @@ def test_call_without_allocations_sizes_its_pieces_for_the_batch():
         X, Y = (rng.normal(0, 1, (B, n)).astype(np.float32) for n in (256, 16))
         got, want = both(net, B, X, Y)
         assert np.abs(want).max() > 0 and np.array_equal(got, want)
+
+
+@pytest.mark.gpu
+def test_batches_of_other_sizes_share_the_table_of_narrow_layers():
+    """The table of narrow layers that lies on the device holds for any number of rows of as many slabs (8 at 1793 .. 2048): a batch of
+    another size neither waits for the stream - which a capture would refuse - nor sums other rows than its own."""
+    Bmax, sizes = 2048, (2048, 1800, 2047)
+    desc = mb.make_desc([dict(units=28), dict(units=32, activation="TANH"), dict(units=17, activation="TANH"), dict(units=10, activation="LINEAR")], Bmax)
+    h = mb.default_hyper(type_optimizer_function=mb.OPTIMIZER["ADAM"], type_loss_function=mb.LOSS["MSE"])
+    gpu, cpu = mb.HipNetwork(desc, h), OracleNetwork(desc, h, threads=8)
+    rng = np.random.default_rng(3)
+    X, Y = (rng.normal(0, 1, (Bmax, n)).astype(np.float32) for n in (28, 10))
+    w = glorot_parameters(desc, 3)
+    for n in (gpu, cpu):
+        n.set_state_propagation(mb.STATE_TRAINING)
+        n.upload_parameters(w)
+    stream = torch.cuda.Stream()
+    gpu.set_stream(stream.cuda_stream)
+    for B in sizes:
+        for n in (gpu, cpu):
+            n.Clear_Training_Arrays()
+            n.Forward_Pass(B, X[:B])
+            n.Compute__Error(B, Y[:B])
+            n.Backward_Pass(B)
+        cpu.Update_Derivative_Weight(B, 1, desc.n_layers)
+        want = cpu.download_gradient()
+        if B == sizes[0]:
+            gpu.Update_Derivative_Weight(B, 1, desc.n_layers)
+            assert_close(gpu.download_gradient(), want, 1e-4, 1e-5 * float(np.abs(want).max()), what="gradient of %d examples" % B)
+            continue
+        gpu.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream, capture_error_mode="thread_local"):
+            gpu.Update_Derivative_Weight(B, 1, desc.n_layers)
+        for replay in range(1, 4):   # each adds the gradient once more
+            graph.replay()
+            torch.cuda.synchronize()
+            assert_close(gpu.download_gradient(), replay * want, 1e-4, 1e-5 * replay * float(np.abs(want).max()), what="gradient of %d examples, replay %d" % (B, replay))
