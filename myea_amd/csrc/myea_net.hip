@@ -2019,6 +2019,8 @@ int Net::early_update_layer(size_t li)
     const char *e = std::getenv("MYEA_EARLY_UPDATE_MIN");   // read at every call: a test lowers it for one network
     const size_t least = e ? (size_t)std::strtoull(e, nullptr, 10) : (size_t)1 << 23;
     if ((first & 3) || (count & 3) || count < least || count == 0) return MYEA_OK;
+    for (const SlabFoldJob &j : fold_pending)   // a narrow layer's gradient is complete at the end of the call
+        if (j.dst == gradient + first) return MYEA_OK;
     MYEA_HIP_TRY(hipEventRecord(update_event, stream));
     MYEA_HIP_TRY(hipStreamWaitEvent(side_stream, update_event, 0));
     std::swap(stream, side_stream);

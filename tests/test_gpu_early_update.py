@@ -106,6 +106,9 @@ CASES = [
      "ADAM", dict(regularization__max_norm_constraints=0.8), ["FIRST_MOMENT", "SECOND_MOMENT"]),
     ("mlp-odd-widths-adam", [dict(units=7), dict(units=13, activation="TANH"), dict(units=9, activation="RELU"), dict(units=3, activation="LINEAR")], 1, 5, "MSE",
      "ADAM", {}, ["FIRST_MOMENT", "SECOND_MOMENT"]),
+    # layers whose gradient is only complete at the end of the call (at most 32 x 32, 512 rows and more)
+    ("mlp-narrow-layers-adam", [dict(units=28), dict(units=32, activation="TANH"), dict(units=32, activation="TANH"), dict(units=8, activation="LINEAR")], 1, 640, "MSE",
+     "ADAM", {}, ["FIRST_MOMENT", "SECOND_MOMENT"]),
     ("mlp-clipped-adam", [dict(units=16), dict(units=32, activation="TANH"), dict(units=8, activation="LINEAR")], 1, 12, "MSE",
      "ADAM", dict(use_clip_gradient=1, clip_gradient=0.05), ["FIRST_MOMENT", "SECOND_MOMENT"]),
     ("mlp-irprop", [dict(units=16), dict(units=32, activation="TANH"), dict(units=8, activation="LINEAR")], 1, 12, "MSE",
