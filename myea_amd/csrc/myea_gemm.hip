@@ -725,10 +725,15 @@ struct ShortOperand<true, WAVES, true> {
     }
 };
 
-// The same in the lanes that multiply it.  Where A has only a few rows, all lanes of an instruction are in their lines, and the trip through
-// LDS and the set-up of the ranges are what remains (1 x 256, k = 784: 7.3 us against 7.6; 8 x 1000, k = 1000 9.0 against 9.9; 16 x 1000 9.3
-// against 9.1; 24 x 2048, k = 2048 17.3 against 14.5).
-constexpr int kShortDirectRows = 8;
+// The same in the lanes that multiply it.  Where A has only a few rows, or a tile's rows of A and of B are few together, the instructions
+// are few lines each, and the trip through LDS and the set-up of the ranges are what remains.  us, direct against turned round: 1 x 256, k = 784
+// 7.3 | 7.6; 8 x 1000, k = 1000 9.0 | 9.9; 16 x 1000 9.3 | 9.1; 24 x 2048, k = 2048 17.3 | 14.5; k = 4096: 9 x 10 21.0 | 23.6, 16 x 16 22.4 |
+// 23.7, 64 x 1 22.9 | 24.3, 14 x 20 22.5 | 23.4, 32 x 4 23.5 | 23.7, 16 x 20 23.1 | 23.3, 16 x 24 24.0 | 23.5.
+inline bool short_direct(const GemmDev &d)
+{
+    constexpr int kRows = 8, kRowsTogether = 34;
+    return d.M <= kRows || min(d.M, 32) + min(d.N, 32) <= kRowsTogether;
+}
 template <int WAVES>
 struct ShortOperand<true, WAVES, false> {
     float reg[2][2][8];   // [slot][group of 16 k's][k]
@@ -862,7 +867,7 @@ int launch_short(hipStream_t stream, GemmDev d, bool a_kc, bool b_kc)
     // share one instead of the second waiting for the first.  us, eight -> four, 333 x 1201 (418 workgroups): k = 64 7.5 -> 5.7, 256
     // 9.5 -> 7.8, 1000 20.9 -> 18.2; up to one per compute unit: 10 x 1000, k = 1000 9.4 against 10.8.
     if (nblocks > kShortMost) launch_short_waves<4>(stream, d, a_kc, b_kc, nblocks);
-    else if (a_kc && b_kc && d.M <= kShortDirectRows) hipLaunchKernelGGL((short_gemm_kernel<true, true, 8, false>), dim3((unsigned)nblocks), dim3(64 * 8), 0, stream, d);
+    else if (a_kc && b_kc && short_direct(d)) hipLaunchKernelGGL((short_gemm_kernel<true, true, 8, false>), dim3((unsigned)nblocks), dim3(64 * 8), 0, stream, d);
     else launch_short_waves<8>(stream, d, a_kc, b_kc, nblocks);
     MYEA_HIP_TRY(hipGetLastError());
     return MYEA_OK;

@@ -1,5 +1,5 @@
 """The short product (few tiles, its wavefronts share k) around the forms its operands are loaded in: whole lines turned round in LDS
-against rows straight into the lanes (up to 8 rows of A), k's that end inside a 16-byte chunk, a run or a round of runs, rows and columns
+against rows straight into the lanes (up to 8 rows of A, or 34 of A and B in a tile), k's that end inside a 16-byte chunk, a run or a round of runs, rows and columns
 that end inside a tile, rows that are not 16-byte aligned, four and eight wavefronts - against float64."""
 import pytest
 import torch
@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("a_kc,b_kc", LAYOUTS)
-@pytest.mark.parametrize("M,N", [(1, 77), (8, 256), (9, 33), (40, 95), (333, 500)])
+@pytest.mark.parametrize("M,N", [(1, 77), (8, 256), (9, 33), (14, 20), (15, 20), (70, 2), (70, 3), (40, 95), (333, 500)])
 @pytest.mark.parametrize("K", [16, 29, 32, 35, 255, 256, 258, 511, 545, 783])
 def test_edges_against_float64(a_kc, b_kc, M, N, K):
     """an accumulator takes one rounding (2^-23 of what it holds, at most the sum of the magnitudes) per 16 k's, a few more join the parts"""
