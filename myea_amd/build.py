@@ -40,10 +40,10 @@ def build(verbose=False):
         _run(["gcc", "-O2", "-fPIC", "-std=c11", "-Wall", "-c", os.path.join(CSRC, src), "-o", obj])
         objs.append(obj)
     _run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB, *objs])
-    # the C++ adaptor's check programs (host code only; link the C ABI)
+    # the check programs of the C++ adaptor and of the host code's headers (host code only; link the C ABI)
     root = os.path.dirname(HERE)
-    for name in ("adaptor_check", "dataset_check", "checkpoint_check"):
-        _run(["g++", "-O2", "-std=c++17", "-Wall", "-fopenmp", os.path.join(root, "tests", "cpp", name + ".cpp"), "-o",
+    for name in ("adaptor_check", "dataset_check", "checkpoint_check", "loop_order_check"):
+        _run(["g++", "-O2", "-std=c++17", "-Wall", "-fopenmp", "-pthread", os.path.join(root, "tests", "cpp", name + ".cpp"), "-o",
               os.path.join(root, "tests", "cpp", name), "-L" + CSRC, "-lmyea_hip", "-Wl,-rpath," + CSRC,
               "-Wl,-rpath,$ORIGIN/../../myea_amd/csrc"])
     return LIB

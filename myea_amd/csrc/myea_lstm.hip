@@ -22,6 +22,7 @@
 
 #include "myea_device_af.h"
 #include "myea_kernels.h"
+#include "myea_loop_order.h"
 #include "myea_net.h"
 #include "myea_reduce.h"
 
@@ -1560,48 +1561,37 @@ int Net::lstm_backward_step_norm(LstmLayer &q, size_t B, size_t s)
     return MYEA_OK;
 }
 
-// Two resident loops at once may each hold compute units that the other's workgroups wait for.  So while more than one network of the
-// process has such layers on a device, a loop waits (on the device) for the loop launched before it on another network's stream; a
-// stream that is being captured is left alone.
+// The resident loops of the networks of this process on a device: myea_loop_order.h.
 namespace {
 
-struct LoopOrder {
-    std::mutex mutex;
-    int networks = 0;
-    hipEvent_t last = nullptr;         // behind the last loop launched
-    const void *owner = nullptr;       // the network that launched it
-};
-LoopOrder g_loop_order[64];
+struct LoopDevice {
+    using Stream = hipStream_t;
+    hipEvent_t last = nullptr;   // the mark
+    int id = -1;
 
-struct LoopTurn {
-    LoopOrder *order = nullptr;
-    const void *net;
-    hipStream_t stream;
-    LoopTurn(const void *n, int device, hipStream_t s) : net(n), stream(s)
+    bool capturing(hipStream_t s)
     {
-        if (device < 0) return;
-        LoopOrder &o = g_loop_order[device];
-        o.mutex.lock();
-        order = &o;
-        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-        if (o.networks < 2 || hipStreamIsCapturing(stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) { leave(); return; }
-        if (!o.last && hipEventCreateWithFlags(&o.last, hipEventDisableTiming) != hipSuccess) { o.last = nullptr; leave(); return; }
-        if (o.owner && o.owner != net) (void)hipStreamWaitEvent(stream, o.last, 0);
+        hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
+        return hipStreamIsCapturing(s, &c) != hipSuccess || c != hipStreamCaptureStatusNone;
     }
-    void leave()
+    void await(hipStream_t s) { (void)hipStreamWaitEvent(s, last, 0); }
+    bool mark(hipStream_t s)
     {
-        if (order) order->mutex.unlock();
-        order = nullptr;
+        if (!last && hipEventCreateWithFlags(&last, hipEventDisableTiming) != hipSuccess) { last = nullptr; return false; }
+        return hipEventRecord(last, s) == hipSuccess;
     }
-    ~LoopTurn()
+    void wait_idle()
     {
-        if (!order) return;
-        if (hipEventRecord(order->last, stream) == hipSuccess) order->owner = net;
-        leave();
+        int here = -1;
+        if (hipGetDevice(&here) != hipSuccess || (here != id && hipSetDevice(id) != hipSuccess)) return;
+        (void)hipDeviceSynchronize();
+        if (here != id) (void)hipSetDevice(here);
     }
-    LoopTurn(const LoopTurn &) = delete;
-    LoopTurn &operator=(const LoopTurn &) = delete;
 };
+LoopOrder<LoopDevice> g_loop_order[64];
+using HipLoopTurn = LoopTurn<LoopDevice>;
+
+LoopOrder<LoopDevice> *loop_order(int device) { return device < 0 ? nullptr : &g_loop_order[device]; }
 
 }  // namespace
 
@@ -1610,20 +1600,19 @@ int Net::loop_order_join()
     int dev = -1;
     MYEA_HIP_TRY(hipGetDevice(&dev));
     if (dev < 0 || dev >= 64 || loop_device >= 0) return MYEA_OK;
-    LoopOrder &o = g_loop_order[dev];
-    std::lock_guard<std::mutex> lock(o.mutex);
+    LoopOrder<LoopDevice> &o = g_loop_order[dev];
+    {
+        std::lock_guard<std::mutex> lock(o.mutex);
+        o.device.id = dev;
+    }
+    o.join();
     loop_device = dev;
-    if (++o.networks == 2) (void)hipDeviceSynchronize();   // the first network's loops so far have left no event behind
     return MYEA_OK;
 }
 
 void Net::loop_order_leave()
 {
-    if (loop_device < 0) return;
-    LoopOrder &o = g_loop_order[loop_device];
-    std::lock_guard<std::mutex> lock(o.mutex);
-    --o.networks;
-    if (o.owner == this) o.owner = nullptr;
+    if (loop_device >= 0) g_loop_order[loop_device].leave(this);
     loop_device = -1;
 }
 
@@ -1694,7 +1683,7 @@ int Net::lstm_forward_layer(size_t li, size_t B)
             lstm_resident_dirs(o, rd);
             prof_begin(kProfLstmForwardLoop);
             {
-                LoopTurn turn(this, loop_device, stream);
+                HipLoopTurn turn(loop_order(loop_device), this, stream);
                 MYEA_TRY(launch_lstm_planes_forward(stream, plan, T, B, d.batch_size, o.lstm->C, dirs, rd, planes_sync, resident_flag, fault, planes_exchange, planes_exchange_floats));
             }
             prof_end(dirs * loop_work, 1);
@@ -1715,7 +1704,7 @@ int Net::lstm_forward_layer(size_t li, size_t B)
             lstm_resident_dirs(o, rd);
             prof_begin(kProfLstmForwardLoop);
             {
-                LoopTurn turn(this, loop_device, stream);
+                HipLoopTurn turn(loop_order(loop_device), this, stream);
                 MYEA_TRY(launch_lstm_resident_forward(stream, plan, T, B, d.batch_size, o.lstm->C, dirs, rd, resident_sync, resident_flag, fault));
             }
             prof_end(dirs * loop_work, 1);
@@ -1824,7 +1813,7 @@ int Net::lstm_backward_layer(size_t li, size_t B)
             lstm_resident_dirs(o, rd);
             prof_begin(kProfLstmBackwardLoop);
             {
-                LoopTurn turn(this, loop_device, stream);
+                HipLoopTurn turn(loop_order(loop_device), this, stream);
                 MYEA_TRY(launch_lstm_planes_backward(stream, plan, T, B, d.batch_size, o.lstm->C, dirs, rd, planes_sync, resident_flag, fault, planes_shares, planes_shares_floats));
             }
             prof_end(dirs * loop_work, 1);
@@ -1844,7 +1833,7 @@ int Net::lstm_backward_layer(size_t li, size_t B)
             lstm_resident_dirs(o, rd);
             prof_begin(kProfLstmBackwardLoop);
             {
-                LoopTurn turn(this, loop_device, stream);
+                HipLoopTurn turn(loop_order(loop_device), this, stream);
                 MYEA_TRY(launch_lstm_resident_backward(stream, plan, T, B, d.batch_size, o.lstm->C, dirs, rd, resident_sync, resident_flag, fault));
             }
             prof_end(dirs * loop_work, 1);
