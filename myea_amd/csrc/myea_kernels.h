@@ -345,7 +345,8 @@ struct LstmPlanesPlan {
 };
 int lstm_planes_plan(size_t C, size_t cells_per_block, size_t B, size_t Bmax, int dirs, LstmPlanesPlan *plan);
 size_t lstm_planes_sync_words();
-// floats of the forward loop's exchange buffer (16-byte aligned, cleared by the call) for up to B examples per direction
+// floats of the forward loop's exchange buffer (16-byte aligned, cleared by the call) for up to B examples per direction: no more than the
+// largest batch that there is a plan for takes
 size_t lstm_planes_exchange_floats(size_t C, size_t B, int dirs);
 int launch_lstm_planes_forward(hipStream_t s, const LstmPlanesPlan &plan, size_t T, size_t B, size_t Bmax, size_t C, int dirs, const LstmResidentDir *dir,
                                unsigned *sync, unsigned *host_flag, unsigned *fault, float *exchange, size_t exchange_floats);

@@ -687,6 +687,10 @@ size_t backward_most_tiles(size_t C, int dirs)
 // Forward: 480 x 3712 (29 tiles) 894 | 1743, 300 x 3712 790 | 832, 200 x 7424 839 | 867; 100 x 8189 (16) 450 | 515, 14848 (29) 836 | 756.
 size_t forward_most_tiles(size_t C) { return C <= 128 ? 16 : 29; }
 
+constexpr int kMostCus = 256;   // the buffers are sized for
+// groups of one direction that are resident at once
+size_t groups_that_fit(int cus, size_t C, int dirs) { return (size_t)cus / 8 / ((C + kCells - 1) / kCells) * 8 / (size_t)dirs; }
+
 }  // namespace
 
 int lstm_planes_plan(size_t C, size_t cells_per_block, size_t B, size_t Bmax, int dirs, LstmPlanesPlan *plan)
@@ -697,8 +701,9 @@ int lstm_planes_plan(size_t C, size_t cells_per_block, size_t B, size_t Bmax, in
     int dev = -1, cus = 0;
     MYEA_HIP_TRY(hipGetDevice(&dev));
     MYEA_HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    cus = std::min(cus, kMostCus);
     const int members = (int)(C + kCells - 1) / kCells;
-    const size_t most = (size_t)(cus / 8 / members * 8) / (size_t)dirs;   // groups of one direction that fit
+    const size_t most = groups_that_fit(cus, C, dirs);
     if (most == 0) return MYEA_OK;
     const size_t tiles = (B + kRows - 1) / kRows, rs = (tiles + most - 1) / most;
     // offsets into a time step's rows are 32 bits wide (a group's exchange: 29 tiles x 192 KiB forward, 8 x 2 MiB backward)
@@ -715,18 +720,24 @@ int lstm_planes_plan(size_t C, size_t cells_per_block, size_t B, size_t Bmax, in
     return MYEA_OK;
 }
 
+// row tiles of all groups of a direction, those of the last one rounded up, for up to B examples
+static size_t planes_tiles(size_t C, size_t B, int dirs, size_t most_tiles)
+{
+    const size_t most = groups_that_fit(kMostCus, C, dirs);
+    return std::min((B + kRows - 1) / kRows + most, most * most_tiles);
+}
+
 size_t lstm_planes_exchange_floats(size_t C, size_t B, int dirs)
 {
     if (C < 16 || C > 512 || B == 0) return 0;
-    const size_t members = (C + kCells - 1) / kCells, tiles = (B + kRows - 1) / kRows + 256 / members;   // (a group's row tiles are rounded up)
-    return (size_t)dirs * tiles * ((C + 31) / 32) * 3072 * kSlots / sizeof(float);
+    return (size_t)dirs * planes_tiles(C, B, dirs, forward_most_tiles(C)) * ((C + 31) / 32) * 3072 * kSlots / sizeof(float);
 }
 
 size_t lstm_planes_shares_floats(size_t C, size_t B, int dirs)
 {
     if (C < 16 || C > 512 || B == 0) return 0;
-    const size_t members = (C + kCells - 1) / kCells, tiles = (B + kRows - 1) / kRows + 256 / members;
-    return (size_t)dirs * 2 * tiles * members * members * 256;
+    const size_t members = (C + kCells - 1) / kCells;
+    return (size_t)dirs * 2 * planes_tiles(C, B, dirs, backward_most_tiles(C, dirs)) * members * members * 256;
 }
 
 static int prepare(hipStream_t s, const LstmPlanesPlan &plan, size_t T, size_t B, size_t Bmax, size_t C, int dirs, unsigned *sync, unsigned *host_flag, unsigned *fault,

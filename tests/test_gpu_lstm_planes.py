@@ -3,6 +3,8 @@ block of k's without an owner), one member, a last member of one cell, one and s
 them, examples missing from the last tile, more steps than the exchange buffer has slots, two directions, zoneout, a smaller batch
 behind a larger one - against one launch per time step (MYEA_LSTM_RESIDENT=0; the two paths sum in another order and round their gate
 functions differently by a few ulp: rel 1e-4 / abs 1e-5 as for the other LSTM paths) - and what the planes cannot hold."""
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
@@ -61,6 +63,34 @@ def test_lines_between_the_backward_loop_and_one_launch_a_step(cells, both, loop
         assert _loop_launches(net) == launches[B], "%d examples" % B
         net.profile_enable(False)
         _compare(desc, net, steps, B, T, "%d examples" % B)
+
+
+class _Plan(C.Structure):
+    _fields_ = [("ok", C.c_bool), ("backward", C.c_bool)] + [(n, C.c_int) for n in ("members", "rs", "row_tiles", "row_groups", "grid", "cus")]
+
+
+@pytest.mark.parametrize("dirs", [1, 2])
+def test_every_plan_fits_the_buffers_of_a_larger_batch(dirs):
+    lib = mb.load_library()
+    plan_of = getattr(lib, "_ZN4myea16lstm_planes_planEmmmmiPNS_14LstmPlanesPlanE")
+    plan_of.argtypes = [C.c_size_t] * 4 + [C.c_int, C.POINTER(_Plan)]
+    floats = [getattr(lib, "_ZN4myea%sEmmi" % n) for n in ("27lstm_planes_exchange_floats", "25lstm_planes_shares_floats")]
+    for f in floats:
+        f.argtypes, f.restype = [C.c_size_t, C.c_size_t, C.c_int], C.c_size_t
+    for cells in (16, 17, 40, 100, 128, 129, 200, 224, 256, 257, 300, 320, 352, 448, 480, 500, 512):
+        largest, plans = [0, 0], 0
+        for B in sorted(set(list(range(1, 600)) + [n * 16 + d for n in range(40, 600, 7) for d in (0, 1, 15)] + [2 ** n + d for n in range(10, 17) for d in (0, 1)])):
+            plan = _Plan()
+            assert plan_of(cells, 1, B, B, dirs, C.byref(plan)) == 0
+            if plan.ok:
+                tiles = dirs * plan.row_groups * plan.rs
+                plans += 1
+                largest[0] = max(largest[0], tiles * ((cells + 31) // 32) * 3072 * 4 // 4)
+                if plan.backward:
+                    largest[1] = max(largest[1], tiles * 2 * plan.members ** 2 * 256)
+            for f, most in zip(floats, largest):
+                assert f(cells, B, dirs) >= most, (cells, B)
+        assert plans > 100 and min(largest) > 0
 
 
 @pytest.mark.parametrize("cells,B", [(40, 20), (300, 200)])

@@ -38,6 +38,17 @@ def test_narrow_kernel_never_exceeds_its_bound():
         assert reached <= most(27, 28, rows), rows
 
 
+def test_buffers_of_the_time_loops_end_where_the_loops_do():
+    """sizes at any batch beyond the last plan: 8 groups of 4 tiles, two steps of 30 x 30 KiB each, at 480 cells, one tile a group at 512"""
+    shares, exchange = getattr(mb.load_library(), "_ZN4myea25lstm_planes_shares_floatsEmmi"), getattr(mb.load_library(), "_ZN4myea27lstm_planes_exchange_floatsEmmi")
+    for f in (shares, exchange):
+        f.argtypes, f.restype = [C.c_size_t, C.c_size_t, C.c_int], C.c_size_t
+    for B in (4096, 16384, 10 ** 6):
+        assert shares(480, B, 1) == 8 * 4 * 2 * 30 * 30 * 256 and shares(512, B, 1) == shares(512, B, 2) == 8 * 2 * 32 * 32 * 256
+        assert exchange(480, B, 1) <= 8 * 29 * 15 * 3072
+    assert max(f(c, 10 ** 7, d) for f in (shares, exchange) for c in range(16, 513) for d in (1, 2)) <= 2 ** 25   # 128 MiB
+
+
 def _gradients(specs, Bmax, T, B, seed):
     desc = mb.make_desc(specs, Bmax, T)
     h = mb.default_hyper(type_optimizer_function=mb.OPTIMIZER["ADAM"], type_loss_function=mb.LOSS["MSE"])
