@@ -11,7 +11,7 @@ import torch
 
 from myea_amd import binding as mb
 from tests.common import assert_close, environment, run_step
-from tests.test_gpu_lstm_resident import ABS, REL, _compare, _loop_launches, _net, _setup, lstm, zone
+from tests.test_gpu_lstm_resident import ABS, REL, _compare, _loop_launches, _net, _setup, lstm, planes_plan, zone
 
 pytestmark = pytest.mark.gpu
 
@@ -65,23 +65,16 @@ def test_lines_between_the_backward_loop_and_one_launch_a_step(cells, both, loop
         _compare(desc, net, steps, B, T, "%d examples" % B)
 
 
-class _Plan(C.Structure):
-    _fields_ = [("ok", C.c_bool), ("backward", C.c_bool)] + [(n, C.c_int) for n in ("members", "rs", "row_tiles", "row_groups", "grid", "cus")]
-
-
 @pytest.mark.parametrize("dirs", [1, 2])
 def test_every_plan_fits_the_buffers_of_a_larger_batch(dirs):
     lib = mb.load_library()
-    plan_of = getattr(lib, "_ZN4myea16lstm_planes_planEmmmmiPNS_14LstmPlanesPlanE")
-    plan_of.argtypes = [C.c_size_t] * 4 + [C.c_int, C.POINTER(_Plan)]
     floats = [getattr(lib, "_ZN4myea%sEmmi" % n) for n in ("27lstm_planes_exchange_floats", "25lstm_planes_shares_floats")]
     for f in floats:
         f.argtypes, f.restype = [C.c_size_t, C.c_size_t, C.c_int], C.c_size_t
     for cells in (16, 17, 40, 100, 128, 129, 200, 224, 256, 257, 300, 320, 352, 448, 480, 500, 512):
         largest, plans = [0, 0], 0
         for B in sorted(set(list(range(1, 600)) + [n * 16 + d for n in range(40, 600, 7) for d in (0, 1, 15)] + [2 ** n + d for n in range(10, 17) for d in (0, 1)])):
-            plan = _Plan()
-            assert plan_of(cells, 1, B, B, dirs, C.byref(plan)) == 0
+            plan = planes_plan(cells, B, dirs)
             if plan.ok:
                 tiles = dirs * plan.row_groups * plan.rs
                 plans += 1
@@ -122,8 +115,8 @@ def test_weights_beyond_the_planes(cells, B):
         for a, b in zip(*out):
             same = np.isfinite(a) & np.isfinite(b)
             assert np.array_equal(np.isnan(a), np.isnan(b)) and np.array_equal(a[~same], b[~same], equal_nan=True)
-            scale = float(np.abs(b[same]).max())
-            assert_close(a[same] / scale, b[same] / scale, REL, ABS, what="weights of %g" % value)
+            assert (np.abs(b[same]) < 1e3).any()   # ordinary values among them are held to the ordinary tolerance
+            assert_close(a[same], b[same], REL, ABS, what="weights of %g" % value)
 
 
 def test_two_networks_on_two_streams_take_turns():

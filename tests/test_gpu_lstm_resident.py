@@ -1,7 +1,9 @@
-"""The LSTM time loop as one resident launch per layer and pass (C = 128, 256, 512 cells; 1024 forward only), through the
-C ABI: against the same library with one launch per time step (MYEA_LSTM_RESIDENT=0), against the CPU oracle, and the
-bounded wait's give-up path.  Tolerance rel 1e-4 / abs 1e-5 (the resident kernels use the exp2 and reciprocal
-instructions in the gate functions, the per-step kernels expf and a division: a few ulp apart)."""
+"""The LSTM time loop as one resident launch per layer and pass, through the C ABI: against the same library with one launch per time step
+(MYEA_LSTM_RESIDENT=0), against the CPU oracle, and the bounded wait's give-up path.  Up to 512 cells the loops run on the BF16 matrix
+cores; the FP32 instruction has the backward loop of 512 cells at more than one row of 16 examples a group, in two forms - a member's two chains
+in two sets of wavefronts, or (MYEA_LSTM_BACKWARD_SETS=0) in one instruction stream - and both loops of 1024.
+Tolerance rel 1e-4 / abs 1e-5 (the resident kernels use the exp2 and reciprocal instructions in the gate functions, the
+per-step kernels expf and a division: a few ulp apart)."""
 import ctypes as C
 
 import numpy as np
@@ -21,18 +23,40 @@ FORWARD_LOOP, BACKWARD_LOOP = 5, 6   # profile families of the time loops
 lstm = lambda units, **kw: dict(type="lstm", units=units, **kw)
 zone = lambda units, **kw: dict(type="lstm", units=units, dropout="ZONEOUT", keep=0.3, keep_output=0.2, **kw)
 
-# name, layers, T, B, Bmax, resident backward loop too
+class PlanesPlan(C.Structure):
+    _fields_ = [("ok", C.c_bool), ("backward", C.c_bool)] + [(n, C.c_int) for n in ("members", "rs", "row_tiles", "row_groups", "grid", "cus")]
+
+
+def planes_plan(cells, B, dirs=1):
+    """how a layer runs on the BF16 matrix cores: ok (forward) and backward say whether it does, rs how many row tiles a group has"""
+    plan_of = getattr(mb.load_library(), "_ZN4myea16lstm_planes_planEmmmmiPNS_14LstmPlanesPlanE")
+    plan_of.argtypes = [C.c_size_t] * 4 + [C.c_int, C.POINTER(PlanesPlan)]
+    plan = PlanesPlan()
+    assert plan_of(cells, 1, B, B, dirs, C.byref(plan)) == 0
+    return plan
+
+
+def _fp32_backward(layers, B):
+    """the FP32 instruction has the backward loop of the layers that have a loop of 512 or 1024 cells"""
+    return [not planes_plan(_width(l), B, 2 if l.use_bidirectional else 1).backward for l in layers]
+
+
+# name, layers, T, B, Bmax, which layers' backward loops are the FP32 instruction's
 CASES = [
-    ("128-cells-last-chain-ragged", [dict(units=24), lstm(128), dict(units=128, activation="LINEAR")], 9, 70, 72, True),
-    ("128-cells-second-chain-empty", [dict(units=8), lstm(128), dict(units=128, activation="LINEAR")], 5, 13, 16, True),
-    ("256-cells-two-directions", [dict(units=12), lstm(256, bidirectional=True), dict(units=256, activation="TANH")], 5, 33, 40, True),
-    ("512-cells-zoneout-stacked", [dict(units=16), zone(512), lstm(128), dict(units=128, activation="LINEAR")], 4, 48, 48, True),
-    ("512-cells-two-directions-ragged", [dict(units=9), lstm(512, bidirectional=True), dict(units=512, activation="LINEAR")], 4, 41, 44, True),
-    ("1024-cells-two-directions", [dict(units=10), lstm(1024, bidirectional=True), dict(units=1024, activation="LINEAR")], 3, 40, 40, True),
-    ("1024-cells-ragged-seven-steps", [dict(units=6), lstm(1024), dict(units=1024, activation="LINEAR")], 7, 45, 48, True),
-    ("1024-cells-two-steps", [dict(units=5), lstm(1024), dict(units=1024, activation="LINEAR")], 2, 33, 33, True),
-    ("1024-cells-twelve-steps-zoneout", [dict(units=7), zone(1024, bidirectional=True), dict(units=1024, activation="LINEAR")], 12, 64, 64, True),
-    ("two-steps", [dict(units=6), lstm(256), dict(units=256, activation="LINEAR")], 2, 32, 32, True),
+    ("128-cells-last-chain-ragged", [dict(units=24), lstm(128), dict(units=128, activation="LINEAR")], 9, 70, 72, [False]),
+    ("128-cells-second-chain-empty", [dict(units=8), lstm(128), dict(units=128, activation="LINEAR")], 5, 13, 16, [False]),
+    ("256-cells-two-directions", [dict(units=12), lstm(256, bidirectional=True), dict(units=256, activation="TANH")], 5, 33, 40, [False]),
+    ("512-cells-zoneout-stacked", [dict(units=16), zone(512), lstm(128), dict(units=128, activation="LINEAR")], 4, 48, 48, [False, False]),
+    ("512-cells-two-directions-ragged", [dict(units=9), lstm(512, bidirectional=True), dict(units=512, activation="LINEAR")], 4, 41, 44, [False]),
+    ("512-cells-beyond-a-row-zoneout-stacked", [dict(units=16), zone(512), lstm(128), dict(units=128, activation="LINEAR")], 4, 141, 144, [True, False]),
+    ("512-cells-beyond-a-row-two-directions", [dict(units=9), lstm(512, bidirectional=True), dict(units=512, activation="LINEAR")], 4, 70, 70, [True]),
+    ("512-cells-beyond-a-row-two-directions-zoneout", [dict(units=7), zone(512, bidirectional=True), dict(units=512, activation="LINEAR")], 6, 128, 128, [True]),
+    ("512-cells-beyond-a-row-two-steps", [dict(units=5), lstm(512), dict(units=512, activation="LINEAR")], 2, 256, 256, [True]),
+    ("1024-cells-two-directions", [dict(units=10), lstm(1024, bidirectional=True), dict(units=1024, activation="LINEAR")], 3, 40, 40, [True]),
+    ("1024-cells-ragged-seven-steps", [dict(units=6), lstm(1024), dict(units=1024, activation="LINEAR")], 7, 45, 48, [True]),
+    ("1024-cells-two-steps", [dict(units=5), lstm(1024), dict(units=1024, activation="LINEAR")], 2, 33, 33, [True]),
+    ("1024-cells-twelve-steps-zoneout", [dict(units=7), zone(1024, bidirectional=True), dict(units=1024, activation="LINEAR")], 12, 64, 64, [True]),
+    ("two-steps", [dict(units=6), lstm(256), dict(units=256, activation="LINEAR")], 2, 32, 32, [False]),
 ]
 
 
@@ -82,38 +106,33 @@ def _loop_launches(net):
     return net.profile_read(FORWARD_LOOP)[0], net.profile_read(BACKWARD_LOOP)[0]
 
 
-# the backward loop has two resident forms: split along k (members exchange partial sums; the default) and split along the
-# columns of dh (members read each other's gate deltas; MYEA_LSTM_BACKWARD_KSPLIT=0); at 512 cells the column form runs a
-# member's two chains in two sets of wavefronts, or (MYEA_LSTM_BACKWARD_SETS=0) in one instruction stream as at other widths
-FORMS = [("backward-split-along-k", "1", "1"), ("backward-split-along-columns", "0", "1")]
-LOOP_CASES = [c + f[1:] for c in CASES for f in FORMS] + [c + ("0", "0") for c in CASES if "512-cells" in c[0]]
-LOOP_IDS = ["%s-%s" % (f[0], c[0]) for c in CASES for f in FORMS] + ["backward-split-along-columns-one-stream-" + c[0] for c in CASES if "512-cells" in c[0]]
+LOOP_CASES = [c + ("1",) for c in CASES] + [c + ("0",) for c in CASES if "beyond-a-row" in c[0]]
+LOOP_IDS = [c[0] + ("" if c[-1] == "1" else "-one-stream") for c in LOOP_CASES]
 
 
-@pytest.mark.parametrize("name,specs,T,B,Bmax,backward,ksplit,sets", LOOP_CASES, ids=LOOP_IDS)
-def test_resident_loop_matches_one_launch_per_step_and_the_oracle(name, specs, T, B, Bmax, backward, ksplit, sets):
+@pytest.mark.parametrize("name,specs,T,B,Bmax,fp32,sets", LOOP_CASES, ids=LOOP_IDS)
+def test_resident_loop_matches_one_launch_per_step_and_the_oracle(name, specs, T, B, Bmax, fp32, sets):
     desc, h, w, masks, X, Y = _setup(specs, T, B, Bmax, seed=21)
     resident = _net(desc, h, w, masks)
     stepwise = _net(desc, h, w, masks)
-    cpu = OracleNetwork(desc, h)
+    cpu = OracleNetwork(desc, h, threads=8)
     cpu.set_state_propagation(mb.STATE_TRAINING)
     cpu.upload_parameters(w)
     if masks is not None:
         cpu.upload_zoneout_masks(masks)
     cpu.Clear_Training_Arrays()
     layers = [desc.layers[i] for i in range(desc.n_layers) if desc.layers[i].type_layer == mb.LAYER_LSTM]
-    wide = [l for l in layers]   # every LSTM layer of these cases has a resident form
+    assert _fp32_backward(layers, B) == fp32
     per_step = sum((2 if l.use_bidirectional else 1) * (T - 1) for l in layers)
     for step in range(2):
-        with environment(MYEA_LSTM_BACKWARD_KSPLIT=ksplit, MYEA_LSTM_BACKWARD_SETS=sets):
+        with environment(MYEA_LSTM_BACKWARD_SETS=sets):
             resident.profile_enable(True)
             resident.Reset__Loss()
             run_step(resident, B, X, Y, update=False)
             fwd, bwd = _loop_launches(resident)
             resident.profile_enable(False)
-        assert fwd == len(wide), "the forward time loops did not run as one launch per layer"
-        if backward:
-            assert bwd == len(wide), "the backward time loops did not run as one launch per layer"
+        assert fwd == len(layers), "the forward time loops did not run as one launch per layer"
+        assert bwd == len(layers), "the backward time loops did not run as one launch per layer"
         with environment(MYEA_LSTM_RESIDENT=0):
             stepwise.profile_enable(True)
             stepwise.Reset__Loss()
@@ -132,20 +151,25 @@ def test_resident_loop_matches_one_launch_per_step_and_the_oracle(name, specs, T
         stepwise.upload_parameters(wc)
 
 
-@pytest.mark.parametrize("ksplit", ["1", "0"], ids=["backward-split-along-k", "backward-split-along-columns"])
-def test_bias_and_peephole_gradients_summed_inside_the_backward_loop(ksplit):
+@pytest.mark.parametrize("specs,T,Bmax,batches,fp32,sets", [
+    ([dict(units=12), lstm(256, bidirectional=True), lstm(128), dict(units=128, activation="LINEAR")], 7, 80, (80, 45), (False, False), "1"),
+    ([dict(units=12), lstm(512, bidirectional=True), dict(units=512, activation="LINEAR")], 5, 128, (128, 70, 41), (True, True, False), "1"),
+    ([dict(units=12), lstm(512), dict(units=512, activation="LINEAR")], 5, 150, (150, 129), (True, True), "0"),
+    ([dict(units=12), lstm(1024), dict(units=1024, activation="LINEAR")], 3, 60, (60, 20), (True, True), "1"),
+], ids=["256-and-128-cells", "512-cells-two-directions", "512-cells-one-stream", "1024-cells"])
+def test_bias_and_peephole_gradients_summed_inside_the_backward_loop(specs, T, Bmax, batches, fp32, sets):
     """the resident backward loop sums the bias and peephole gradients of its layer as it goes; MYEA_LSTM_RESIDENT_SUMS=0 has the
     weight-gradient pass read the gate deltas once more instead: the same gradient either way, with examples missing from the last
     group, in both directions, and when a smaller batch follows a larger one"""
-    specs = [dict(units=12), lstm(256, bidirectional=True), lstm(128), dict(units=128, activation="LINEAR")]
-    T, Bmax = 7, 80
     desc, h, w, masks, X, Y = _setup(specs, T, Bmax, Bmax, seed=33)
     inside, apart = _net(desc, h, w, None), _net(desc, h, w, None)
-    for B in (80, 45):
-        with environment(MYEA_LSTM_BACKWARD_KSPLIT=ksplit):
+    layers = [desc.layers[i] for i in range(desc.n_layers) if desc.layers[i].type_layer == mb.LAYER_LSTM]
+    for B, at in zip(batches, fp32):
+        assert _fp32_backward(layers, B) == [at] * len(layers)
+        with environment(MYEA_LSTM_BACKWARD_SETS=sets):
             inside.profile_enable(True)
             run_step(inside, B, X[:B], Y[:B], update=False)
-            assert _loop_launches(inside)[1] == 2, "the backward time loops did not run as one launch per layer"
+            assert _loop_launches(inside)[1] == len(layers), "the backward time loops did not run as one launch per layer"
             inside.profile_enable(False)
             with environment(MYEA_LSTM_RESIDENT_SUMS="0"):
                 run_step(apart, B, X[:B], Y[:B], update=False)
@@ -156,31 +180,33 @@ def test_bias_and_peephole_gradients_summed_inside_the_backward_loop(ksplit):
             n.Update_Parameter(B, B)
 
 
-@pytest.mark.parametrize("name,specs,T,B,Bmax", [(c[0], c[1], c[2], c[3], c[4]) for c in CASES if "512-cells" in c[0] or "1024-cells" in c[0]],
-                         ids=[c[0] for c in CASES if "512-cells" in c[0] or "1024-cells" in c[0]])
-def test_the_path_of_a_late_group(name, specs, T, B, Bmax):
-    """At 512 and 1024 cells a unit requests the next unit's first tiles between its own last MFMAs if the other chain's
-    counter is complete by then, behind them if not; which of the two happens depends on timing.  Here the second is forced
-    (every unit is told "not yet") and held against the oracle."""
+LATE_CASES = [c for c in CASES if True in c[5]]
+
+
+@pytest.mark.parametrize("name,specs,T,B,Bmax,fp32", LATE_CASES, ids=[c[0] for c in LATE_CASES])
+def test_the_path_of_a_late_group(name, specs, T, B, Bmax, fp32):
+    """On the FP32 instruction (1024 cells; the backward loop of 512 in one instruction stream) a unit requests the next unit's first tiles
+    between its own last MFMAs if the other chain's counter is complete by then, behind them if not; which of the two happens
+    depends on timing.  Here the second is forced (every unit is told "not yet") and held against the oracle."""
     desc, h, w, masks, X, Y = _setup(specs, T, B, Bmax, seed=23)
     zone_masks = masks if any(s.get("dropout") == "ZONEOUT" for s in specs) else None
     gpu = _net(desc, h, w, zone_masks)
-    cpu = OracleNetwork(desc, h)
+    cpu = OracleNetwork(desc, h, threads=8)
     cpu.set_state_propagation(mb.STATE_TRAINING)
     cpu.upload_parameters(w)
     if zone_masks is not None:
         cpu.upload_zoneout_masks(zone_masks)
     cpu.Clear_Training_Arrays()
-    # the backward form that stages tiles, with a member's two chains in one instruction stream (the form that has the two paths)
-    with environment(MYEA_LSTM_RESIDENT_TEST_NEVER_EARLY=1, MYEA_LSTM_BACKWARD_KSPLIT=0, MYEA_LSTM_BACKWARD_SETS=0):
+    with environment(MYEA_LSTM_RESIDENT_TEST_NEVER_EARLY=1, MYEA_LSTM_BACKWARD_SETS=0):
         gpu.profile_enable(True)
         for n in (gpu, cpu):
             n.Reset__Loss()
             run_step(n, B, X[:B], Y[:B], update=False)
         fwd, bwd = _loop_launches(gpu)
         gpu.profile_enable(False)
-    layers = sum(1 for i in range(desc.n_layers) if desc.layers[i].type_layer == mb.LAYER_LSTM)
-    assert fwd == layers and bwd == layers, "the time loops did not run as one launch per layer"
+    layers = [desc.layers[i] for i in range(desc.n_layers) if desc.layers[i].type_layer == mb.LAYER_LSTM]
+    assert fwd == len(layers) and bwd == len(layers), "the time loops did not run as one launch per layer"
+    assert _fp32_backward(layers, B) == fp32
     _compare(desc, gpu, cpu, B, T, "late path")
 
 
@@ -190,7 +216,7 @@ def test_a_smaller_batch_after_a_larger_one():
     T, Bmax = 6, 64
     desc, h, w, masks, X, Y = _setup(specs, T, Bmax, Bmax, seed=5)
     gpu = _net(desc, h, w, None)
-    cpu = OracleNetwork(desc, h)
+    cpu = OracleNetwork(desc, h, threads=8)
     cpu.set_state_propagation(mb.STATE_TRAINING)
     cpu.upload_parameters(w)
     cpu.Clear_Training_Arrays()
@@ -202,12 +228,15 @@ def test_a_smaller_batch_after_a_larger_one():
         _compare(desc, gpu, cpu, B, T, "batch %d" % B)
 
 
-def test_a_wait_that_gives_up_is_reported_once_and_the_network_carries_on_per_step():
+@pytest.mark.parametrize("cells,B,tiles", [(128, 32, 1), (300, 200, 2), (1024, 32, 0)], ids=["128-cells", "300-cells-two-row-tiles-a-group", "1024-cells-across-two-xcds"])
+def test_a_wait_that_gives_up_is_reported_once_and_the_network_carries_on_per_step(cells, B, tiles):
     """Every group is told to expect a member that does not exist: the first wait between time steps runs out of polls,
     every wavefront leaves through the give-up path, the next call that looks reports MYEA_E_DEVICE, and from then on the
     network uses one launch per time step."""
-    specs = [dict(units=8), lstm(128), dict(units=128, activation="LINEAR")]
-    T, B = 5, 32
+    specs = [dict(units=8), lstm(cells), dict(units=cells, activation="LINEAR")]
+    T = 5
+    plan = planes_plan(cells, B)
+    assert (plan.rs if plan.ok else 0) == tiles
     desc, h, w, masks, X, Y = _setup(specs, T, B, B, seed=7)
     gpu = _net(desc, h, w, None)
     with environment(MYEA_LSTM_RESIDENT_TEST_ABSENT_MEMBER=1, MYEA_LSTM_RESIDENT_SPIN_POLLS=64):
@@ -216,7 +245,7 @@ def test_a_wait_that_gives_up_is_reported_once_and_the_network_carries_on_per_st
             gpu.synchronize()
     assert e.value.code == mb.E_DEVICE and "gave up" in str(e.value)
     gpu.synchronize()   # reported once
-    cpu = OracleNetwork(desc, h)
+    cpu = OracleNetwork(desc, h, threads=8)
     cpu.set_state_propagation(mb.STATE_TRAINING)
     cpu.upload_parameters(w)
     cpu.Clear_Training_Arrays()
@@ -230,26 +259,29 @@ def test_a_wait_that_gives_up_is_reported_once_and_the_network_carries_on_per_st
     _compare(desc, gpu, cpu, B, T, "after the give-up")
 
 
-@pytest.mark.parametrize("cells,ksplit", [(128, "1"), (128, "0"), (512, "0"), (1024, "0")],
-                         ids=["backward-split-along-k", "backward-split-along-columns", "512-cells-a-set-of-wavefronts-per-chain", "1024-cells-across-two-xcds"])
-def test_a_backward_wait_that_gives_up_is_reported_too(cells, ksplit):
-    """the same forced give-up in the backward loop, in each of its forms (at 1024 cells with tile loads into LDS in flight
-    when the wait begins; at 512 cells every wait of the two sets of wavefronts - for the group, for the turn, for each other -
-    runs out on its own): the forward pass runs normally, the backward loop's first wait between steps runs out of polls and
-    every wavefront leaves"""
+# the row tiles a group has on the BF16 matrix cores, 0: the FP32 instruction's loop
+@pytest.mark.parametrize("cells,B,tiles,sets", [(128, 32, 1, "1"), (300, 200, 2, "1"), (512, 32, 1, "1"), (512, 141, 0, "1"), (512, 141, 0, "0"), (1024, 32, 0, "1")],
+                         ids=["128-cells", "300-cells-two-row-tiles-a-group", "512-cells", "512-cells-a-set-of-wavefronts-per-chain", "512-cells-one-stream",
+                              "1024-cells-across-two-xcds"])
+def test_a_backward_wait_that_gives_up_is_reported_too(cells, B, tiles, sets):
+    """the same forced give-up in the backward loop, in each of its forms (on the FP32 instruction with tile loads into LDS in flight when the
+    wait begins; in the form of two sets of wavefronts every wait - for the group, for the turn, for each other - runs out on its own):
+    the forward pass runs normally, the backward loop's first wait between steps runs out of polls and every wavefront leaves"""
     specs = [dict(units=8), lstm(cells), dict(units=cells, activation="LINEAR")]
-    T, B = 5, 32
+    T = 5
+    plan = planes_plan(cells, B)
+    assert (plan.rs if plan.backward else 0) == tiles
     desc, h, w, masks, X, Y = _setup(specs, T, B, B, seed=9)
     gpu = _net(desc, h, w, None)
     gpu.Forward_Pass(B, X)
     gpu.Compute__Error(B, Y)
     gpu.synchronize()
-    with environment(MYEA_LSTM_RESIDENT_TEST_ABSENT_MEMBER=1, MYEA_LSTM_RESIDENT_SPIN_POLLS=64, MYEA_LSTM_BACKWARD_KSPLIT=ksplit):
+    with environment(MYEA_LSTM_RESIDENT_TEST_ABSENT_MEMBER=1, MYEA_LSTM_RESIDENT_SPIN_POLLS=64, MYEA_LSTM_BACKWARD_SETS=sets):
         gpu.Backward_Pass(B)
         with pytest.raises(mb.MyeaError) as e:
             gpu.synchronize()
     assert e.value.code == mb.E_DEVICE and "gave up" in str(e.value)
-    cpu = OracleNetwork(desc, h)
+    cpu = OracleNetwork(desc, h, threads=8)
     cpu.set_state_propagation(mb.STATE_TRAINING)
     cpu.upload_parameters(w)
     cpu.Clear_Training_Arrays()
@@ -278,7 +310,7 @@ def test_weight_contractions_beside_the_backward_loop_change_nothing(cells):
     T, B = 6, 64
     desc, h, w, masks, X, Y = _setup(specs, T, B, B, seed=13)
     combined, separate = _net(desc, h, w, None), _net(desc, h, w, None)
-    cpu = OracleNetwork(desc, h)
+    cpu = OracleNetwork(desc, h, threads=8)
     cpu.set_state_propagation(mb.STATE_TRAINING)
     cpu.upload_parameters(w)
     cpu.Clear_Training_Arrays()
