@@ -12,7 +12,7 @@
 //     k = C into contiguous quarters; backward: the CELLS columns of dh, wavefront w takes the k range of gate w.  Either
 //     way a wavefront holds its [columns][k range] slice of Wrec (WrecT) in registers for the whole launch (at most 128
 //     registers per lane) in the operand layout of v_mfma_f32_16x16x4_f32;
-//   * a GROUP is the set of workgroups that cover all C cells for 2 x ROWS examples of one direction (ROWS = 16 RS):
+//   * a GROUP is the set of workgroups that cover all C cells for 2 x ROWS examples of one direction (ROWS = 16):
 //     C / CELLS members.  A member is a workgroup of four wavefronts - one per SIMD - that lives for all T steps and keeps
 //     its slice of the recurrent matrix in registers.  It works on two independent CHAINS of ROWS examples in turn: a
 //     UNIT is one time step of one chain, and the units of the two chains alternate in program order.
@@ -72,9 +72,9 @@ constexpr int kLocalAux = 16;      // cache policy of the LOCAL protocol's tile 
 #define MYEA_SCOPE_WORKGROUP __HIP_MEMORY_SCOPE_WORKGROUP
 
 // LDS of a workgroup: every wavefront's tiles of one unit, and the partial tiles of the two chains
-constexpr size_t forward_lds(int kw, int cells, int rs) { return ((size_t)4 * (kw / 32) * 16 * rs * 32 + (size_t)2 * 4 * 16 * rs * (4 * cells + 8)) * sizeof(float); }
+constexpr size_t forward_lds() { return ((size_t)4 * (256 / 32) * 16 * 32 + (size_t)2 * 4 * 16 * (4 * 16 + 8)) * sizeof(float); }
 constexpr size_t backward_sets_lds(int c) { return ((size_t)8 * (c / 32 < 8 ? c / 32 : 8) * 16 * 32 + (size_t)2 * 4 * 16 * 17) * sizeof(float); }
-constexpr size_t backward_lds(int c, int rs) { return ((size_t)4 * (c >= 512 && rs == 1 ? c / 64 : c / 32) * 16 * rs * 32 + (size_t)2 * 4 * 16 * rs * 17) * sizeof(float); }
+constexpr size_t backward_lds(int c) { return ((size_t)4 * (c / 64) * 16 * 32 + (size_t)2 * 4 * 16 * 17) * sizeof(float); }
 
 template <int N>
 __device__ __forceinline__ void wait_vm() { __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14)); }   // vmcnt(N)
@@ -246,16 +246,15 @@ struct ResidentGeometry {
 namespace {
 
 // ---- forward ---------------------------------------------------------------------------------------------------------
-// KW = C / 4: k's per wavefront.  Chain 0 holds the group's first ROWS examples, chain 1 the next ROWS.
+// 1024 cells, KW = C / 4 k's per wavefront.  Chain 0 holds the group's first ROWS examples, chain 1 the next ROWS.
 // Per lane the addresses of its (example, cell) pair(s) and of its tile rows are set up once and then stepped.
 using Chain0 = std::integral_constant<int, 0>;
 using Chain1 = std::integral_constant<int, 1>;
 
-template <int KW, int CELLS, int RS>
 __global__ __launch_bounds__(kThreads, 1) void lstm_resident_forward_kernel(ResidentGeometry g, LstmResidentDir d0, LstmResidentDir d1, SyncWords w)
 {
-    constexpr int C = 4 * KW, G = 4 * C;
-    constexpr int NB = 4 * CELLS, NCT = NB / 16, ROWS = 16 * RS, NT = KW / 32;
+    constexpr int C = 1024, G = 4 * C, KW = C / 4, CELLS = 16, ROWS = 16;
+    constexpr int NB = 4 * CELLS, NCT = NB / 16, NT = KW / 32;
     constexpr int LPT = ROWS / 8;                 // direct loads per tile
     constexpr int PAIRS = ROWS * CELLS / kThreads;
     constexpr int NSTORE = 7 * PAIRS;             // stores of a unit
@@ -352,7 +351,7 @@ __global__ __launch_bounds__(kThreads, 1) void lstm_resident_forward_kernel(Resi
             p_tile[ch][q] = d.h + ((size_t)t_first * Bmax + min((rg * 2 + ch) * ROWS + r, B - 1)) * C + wave * KW + chunk * 4;
         }
 
-    f32x4 acc[RS][NCT];
+    f32x4 acc[NCT];
     unsigned seen = 0;   // the next unit's counter as read during the MFMAs
 
     auto load_inputs = [&](auto ch) {   // input sums (and zoneout masks) of the step the chain's pointers are at
@@ -394,16 +393,11 @@ __global__ __launch_bounds__(kThreads, 1) void lstm_resident_forward_kernel(Resi
             const float *tile = stage + i * ROWS * 32;
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-                f32x4 fa[RS];
-#pragma unroll
-                for (int rs = 0; rs < RS; ++rs) fa[rs] = ATile<ROWS, kAux>::chunk(tile, rs * 16 + col16, h * 4 + quad);
+                const f32x4 fa = ATile<ROWS, kAux>::chunk(tile, col16, h * 4 + quad);
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
 #pragma unroll
-                    for (int ct = 0; ct < NCT; ++ct)
-#pragma unroll
-                        for (int rs = 0; rs < RS; ++rs)
-                            acc[rs][ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[rs][e], breg[i][h][ct][e], acc[rs][ct], 0, 0, 0);
+                    for (int ct = 0; ct < NCT; ++ct) acc[ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[e], breg[i][h][ct][e], acc[ct], 0, 0, 0);
             }
         }
     };
@@ -417,9 +411,7 @@ __global__ __launch_bounds__(kThreads, 1) void lstm_resident_forward_kernel(Resi
     auto head = [&](auto ch, auto all_landed) {
         constexpr int c = decltype(ch)::value;
 #pragma unroll
-        for (int rs = 0; rs < RS; ++rs)
-#pragma unroll
-            for (int ct = 0; ct < NCT; ++ct) acc[rs][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int ct = 0; ct < NCT; ++ct) acc[ct] = f32x4{0.f, 0.f, 0.f, 0.f};
         if (decltype(all_landed)::value) wait_vm<0>(); else wait_vm<NSTORE>();
         mfma_tiles(ch, I0{}, IA{});
         __builtin_amdgcn_sched_barrier(0);   // keeps the MFMAs above in front of the wait
@@ -475,11 +467,9 @@ __global__ __launch_bounds__(kThreads, 1) void lstm_resident_forward_kernel(Resi
         if (!FIRST) {
             float *to = part + wave * ROWS * kStride;
 #pragma unroll
-            for (int rs = 0; rs < RS; ++rs)
+            for (int ct = 0; ct < NCT; ++ct)
 #pragma unroll
-                for (int ct = 0; ct < NCT; ++ct)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) to[(rs * 16 + quad * 4 + r) * kStride + ct * 16 + col16] = acc[rs][ct][r];
+                for (int r = 0; r < 4; ++r) to[(quad * 4 + r) * kStride + ct * 16 + col16] = acc[ct][r];
             lds_barrier();
         }
 #pragma unroll
@@ -574,27 +564,24 @@ __device__ __forceinline__ void store_column_sums(const double (&sums)[7], float
 // CELLS = 16 columns of dh; wavefront w contracts over the k range of gate w (k = gate * C + cell of dG[t']) against its
 // slice of the transposed packed matrix WrecT [C][4C].  j counts the steps of this pass: the direction's own step is
 // s = T - 1 - j.  j = 0 has no recurrent term and no terms from a later step; s = 0 writes no forget-gate delta.
-template <int CC, int RS>
+template <int CC>
 __global__ __launch_bounds__(kThreads, 1) void lstm_resident_backward_kernel(ResidentGeometry g, LstmResidentDir d0, LstmResidentDir d1, SyncWords w)
 {
     constexpr int C = CC, G = 4 * C, CELLS = 16;
-    constexpr int ROWS = 16 * RS, NT = C / 32;    // tiles of 32 k in a gate's range
+    constexpr int ROWS = 16, NT = C / 32;         // tiles of 32 k in a gate's range
     constexpr int LPT = ROWS / 8;
     constexpr int PAIRS = ROWS * CELLS / kThreads;
     constexpr int NSTORE = 6 * PAIRS;
-    constexpr int A1 = NT / 4, P1 = (3 * NT) / 4;
     constexpr int kStride = 17;
-    // WIDE (C = 1024): a unit's gate deltas (16 examples x 4096 k = 256 KiB) do not fit LDS at once.  They pass through two
+    // A unit's gate deltas (at 1024 cells 16 examples x 4096 k = 256 KiB) do not fit LDS at once.  They pass through two
     // half buffers of NT / 4 tiles per wavefront in four groups: while group g is contracted, group g + 2 lands in the half
-    // that group g has just left.  Its 64 members span two XCDs: device-scope stores of the gate deltas, device-scope
+    // that group g has just left.  The 64 members of 1024 cells span two XCDs: device-scope stores of the gate deltas, device-scope
     // counter, tile loads served beyond the XCD's L2 (as in the forward loop of this width).
     constexpr bool AGENT = C > 512;               // 64 members: the group spans two XCDs
-    constexpr bool WIDE = C >= 512 && RS == 1;    // a unit's tiles pass through half as many LDS slots, requested a quarter of the unit ahead
-    constexpr int SLOTS = WIDE ? NT / 2 : NT, NG = NT / 4;   // tiles of LDS per wavefront; tiles per group
+    constexpr int SLOTS = NT / 2, NG = NT / 4;    // tiles of LDS per wavefront; tiles per group
     constexpr int kStage = SLOTS * ROWS * 32, kPart = 4 * ROWS * kStride;
     constexpr int kAux = AGENT ? 16 : kLocalAux;
-    static_assert(!WIDE || RS == 1, "the wide form has one set of rows per chain");
-    static_assert(NT >= 4 && (WIDE ? 3 * NG * LPT + 9 : NT * LPT) + NSTORE < 64, "vmcnt has 6 bits");
+    static_assert(NT >= 4 && 3 * NG * LPT + 9 + NSTORE < 64, "vmcnt has 6 bits");
     extern __shared__ __attribute__((aligned(16))) float smem[];
     __shared__ unsigned s_arrive[2];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col16 = lane & 15, quad = lane >> 4;
@@ -667,7 +654,7 @@ __global__ __launch_bounds__(kThreads, 1) void lstm_resident_backward_kernel(Res
             p_tile[ch][q] = d.dG + ((size_t)t_first * Bmax + min((rg * 2 + ch) * ROWS + r, B - 1)) * G + (size_t)wave * C + chunk * 4;
         }
 
-    f32x4 acc[RS][2];
+    f32x4 acc[2];
     unsigned seen = 0;
 
     auto load_operands = [&](auto ch, bool with_cp) {   // of the step the chain's pointers are at; with_cp: not the direction's first step, which has no step before it
@@ -697,10 +684,10 @@ __global__ __launch_bounds__(kThreads, 1) void lstm_resident_backward_kernel(Res
             for (int q = 0; q < LPT; ++q) p_tile[c][q] += step_g;
         }
     };
-    auto load_tiles = [&](auto ch) {   // dG of the chain's step processed before the one its pointers are at: all of it, or (WIDE) its first group
-        load_tile_range(ch, std::integral_constant<int, 0>{}, std::integral_constant<int, WIDE ? NG : SLOTS>{}, std::integral_constant<bool, !WIDE>{});
+    auto load_tiles = [&](auto ch) {   // dG of the chain's step processed before the one its pointers are at: its first group
+        load_tile_range(ch, std::integral_constant<int, 0>{}, std::integral_constant<int, NG>{}, std::false_type{});
     };
-    // WIDE: one tile at a time, the next tile's operand read from LDS while this one's MFMAs run
+    // one tile at a time, the next tile's operand read from LDS while this one's MFMAs run
     auto read_tile = [&](auto i, f32x4 (&fa)[2]) {
         const float *tile = stage + (decltype(i)::value % SLOTS) * ROWS * 32;
 #pragma unroll
@@ -710,7 +697,7 @@ __global__ __launch_bounds__(kThreads, 1) void lstm_resident_backward_kernel(Res
 #pragma unroll
         for (int h = 0; h < 2; ++h)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) acc[0][e & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[h][e], breg[decltype(i)::value][h][e], acc[0][e & 1], 0, 0, 0);
+            for (int e = 0; e < 4; ++e) acc[e & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[h][e], breg[decltype(i)::value][h][e], acc[e & 1], 0, 0, 0);
     };
     auto mfma_tiles = [&](auto first, auto last) {
 #pragma unroll
@@ -718,58 +705,46 @@ __global__ __launch_bounds__(kThreads, 1) void lstm_resident_backward_kernel(Res
             const float *tile = stage + (i % SLOTS) * ROWS * 32;
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-                f32x4 fa[RS];
+                const f32x4 fa = ATile<ROWS, kAux>::chunk(tile, col16, h * 4 + quad);
 #pragma unroll
-                for (int rs = 0; rs < RS; ++rs) fa[rs] = ATile<ROWS, kAux>::chunk(tile, rs * 16 + col16, h * 4 + quad);
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-#pragma unroll
-                    for (int rs = 0; rs < RS; ++rs)
-                        acc[rs][e & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[rs][e], breg[i][h][e], acc[rs][e & 1], 0, 0, 0);
+                for (int e = 0; e < 4; ++e) acc[e & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[e], breg[i][h][e], acc[e & 1], 0, 0, 0);
             }
         }
     };
     using I0 = std::integral_constant<int, 0>;
-    using IA = std::integral_constant<int, A1>;
-    using IP = std::integral_constant<int, P1>;
+    using I1 = std::integral_constant<int, NG>;
+    using I3 = std::integral_constant<int, 3 * NG>;
     using IN = std::integral_constant<int, NT>;
 
     auto head = [&](auto ch, auto all_landed) {
         constexpr int c = decltype(ch)::value;
-#pragma unroll
-        for (int rs = 0; rs < RS; ++rs) { acc[rs][0] = f32x4{0.f, 0.f, 0.f, 0.f}; acc[rs][1] = f32x4{0.f, 0.f, 0.f, 0.f}; }
+        acc[0] = f32x4{0.f, 0.f, 0.f, 0.f}; acc[1] = f32x4{0.f, 0.f, 0.f, 0.f};
         if (decltype(all_landed)::value) wait_vm<0>(); else wait_vm<NSTORE>();   // the unit's first group has landed
-        if constexpr (WIDE) {
-            // The loads of a tile are issued one tile at a time between the MFMAs, never as a burst: a compute unit's address path
-            // takes 16 clocks per 1 KiB load instruction, and a wavefront that issues sixteen of them in a row stands still for
-            // as long as sixty-four MFMAs take.  Here: the second group into the second half, which the other chain has left.
-            f32x4 fa[2][2];
-            read_tile(I0{}, fa[0]);
-            static_for<0, NG>([&](auto i) {
-                constexpr int I = decltype(i)::value;
-                __builtin_amdgcn_sched_barrier(0);
-                if (I + 1 < NG) read_tile(std::integral_constant<int, I + 1>{}, fa[(I + 1) & 1]);
-                mfma_tile(i, fa[I & 1]);
-                load_tile_range(ch, std::integral_constant<int, I + NG>{}, std::integral_constant<int, I + NG + 1>{}, std::false_type{});
-            });
+        // The loads of a tile are issued one tile at a time between the MFMAs, never as a burst: a compute unit's address path
+        // takes 16 clocks per 1 KiB load instruction, and a wavefront that issues sixteen of them in a row stands still for
+        // as long as sixty-four MFMAs take.  Here: the second group into the second half, which the other chain has left.
+        f32x4 fa[2][2];
+        read_tile(I0{}, fa[0]);
+        static_for<0, NG>([&](auto i) {
+            constexpr int I = decltype(i)::value;
             __builtin_amdgcn_sched_barrier(0);
-            wait_vm<NG * LPT>();             // the stores of the unit before are older than the second group's loads
-        } else {
-            mfma_tiles(I0{}, IA{});
-            __builtin_amdgcn_sched_barrier(0);   // keeps the MFMAs above in front of the wait
-            wait_vm<0>();
-        }
+            if (I + 1 < NG) read_tile(std::integral_constant<int, I + 1>{}, fa[(I + 1) & 1]);
+            mfma_tile(i, fa[I & 1]);
+            load_tile_range(ch, std::integral_constant<int, I + NG>{}, std::integral_constant<int, I + NG + 1>{}, std::false_type{});
+        });
+        __builtin_amdgcn_sched_barrier(0);
+        wait_vm<NG * LPT>();             // the stores of the unit before are older than the second group's loads
         wave_arrive<AGENT>(counters + (1 - c) * kSyncStride, &s_arrive[1 - c]);
     };
     // FIRST: the pass's first step of the chain (no recurrent term, nothing from a later step); s: the direction's step
     auto tail = [&](auto ch, auto first_tag, int s, unsigned wait_for) -> bool {
         constexpr int c = decltype(ch)::value;
         constexpr bool FIRST = decltype(first_tag)::value;
-        // WIDE: every unit must issue the same number of loads, the waits count them - where `s` is a literal zero the compiler
+        // every unit must issue the same number of loads, the waits count them - where `s` is a literal zero the compiler
         // would drop the load of the state before it
-        if (WIDE) asm volatile("" : "+s"(s));
+        asm volatile("" : "+s"(s));
         load_operands(ch, s > 0);
-        if constexpr (!FIRST && WIDE) {
+        if constexpr (!FIRST) {
             // tile i's MFMAs, then the loads of the tile that takes a slot no longer read: i + 8 of this unit (two groups ahead
             // of its use minus one), or - the last group - tile i - 24 of the other chain's next unit, if that chain's step is
             // complete by then.  The waits count what was issued behind the tile they wait for (two loads per tile, the eight
@@ -779,7 +754,7 @@ __global__ __launch_bounds__(kThreads, 1) void lstm_resident_backward_kernel(Res
             f32x4 fa[2][2];
             __builtin_amdgcn_sched_barrier(0);
             wait_vm<(NG - 1) * LPT + kOps>();
-            read_tile(IA{}, fa[NG & 1]);
+            read_tile(I1{}, fa[NG & 1]);
             static_for<NG, 3 * NG>([&](auto i) {
                 constexpr int I = decltype(i)::value;
                 __builtin_amdgcn_sched_barrier(0);
@@ -805,32 +780,22 @@ __global__ __launch_bounds__(kThreads, 1) void lstm_resident_backward_kernel(Res
                 __builtin_amdgcn_sched_barrier(0);
             } else {   // the other chain is late (or has no further unit): this unit's last group first, then the wait, then its tiles in a row
                 wait_vm<0>();
-                mfma_tiles(IP{}, IN{});
+                mfma_tiles(I3{}, IN{});
                 __builtin_amdgcn_sched_barrier(0);
                 if (wait_for) {
                     if (!wave_wait(w, counters + (1 - c) * kSyncStride, target, g.spin_polls)) return false;
                     load_tiles(std::integral_constant<int, 1 - c>{});
                 }
             }
-        } else if (!FIRST) {
-            mfma_tiles(IA{}, IP{});
-            if (wait_for) seen = __hip_atomic_load(counters + (1 - c) * kSyncStride, __ATOMIC_RELAXED, MYEA_SCOPE_AGENT);
-            mfma_tiles(IP{}, IN{});
-            __builtin_amdgcn_sched_barrier(0);   // the counter's value is looked at after the MFMAs, not right behind its load
-        }
-        if (wait_for && (FIRST || !WIDE)) {
-            const unsigned target = wait_for * members;
-            const bool there = !FIRST && (int)(__builtin_amdgcn_readfirstlane(seen) - target) >= 0;
-            if (!there && !wave_wait(w, counters + (1 - c) * kSyncStride, target, g.spin_polls)) return false;
+        } else if (wait_for) {
+            if (!wave_wait(w, counters + (1 - c) * kSyncStride, wait_for * members, g.spin_polls)) return false;
             load_tiles(std::integral_constant<int, 1 - c>{});
         }
         float *part = parts + c * kPart;
         if (!FIRST) {
             float *to = part + wave * ROWS * kStride;
 #pragma unroll
-            for (int rs = 0; rs < RS; ++rs)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) to[(rs * 16 + quad * 4 + r) * kStride + col16] = acc[rs][0][r] + acc[rs][1][r];
+            for (int r = 0; r < 4; ++r) to[(quad * 4 + r) * kStride + col16] = acc[0][r] + acc[1][r];
             lds_barrier();
         }
 #pragma unroll
@@ -1336,50 +1301,19 @@ using ResidentKernel = void (*)(ResidentGeometry, LstmResidentDir, LstmResidentD
 struct KernelInfo {
     ResidentKernel fn = nullptr;
     size_t lds = 0;
-    int cells = 0;
     int threads = kThreads;
     bool ready = false;
     hipError_t status = hipSuccess;
     int per_cu = 0;   // workgroups of this kernel a compute unit can hold
 };
 
-template <int KW, int CELLS, int RS>
-KernelInfo forward_info()
-{
-    KernelInfo k;
-    k.fn = lstm_resident_forward_kernel<KW, CELLS, RS>;
-    k.lds = forward_lds(KW, CELLS, RS);
-    k.cells = CELLS;
-    return k;
-}
-template <int C, int RS>
-KernelInfo backward_info()
-{
-    KernelInfo k;
-    k.fn = lstm_resident_backward_kernel<C, RS>;
-    k.lds = backward_lds(C, RS);
-    k.cells = 16;
-    return k;
-}
-
-template <int C>
-KernelInfo sets_info()
-{
-    KernelInfo k;
-    k.fn = lstm_resident_backward_sets_kernel<C>;
-    k.lds = backward_sets_lds(C);
-    k.cells = 16;
-    k.threads = 2 * kThreads;
-    return k;
-}
-
 // What the loops of myea_lstm_planes.hip leave to these: both passes at 1024 cells, whose members span two XCDs, and the backward pass at
 // 512 cells and more than one row of 16 examples a group (256 examples, 64 time steps: 454 us here, 619 there; up to 128 examples 460
 // here, 237 there).
-KernelInfo g_forward_1024 = forward_info<256, 16, 1>();
-KernelInfo g_backward_512 = backward_info<512, 1>(), g_backward_1024 = backward_info<1024, 1>();
+KernelInfo g_forward_1024 = {lstm_resident_forward_kernel, forward_lds()};
+KernelInfo g_backward_512 = {lstm_resident_backward_kernel<512>, backward_lds(512)}, g_backward_1024 = {lstm_resident_backward_kernel<1024>, backward_lds(1024)};
 // the 512-cell backward loop with one chain per set of four wavefronts
-KernelInfo g_sets_512 = sets_info<512>();
+KernelInfo g_sets_512 = {lstm_resident_backward_sets_kernel<512>, backward_sets_lds(512), 2 * kThreads};
 
 // MYEA_LSTM_BACKWARD_SETS=0 keeps the backward loop's two chains in one instruction stream
 bool sets_disabled()
@@ -1500,7 +1434,7 @@ int lstm_resident_plan(size_t C, size_t cells_per_block, size_t B, int dirs, boo
         if (rc != MYEA_OK) return rc;
     }
     if (!dev->usable) return MYEA_OK;
-    const int members = (int)C / k->cells;
+    const int members = (int)C / 16;
     const bool agent = members > dev->cus / 8;
     const int row_groups = (int)((B + 31) / 32);
     int grid = 0;
