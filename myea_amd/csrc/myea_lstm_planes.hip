@@ -33,8 +33,9 @@
 // barrier; backward, the unit before is contracted while the gates of this one are worked on.
 //
 // Measured (MI355X, microseconds a pass, one launch per time step or the FP32 loops -> here; forward, backward): 200 cells x 60 examples x 50
-// steps 271 -> 107, 274 -> 107; 512 x 16 x 64 365 -> 178, 412 -> 200; 512 x 256 x 64 410 -> 255, stays (see lstm_planes_plan); 300 x 128 x
-// 30, two directions 290 -> 104, 293 -> 147; 64 x 512 x 30 130 -> 63, 107 -> 56; 480 x 512 x 30 568 -> 234, 649 -> 624.  What bounds a step
+// steps 271 -> 107, 274 -> 107; 512 x 16 x 64 365 -> 178, 412 -> 200; 512 x 256 x 64 410 -> 255, stays (see backward_most_tiles); 300 x 128 x
+// 30, two directions 290 -> 104, 293 -> 147; 64 x 512 x 30 130 -> 63, 107 -> 56; 480 x 512 x 30 568 -> 234, 649 -> 624; 128 x 256 x 32 127 -> 69,
+// 102 -> 66; 256 x 256 x 32 173 -> 79, 153 -> 80; 256 x 1024 x 32 466 -> 209, 582 -> 449.  What bounds a step
 // of one row tile at 512 cells: 0.6 us of gate math behind the partial tiles, 0.6 of products, 0.5 from a store to another
 // member's look, the rest the looks themselves; of several: the exchange (48 KB a unit and member forward, 96 KB backward).
 //
