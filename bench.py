@@ -29,11 +29,11 @@ if ROOT not in sys.path:
 RECORDED_TRAFFIC = {"fc4096x4_b1024_adam": dict(bytes_per_launch=2958506 * 1024 / 10,
                                                 source="recorded constant, not measured in this run: profiles/hbm_traffic__fc4096x4_b1024_adam__pmc.txt"),
                     # the two resident time loops of one layer (forward + backward launch), mean per launch
-                    "lstm512x2_t64_b256_amsgrad": dict(bytes_per_launch=(2 * 98055.1 + 230411.5 + 2 * 203936.9 + 197795.6) * 1024 / 2,
+                    "lstm512x2_t64_b256_amsgrad": dict(bytes_per_launch=(2 * 83624.0 + 232740.0 + 2 * 203658.0 + 197804.0) * 1024 / 2,
                                                        source="recorded constant, not measured in this run: profiles/lstm_resident__lstm512x2_t64_b256_amsgrad__pmc.txt")}
 from myea_amd.synthetic import simple_debug_layers  # noqa: E402  (no device is touched by the import)
 
-PEAK_FP32_MFMA_TFLOPS = 157.3   # MI355X dense FP32 matrix: the resident LSTM time loops
+PEAK_FP32_MFMA_TFLOPS = 157.3   # MI355X dense FP32 matrix: what the resident LSTM time loops are priced by (those on the BF16 matrix cores too)
 PEAK_CONTRACTION_TFLOPS = 2516.6 / 6   # MI355X dense BF16 matrix, six products a multiplication: the contractions
 SUSTAINED_CONTRACTION_TFLOPS = 1143.0 / 6   # the rate a large BF16 product of the vendor's library was measured to sustain, over six
 PEAK_HBM_GBS = 8000.0           # MI355X HBM3E
@@ -418,11 +418,11 @@ def main():
     if alone:
         out["events_pass_update_apart"] = {"steps": args.steps, "ms_per_step": r["ms_per_step_events_alone"]}
     if has_loops:
-        out["time_loops"] = dict(r["time_loops"], kernel="lstm_resident_forward_kernel / lstm_resident_backward_kernel (or one lstm_fused_* launch per step)")
+        out["time_loops"] = dict(r["time_loops"], kernel="lstm_planes_* / lstm_resident_* (or one lstm_fused_* / lstm_step_* launch per step)")
     if args.workload != SECONDARY and args.workload == "fc4096x4_b1024_adam" and not args.no_secondary:
         sec_steps = max(5, 2 * args.steps // 3)
         s = run_workload(SECONDARY, sec_steps, max(2, args.warmup), args.separate_update, args.repeats)
-        loops = dict(s["time_loops"], kernel="lstm_resident_forward_kernel + lstm_resident_backward_kernel: the recurrent contractions and gate math of steps 1 .. T-1, one launch per layer and pass")
+        loops = dict(s["time_loops"], kernel="lstm_planes_forward_kernel + lstm_resident_backward_sets_kernel: the recurrent contractions and gate math of steps 1 .. T-1, one launch per layer and pass")
         sec_traffic = RECORDED_TRAFFIC.get(SECONDARY)
         loops["traffic"] = sec_traffic["bytes_per_launch"] if sec_traffic else None
         if sec_traffic:
